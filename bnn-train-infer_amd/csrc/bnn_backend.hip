@@ -33,6 +33,7 @@ constexpr size_t kPinnedCap = size_t(8) << 20;       // largest transfer staged 
 constexpr size_t kWriteRingBytes = size_t(1) << 20;  // pinned ring for small writes
 constexpr size_t kAsyncWriteMax = size_t(64) << 10;  // writes up to this size return before the copy ends
 constexpr size_t kScratchRowsCap = 4096;              // rows per launch chunk
+constexpr uint32_t kRowsMaxJobs = 8;                  // jobs of one BNNX_LaunchRows call
 constexpr size_t kExecuteScratchBytes = size_t(32) << 20;  // allocated with the device
 
 bool mul_size(size_t a, size_t b, size_t* out) {
@@ -1472,6 +1473,112 @@ EXPORT BNN_Status BNNX_BatchCreateFusedPost(BNN_Device device, const BNN_Job* jo
 EXPORT BNN_Status BNNX_BatchCreateFused(BNN_Device device, const BNN_Job* jobs, uint32_t count, const BNNX_PreOp* pre,
                                         BNNX_Batch* out_batch) {
     return BNNX_BatchCreateFusedPost(device, jobs, count, pre, nullptr, out_batch);
+}
+
+// Multi-row fused launches: nothing is built, the rows' quantised forms live in the device's
+// scratch (stream order makes one scratch enough for any number of launches in flight).
+EXPORT BNN_Status BNNX_LaunchRows(BNN_Device device, const BNN_Job* jobs, uint32_t count, const BNNX_PreOp* pre) {
+    if (device == nullptr || jobs == nullptr || count == 0 || pre == nullptr)
+        return BNN_EINVAL;
+    if (count > kRowsMaxJobs)
+        return BNN_ENOTSUP;
+    if (pre->kind != BNNX_PRE_ROW && pre->kind != BNNX_PRE_RMSNORM && pre->kind != BNNX_PRE_SILU_MUL)
+        return BNN_EINVAL;
+    const uint32_t width = pre->width, rows = jobs[0].rows;
+    if (width == 0 || width % kGroup != 0)
+        return BNN_EINVAL;
+    if ((pre->kind == BNNX_PRE_RMSNORM && (pre->a == nullptr || pre->gain == nullptr)) ||
+        (pre->kind == BNNX_PRE_SILU_MUL && (pre->a == nullptr || pre->b == nullptr)))
+        return BNN_EINVAL;
+    JobPlan plans[kRowsMaxJobs];
+    Span outs[kRowsMaxJobs + 1], reads[4];
+    for (uint32_t i = 0; i < count; ++i) {
+        JobPlan& p = plans[i];
+        const BNN_Status st = plan_job(device, &jobs[i], &p);
+        if (st != BNN_OK)
+            return st;
+        if (!p.f32_in || !p.out_aligned || rows > kScratchRowsCap)
+            return BNN_ENOTSUP;
+        if (p.m->k != width || jobs[i].rows != rows)
+            return BNN_EINVAL;
+        if (pre->kind == BNNX_PRE_ROW) {
+            if (!p.in_aligned)
+                return BNN_ENOTSUP;
+            if (p.in_base != plans[0].in_base || p.in_stride != plans[0].in_stride)
+                return BNN_EINVAL;
+        }
+        outs[i] = span_of(p.out_base, (size_t)(rows - 1u) * p.out_stride + p.out_row);
+    }
+    // the launches of one call read the operands while others write: no output may overlap
+    // an operand or another output
+    const size_t block = (size_t)rows * width * 4u;
+    uint32_t nreads = 0, nouts = count;
+    if (pre->kind == BNNX_PRE_ROW) {
+        reads[nreads++] = span_of(plans[0].in_base, (size_t)(rows - 1u) * plans[0].in_stride + plans[0].in_row);
+    } else {
+        reads[nreads++] = span_of(pre->a, block);
+        if (pre->b)
+            reads[nreads++] = span_of(pre->b, block);
+        if (pre->kind == BNNX_PRE_RMSNORM)
+            reads[nreads++] = span_of(pre->gain, (size_t)width * 4u);
+    }
+    float* const a_out = pre->kind == BNNX_PRE_RMSNORM ? pre->a_out : nullptr;
+    if (a_out)
+        outs[nouts++] = span_of(a_out, block);
+    for (uint32_t i = 0; i < nouts; ++i) {
+        for (uint32_t j = 0; j < i; ++j)
+            if (spans_overlap(outs[i], outs[j]))
+                return BNN_EINVAL;
+        for (uint32_t j = 0; j < nreads; ++j)
+            if (spans_overlap(outs[i], reads[j]))
+                return BNN_EINVAL;
+    }
+    const size_t rscale_at = round_up((size_t)rows * width, 256);
+    if (rscale_at + (size_t)rows * 4u > device->scratch_bytes)
+        return BNN_ENOTSUP;
+    device->mirror_buf = nullptr;
+    if (hipSetDevice(device->ordinal) != hipSuccess)
+        return BNN_EIO;
+    const uint64_t seq = ++device->seq;
+    if (device->async_first_seq == 0)
+        device->async_first_seq = seq;
+    PrepJob pj = {};
+    pj.in = plans[0].in_base;
+    pj.in_stride = plans[0].in_stride;
+    pj.q = reinterpret_cast<int8_t*>(device->scratch);
+    pj.rscale = reinterpret_cast<float*>(device->scratch + rscale_at);
+    pj.k = width;
+    pj.rows = rows;
+    pj.f32 = 1;
+    pj.aligned = 1;
+    hipError_t e = timed(device, KK_PREP, [&] {
+        if (pre->kind == BNNX_PRE_ROW)
+            return launch_prep(device->stream, pj, false, seq, device->flag_dev, device->status_host + 1);
+        RowsArgs ra = {};
+        ra.a = pre->a;
+        ra.b = pre->b;
+        ra.gain = pre->gain;
+        ra.a_out = a_out;
+        ra.q = pj.q;
+        ra.rscale = pj.rscale;
+        ra.err = pre->kind == BNNX_PRE_RMSNORM ? pre->err : nullptr;
+        ra.err_code = pre->err_code;
+        ra.eps = pre->eps;
+        ra.width = width;
+        ra.rows = rows;
+        ra.kind = pre->kind;
+        return launch_rows(device->stream, ra, seq, device->flag_dev, device->status_host + 1);
+    });
+    for (uint32_t i = 0; e == hipSuccess && i < count; ++i) {
+        const GemmJob gj = make_gemm(plans[i], pj, plans[i].out_base, plans[i].out_stride);
+        e = timed(device, KK_GEMM,
+                  [&] { return launch_gemm(device->stream, gj, device->cu_count, seq, device->flag_dev); });
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return BNN_EIO;
+    }
+    return BNN_OK;
 }
 
 EXPORT BNN_Status BNNX_BatchCheck(BNNX_Batch batch) {

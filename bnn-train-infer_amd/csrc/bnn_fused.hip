@@ -25,6 +25,7 @@
 
 #include "bnn_bitplane.h"
 #include "bnn_internal.h"
+#include "bnn_rowsum.h"
 
 #define BNNE_EXPF_QUALIFIER static __device__ __forceinline__
 #include "libc_expf.h"
@@ -55,7 +56,6 @@ __device__ __forceinline__ void fused_exp_table_fill(uint64_t* tab, uint32_t lan
 }
 
 extern "C" __device__ uint32_t __ockl_wfred_max_u32(uint32_t);
-extern "C" __device__ double __ockl_wfred_add_f64(double);
 extern "C" __device__ int __ockl_wfred_add_i32(int);
 
 // Bit planes B..7 of the wave's 64 quantised values q: lane 2b of `word` receives
@@ -69,64 +69,6 @@ __device__ __forceinline__ void plane_words(int q, uint32_t& word, int& sum) {
     put_plane_mask<B>(mask, word);
     if constexpr (B < 7)
         plane_words<B + 1>(q, word, sum);
-}
-
-
-// The sum of the squares in index order, s_{i+1} = F32(s_i + t_i) from s_0 = +0,
-// evaluated in segments of kSegment terms.  Segment j is run from kWindow candidate
-// starts at once (one lane each): the binary32 values whose bit patterns lie around
-// that of F32(E_j), E_j the sum of the earlier terms in binary64.  Afterwards one
-// wave walks the segments in order: when the running sum is one of segment j's
-// candidates, the lane that started from exactly that value has performed the same
-// additions from the same value, and its end value is taken; otherwise the segment
-// is added term by term.  Either way the result is bit-identical to the sequential
-// loop; the walk costs one table lookup per segment in the usual case, where the
-// accumulated rounding of the sequential sum stays within +-16 ulps of E_j.
-constexpr uint32_t kSegment = 128;
-constexpr uint32_t kWindow = 32;
-constexpr uint32_t kChunk = 64;  // terms per binary64 partial sum (one wave's)
-
-// s plus the n terms at p, one rounding per addition, in index order (n % 16 == 0)
-__device__ __forceinline__ float add_in_order_lds(const float* p, uint32_t n, float s) {
-    const float4* p4 = reinterpret_cast<const float4*>(p);
-#pragma unroll 1
-    for (uint32_t i = 0; i < n / 4u; i += 4u) {
-        float4 v[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            v[c] = p4[i + c];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            s = s + v[c].x;
-            s = s + v[c].y;
-            s = s + v[c].z;
-            s = s + v[c].w;
-        }
-    }
-    return s;
-}
-
-// NC interleaved candidate chains of one wave over kSegment terms each
-template <int NC>
-__device__ __forceinline__ void run_chains(float (&c)[NC], const float4* const (&src)[NC]) {
-#pragma unroll 2
-    for (uint32_t i = 0; i < kSegment / 4u; i += 8u) {
-        float4 v[NC][8];
-#pragma unroll
-        for (int r = 0; r < NC; ++r)
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                v[r][q] = src[r][i + q];
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-#pragma unroll
-            for (int r = 0; r < NC; ++r) {
-                c[r] = c[r] + v[r][q].x;
-                c[r] = c[r] + v[r][q].y;
-                c[r] = c[r] + v[r][q].z;
-                c[r] = c[r] + v[r][q].w;
-            }
-    }
 }
 
 
@@ -147,8 +89,8 @@ __device__ __forceinline__ void fused_raise(uint64_t seq, uint64_t* flag, uint64
     __hip_atomic_store(host_status, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-constexpr uint32_t kFusedThreads = 1024;
-constexpr uint32_t kFusedWaves = kFusedThreads / 64;
+constexpr uint32_t kFusedThreads = kRowThreads;
+constexpr uint32_t kFusedWaves = kRowWaves;
 constexpr uint32_t kFusedMaxGroups = kFusedMaxWidth / kGroup;
 constexpr uint32_t kFusedPad = 32;  // spare floats after the row (16-byte aligned product buffers)
 
@@ -330,16 +272,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& fa, uint32_t tiles_t
     __shared__ uint4 planes[GPW > 1 ? kFusedMaxGroups * kPlaneWords / 4 : 1];
     __shared__ uint32_t amax_w[kFusedWaves];
     __shared__ uint64_t exp_tab[32];
-    __shared__ float rms_s;
-    // the speculative sum of squares: binary64 sums of 64 terms, the candidates' end
-    // values (segments 2p and 2p + 1 in the two halves of row p), the segments' first
-    // candidate bit pattern
-    constexpr uint32_t kRowMax = EPT * kFusedThreads;
-    constexpr uint32_t kPairs = kRowMax / kSegment / 2u;
-    __shared__ double chunk_sum[kRowMax / kChunk];
-    __shared__ float seg_end[kPairs * 64u];
-    __shared__ float seg_comp[kPairs * 32u];  // pair p's two segments composed, per candidate of segment 2p
-    __shared__ int seg_base[kPairs * 2u];
+    __shared__ RowSumLds<EPT> sum_lds;
     float* scratch = reinterpret_cast<float*>(scratch4);
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -433,119 +366,13 @@ __device__ __forceinline__ void fused_body(const FusedArgs& fa, uint32_t tiles_t
             for (int i = 0; i < EPT; ++i)
                 xv[i] = xv[i] + bv[i];
         }
-        // the terms, and their binary64 sums per 64 (chunk k / 64)
+        if (fa.a_out && blockIdx.x == 0) {
 #pragma unroll
-        for (int i = 0; i < EPT; ++i) {
-            const uint32_t k = elem(i);
-            const float sq = xv[i] * xv[i];
-            if (live(i)) {
-                scratch[k] = sq;
-                if (fa.a_out && blockIdx.x == 0)
-                    gstore(fa.a_out + k, xv[i]);
-                const double h = __ockl_wfred_add_f64((double)sq);
-                if (lane == 0)
-                    chunk_sum[k / kChunk] = h;
-            }
+            for (int i = 0; i < EPT; ++i)
+                if (live(i))
+                    gstore(fa.a_out + elem(i), xv[i]);
         }
-        lds_barrier();
-        // candidate chains: wave w runs pairs w, w + 16, ... (segments 2p, 2p + 1)
-        const uint32_t nseg = K / kSegment, npairs = (nseg + 1u) / 2u;
-        const uint32_t half = lane >> 5, cand = lane & (kWindow - 1u);
-        constexpr int kPairsPerWave = (kPairs + kFusedWaves - 1) / kFusedWaves;
-        float c[kPairsPerWave];
-        int bs[kPairsPerWave];
-        const float4* src[kPairsPerWave];
-#pragma unroll
-        for (int r = 0; r < kPairsPerWave; ++r) {
-            const uint32_t p = min(wave + kFusedWaves * r, npairs - 1u);
-            // E_{2p}: the chunks before segment 2p; E_{2p+1} adds segment 2p's two
-            double e = 0.0;
-#pragma unroll
-            for (uint32_t cc = 0; cc < kRowMax / kChunk; cc += 64u)
-                if (cc + lane < 4u * p)
-                    e += chunk_sum[cc + lane];
-            e = __ockl_wfred_add_f64(e);
-            if (half)
-                e = e + chunk_sum[4u * p] + chunk_sum[4u * p + 1u];
-            const int base = __float_as_int((float)e) - (int)(kWindow / 2u);
-            bs[r] = base;
-            c[r] = __int_as_float(base + (int)cand);
-            const uint32_t j = min(2u * p + half, nseg - 1u);
-            src[r] = reinterpret_cast<const float4*>(scratch + kSegment * j);
-            if (cand == 0 && wave + kFusedWaves * r < npairs && 2u * p + half < nseg)
-                seg_base[2u * p + half] = base;
-        }
-        if (kPairsPerWave > 1 && wave + kFusedWaves < npairs) {
-            run_chains<kPairsPerWave>(c, src);
-        } else if (wave < npairs) {
-            float c1[1] = {c[0]};
-            const float4* const s1[1] = {src[0]};
-            run_chains<1>(c1, s1);
-            c[0] = c1[0];
-        }
-        // each pair's two segments composed in its own wave: candidate c of segment 2p ends at
-        // a value whose offset in segment 2p + 1's window names the lane that continued from
-        // it; an offset outside that window leaves the marker 0xffffffff (no candidate)
-#pragma unroll
-        for (int r = 0; r < kPairsPerWave; ++r) {
-            const uint32_t pr = wave + kFusedWaves * r;
-            const uint32_t idx = (uint32_t)__float_as_int(c[r]) - (uint32_t)__builtin_amdgcn_readlane(bs[r], 32);
-            const float nxt = __shfl(c[r], (int)(32u + (idx & (kWindow - 1u))));
-            const float comp = 2u * pr + 1u >= nseg ? c[r] : idx < kWindow ? nxt : __int_as_float(-1);
-            if (pr < npairs) {
-                seg_end[pr * 64u + lane] = c[r];
-                if (lane < kWindow)
-                    seg_comp[pr * kWindow + lane] = comp;
-            }
-        }
-        lds_barrier();
-        // the walk (wave 0) over the composed pairs: bits of the running sum, uniform across
-        // the wave
-        if (wave == 0) {
-            float comps[kPairs];
-#pragma unroll
-            for (uint32_t m = 0; m < kPairs; ++m)
-                comps[m] = seg_comp[min(m, npairs - 1u) * kWindow + (lane & (kWindow - 1u))];
-            const int bases = seg_base[min(lane, nseg - 1u)];
-            // branch-free lookups (a scalar branch per step costs more than the step); an
-            // offset outside a window sets a bit above the window's in `any`, a composed miss
-            // leaves the marker (caught by the next offset, or at the end), and either repeats
-            // the walk below
-            uint32_t v = 0, any = 0;
-            if (npairs == kPairs) {
-#pragma unroll
-                for (uint32_t m = 0; m < kPairs; ++m) {
-                    const uint32_t idx = v - (uint32_t)__builtin_amdgcn_readlane(bases, 2u * m);
-                    any |= idx;
-                    v = (uint32_t)__builtin_amdgcn_readlane(__float_as_int(comps[m]), (int)(idx & (kWindow - 1u)));
-                }
-            } else {
-#pragma unroll
-                for (uint32_t m = 0; m < kPairs; ++m) {
-                    const uint32_t idx = v - (uint32_t)__builtin_amdgcn_readlane(bases, 2u * m);
-                    const uint32_t nv =
-                        (uint32_t)__builtin_amdgcn_readlane(__float_as_int(comps[m]), (int)(idx & (kWindow - 1u)));
-                    const bool live = m < npairs;
-                    any |= live ? idx : 0u;
-                    v = live ? nv : v;
-                }
-            }
-            const uint32_t miss = (any & ~(kWindow - 1u)) | (uint32_t)(v == 0xffffffffu);
-            if (miss) {  // the walk with term-by-term additions where the running sum is no candidate
-                v = 0;
-                for (uint32_t j = 0; j < nseg; ++j) {
-                    const uint32_t idx = v - (uint32_t)seg_base[j];
-                    if (idx < kWindow)
-                        v = __float_as_uint(seg_end[(j / 2u) * 64u + (j & 1u) * 32u + idx]);
-                    else
-                        v = __float_as_uint(add_in_order_lds(scratch + kSegment * j, kSegment, __uint_as_float(v)));
-                }
-            }
-            if (lane == 0)
-                rms_s = sqrtf(__uint_as_float(v) / (float)K + fa.eps);
-        }
-        lds_barrier();
-        const float rms = rms_s;
+        const float rms = row_rms<EPT>(xv, K, fa.eps, scratch, sum_lds);
         if (!__builtin_isfinite(rms) || rms == 0.0f) {
             if (tid == 0) {
                 if (fa.err)

@@ -210,6 +210,22 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
 // (bnn_fused.hip).
 hipError_t launch_fused(hipStream_t stream, const FusedArgs& args, uint32_t tiles, uint32_t grid, uint64_t seq,
                         uint64_t* flag, uint64_t* host_status);
+// The pre-operation of a multi-row launch (BNNX_LaunchRows): row r of a, b and a_out starts
+// at r * width; the quantised rows and their scales go to q [rows][width] and rscale [rows].
+struct RowsArgs {
+    const float* a;     // RMSNORM: x; SILU_MUL: gate
+    const float* b;     // RMSNORM: residual (may be null); SILU_MUL: up
+    const float* gain;  // RMSNORM
+    float* a_out;       // RMSNORM: receives x + residual (may be null)
+    int8_t* q;
+    float* rscale;
+    int32_t* err;       // set to err_code when the RMSNORM check fails (may be null)
+    int32_t err_code;
+    float eps;
+    uint32_t width, rows;
+    int32_t kind;       // PRE_RMSNORM or PRE_SILU_MUL
+};
+hipError_t launch_rows(hipStream_t stream, const RowsArgs& args, uint64_t seq, uint64_t* flag, uint64_t* host_status);
 // One layer of a chained batch (BNNX_BatchCreateChain): a GEMM_F32 matrix and the
 // optional mapping of its outputs, out = post_scale * y + post_bias, then ReLU.
 struct ChainLayer {

@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "bnn-accelerator-hip.h"
+#include "attn_rows.h"
 #include "resident.h"
 
 #define BNNE_EXPF_QUALIFIER static __device__ __forceinline__
@@ -1047,6 +1048,14 @@ struct Resident {
     bool allow_fused, fused;
     BNNX_Batch *qkv, *attn_out, *gate_up, *down;
     BNNX_Batch lm_head;
+    // prefill: the activations of a block of block_rows prompt tokens (made by the first call
+    // with more than one token), block_out written by the linear layers and block_in read by
+    // them as buffers of the accelerator, the residual stream and the scores of one layer
+    uint32_t block_rows;
+    BNN_Buffer b_block_out, b_block_in;
+    float *block_out, *block_in, *block_x;
+    float* block_scores;
+    size_t block_score_floats;
     const SignLinear** lin;  // [7 * L + 1]: per layer q, k, v, o, gate, up, down; then lm_head
     uint64_t jobs_per_token, macs_per_token, lm_jobs, lm_macs;
 };
@@ -1414,10 +1423,12 @@ void resident_free(Resident* r) {
     std::free(r->gate_up);
     std::free(r->down);
     std::free(r->lin);
-    for (BNN_Buffer b : {r->b_norm, r->b_q, r->b_k, r->b_v, r->b_y, r->b_o, r->b_gate, r->b_up, r->b_h, r->b_logits})
+    for (BNN_Buffer b : {r->b_norm, r->b_q, r->b_k, r->b_v, r->b_y, r->b_o, r->b_gate, r->b_up, r->b_h, r->b_logits,
+                         r->b_block_out, r->b_block_in})
         BNN_BufferFree(b);
     for (void* p : {(void*)r->x, (void*)r->x2, (void*)r->kc, (void*)r->vc, (void*)r->scores, (void*)r->gains, (void*)r->rope_cos,
-                    (void*)r->rope_sin, (void*)r->emb_bits, (void*)r->emb_scales, (void*)r->err, (void*)r->keys})
+                    (void*)r->rope_sin, (void*)r->emb_bits, (void*)r->emb_scales, (void*)r->err, (void*)r->keys,
+                    (void*)r->block_x, (void*)r->block_scores})
         if (p)
             (void)hipFree(p);
     if (r->pinned)
@@ -1533,6 +1544,204 @@ BNNE_Status step_error(Resident* r, int err) {
     return BNNE_OK;
 }
 
+// Prompt tokens in blocks.  A step of one token is ~170 dependent launches that leave most
+// of the chip idle; a block of tokens runs the same layers as multi-row launches (the linear
+// layers on the matrix cores, BNNX_LaunchRows; attention by attn_rows.hip) with every token's
+// operations in its own step's order, so the cache rows and the logits are the same bits.
+constexpr uint32_t kBlockMinTokens = 3;             // two tokens: 2.1 ms as a block, 2.0 ms one after the other
+constexpr uint32_t kBlockRows = 1024;               // most tokens of a block
+constexpr size_t kBlockScoreFloats = 128u << 20;    // most scores of a block (512 MB)
+
+// Where the parts of a block live, in floats.
+struct BlockLayout {
+    size_t q, k, v, o, gate, up;  // in block_out
+    size_t out_floats, in_floats;
+    BlockLayout(const Resident* r, uint32_t rows) {
+        const size_t n = rows;
+        q = 0, k = q + n * r->C, v = k + n * r->kv_dim, o = v + n * r->kv_dim;
+        gate = o + n * r->C, up = gate + n * r->FF, out_floats = up + n * r->FF;
+        in_floats = n * std::max(r->C, r->FF);  // y; also the unused input view of the wider layers
+    }
+};
+
+// Tokens per block for a call of n tokens from pos0: bounded by the scores of the last block.
+uint32_t block_rows_for(const Resident* r, uint32_t n, uint32_t pos0) {
+    const size_t pitch = ((size_t)pos0 + n + 63u) & ~(size_t)63u;
+    const size_t fit = kBlockScoreFloats / (pitch * r->H);
+    const size_t rows = std::min<size_t>(kBlockRows, std::max<size_t>(fit, 1u));
+    return n <= rows ? n : (uint32_t)(rows >= 64u ? rows & ~(size_t)63u : rows);
+}
+
+void release_block(Resident* r) {
+    (void)hipStreamSynchronize(r->stream);
+    BNN_BufferFree(r->b_block_out);
+    BNN_BufferFree(r->b_block_in);
+    if (r->block_x)
+        (void)hipFree(r->block_x);
+    r->b_block_out = r->b_block_in = nullptr;
+    r->block_x = nullptr;
+    r->block_rows = 0;
+}
+
+// Memory for blocks of `rows` tokens and `scores` scores; grown by doubling, since giving
+// buffers back makes every prepared batch of the device stale.
+BNNE_Status ready_block(Resident* r, uint32_t rows, size_t scores) {
+    BNNE_Status st = BNNE_OK;
+    if (rows > r->block_rows) {
+        rows = std::min(std::max(rows, 2u * r->block_rows), kBlockRows);
+        if (r->block_rows)
+            release_block(r);
+        const BlockLayout at(r, rows);
+        st = alloc_buffer(r, at.out_floats, &r->b_block_out, &r->block_out);
+        if (st == BNNE_OK)
+            st = alloc_buffer(r, at.in_floats, &r->b_block_in, &r->block_in);
+        if (st == BNNE_OK)
+            st = upload(&r->block_x, nullptr, 2u * (size_t)rows * r->C * sizeof(float));
+        if (st != BNNE_OK) {
+            r->block_x = nullptr;
+            release_block(r);
+            return st;
+        }
+        r->block_rows = rows;
+    }
+    if (scores > r->block_score_floats) {
+        if (r->block_scores) {
+            (void)hipStreamSynchronize(r->stream);
+            (void)hipFree(r->block_scores);
+        }
+        r->block_score_floats = 0;
+        r->block_scores = nullptr;
+        st = upload(&r->block_scores, nullptr, scores * sizeof(float));
+        if (st == BNNE_OK)
+            r->block_score_floats = scores;
+        else
+            r->block_scores = nullptr;
+    }
+    return st;
+}
+
+// The jobs of one block-wide launch: `rows` rows of each layer from the given place of
+// block_out, reading block_in (with BNNX_PRE_ROW; otherwise the pre-operation's operands).
+BNNE_Status launch_block(Resident* r, uint32_t rows, std::initializer_list<std::pair<const SignLinear*, size_t>> parts,
+                         const BNNX_PreOp& pre) {
+    BNN_Job jobs[4];
+    uint32_t n = 0;
+    for (const auto& p : parts) {
+        BNN_Job& j = jobs[n++];
+        j = BNN_Job{};
+        j.operation = BNN_OP_GEMM_F32;
+        j.matrix = p.first->shards()[0].matrix;
+        j.input = BNN_BufferView{r->b_block_in, BNN_TYPE_F32, 0, 0};
+        j.output = BNN_BufferView{r->b_block_out, BNN_TYPE_F32, p.second * sizeof(float), 0};
+        j.rows = rows;
+    }
+    return accel_status(BNNX_LaunchRows(r->dev, jobs, n, &pre), "BNNX_LaunchRows");
+}
+
+// Whether the block path takes this model: the fused step's shapes, every layer one matrix.
+bool block_path(const Resident* r) {
+    if (!r->fused || r->HD != kRowsHeadDim)
+        return false;
+    for (size_t i = 0; i < 7 * (size_t)r->L; ++i)
+        if (r->lin[i]->shards().size() != 1)
+            return false;
+    return true;
+}
+
+// The launches of `rows` tokens (tokens_dev) at positions pos0 .. pos0 + rows - 1; leaves the
+// last token's residual stream in x and o, where the lm_head batch reads them.
+BNNE_Status enqueue_block(Resident* r, const int32_t* tokens_dev, uint32_t rows, uint32_t pos0, bool first) {
+    const uint32_t C = r->C, HD = r->HD;
+    const BlockLayout at(r, r->block_rows);
+    float* const x = r->block_x;
+    float* const x2 = x + (size_t)r->block_rows * C;
+    float* const o = r->block_out + at.o;
+    const float* attn_norm = r->gains;
+    const float* ffn_norm = r->gains + (size_t)r->L * C;
+    const float* q_norm = r->gains + 2 * (size_t)r->L * C;
+    const float* k_norm = q_norm + (size_t)r->L * HD;
+    launch_embed_rows(r->stream, tokens_dev, rows, r->emb_bits, r->emb_scales, C, x, first ? r->err : nullptr,
+                      first ? r->logit_bad : nullptr);
+    BNNE_Status st = BNNE_OK;
+    for (uint32_t l = 0; l < r->L && st == BNNE_OK; ++l) {
+        const SignLinear* const* p = r->lin + 7 * (size_t)l;
+        BNNX_PreOp norm{};
+        norm.kind = BNNX_PRE_RMSNORM;
+        norm.width = C;
+        norm.a = x;
+        norm.b = l ? o : nullptr;
+        norm.gain = attn_norm + (size_t)l * C;
+        norm.a_out = x2;
+        norm.eps = r->eps;
+        norm.err = r->err;
+        norm.err_code = 1;
+        st = launch_block(r, rows, {{p[0], at.q}, {p[1], at.k}, {p[2], at.v}}, norm);
+        if (st != BNNE_OK)
+            break;
+        AttnRows a{};
+        a.rows = rows, a.pos0 = pos0;
+        a.heads = r->H, a.kv_heads = r->Hk, a.kv_dim = r->kv_dim;
+        a.eps = r->eps, a.scale = 1.0f / sqrtf((float)HD);
+        a.q = r->block_out + at.q, a.k = r->block_out + at.k, a.v = r->block_out + at.v;
+        a.q_gain = q_norm + (size_t)l * HD, a.k_gain = k_norm + (size_t)l * HD;
+        a.cosv = r->rope_cos, a.sinv = r->rope_sin;
+        a.kc = r->kc + (size_t)l * r->n_ctx * r->kv_dim, a.vc = r->vc + (size_t)l * r->n_ctx * r->kv_dim;
+        a.scores = r->block_scores, a.score_pitch = (pos0 + rows + 63u) & ~63u;
+        a.y = r->block_in;
+        a.err = r->err;
+        launch_attn_rows(r->stream, a);
+        BNNX_PreOp row{};
+        row.kind = BNNX_PRE_ROW;
+        row.width = C;
+        st = launch_block(r, rows, {{p[3], at.o}}, row);
+        if (st != BNNE_OK)
+            break;
+        norm.a = x2;
+        norm.b = o;
+        norm.gain = ffn_norm + (size_t)l * C;
+        norm.a_out = x;
+        st = launch_block(r, rows, {{p[4], at.gate}, {p[5], at.up}}, norm);
+        if (st != BNNE_OK)
+            break;
+        BNNX_PreOp silu{};
+        silu.kind = BNNX_PRE_SILU_MUL;
+        silu.width = r->FF;
+        silu.a = r->block_out + at.gate;
+        silu.b = r->block_out + at.up;
+        st = launch_block(r, rows, {{p[6], at.o}}, silu);
+    }
+    if (st != BNNE_OK)
+        return st;
+    const size_t last = (size_t)(rows - 1u) * C;
+    hipError_t e = hipMemcpyAsync(r->x, x + last, (size_t)C * sizeof(float), hipMemcpyDeviceToDevice, r->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(r->o, o + last, (size_t)C * sizeof(float), hipMemcpyDeviceToDevice, r->stream);
+    return e == hipSuccess ? BNNE_OK : hip_error(e, "last token's row");
+}
+
+// Every block of a call's tokens, then the lm_head of the last one (when `head`).  The tokens
+// are staged through the pinned words that greedy runs return theirs in (calls are
+// synchronous: neither is in use).
+BNNE_Status enqueue_blocks(Resident* r, const int32_t* tokens, uint32_t n, uint32_t pos0, bool head) {
+    const uint32_t rows = block_rows_for(r, n, pos0);
+    const size_t pitch = ((size_t)pos0 + n + 63u) & ~(size_t)63u;
+    BNNE_Status st = ready_block(r, rows, pitch * r->H * rows);
+    if (st == BNNE_OK)
+        st = ready_batches(r);  // growing the block frees buffers, which makes batches stale
+    if (st != BNNE_OK)
+        return st;
+    std::memcpy(r->pinned_tokens, tokens, (size_t)n * sizeof(int32_t));
+    const hipError_t e =
+        hipMemcpyAsync(r->tokens_dev, r->pinned_tokens, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, r->stream);
+    if (e != hipSuccess)
+        return hip_error(e, "prompt tokens");
+    for (uint32_t t = 0; t < n && st == BNNE_OK; t += rows)
+        st = enqueue_block(r, r->tokens_dev + t, std::min(rows, n - t), pos0 + t, t == 0);
+    if (head && st == BNNE_OK)
+        st = accel_status(BNNX_BatchLaunch(r->lm_head), "BNNX_BatchLaunch");
+    return st;
+}
+
 }  // namespace
 
 BNNE_Status resident_step(bnne_context* c, Resident* r, const int32_t* tokens, uint32_t n, uint32_t pos0,
@@ -1542,18 +1751,41 @@ BNNE_Status resident_step(bnne_context* c, Resident* r, const int32_t* tokens, u
     if (e != hipSuccess)
         return hip_error(e, "hipSetDevice");
     BNNE_Status st = ready_batches(r);
-    for (uint32_t i = 0; i < n && st == BNNE_OK; ++i)
-        st = enqueue_token(r, pos0 + i, (uint32_t)tokens[i], nullptr, nullptr, nullptr, logits && i + 1 == n, i == 0);
-    e = hipGetLastError();
-    // the error word and the logits come back behind the last launch, into pinned memory
     int* const err_host = reinterpret_cast<int*>(r->pinned + r->V);
-    if (st == BNNE_OK && e == hipSuccess)
-        e = hipMemcpyAsync(err_host, r->err, sizeof(int), hipMemcpyDeviceToHost, r->stream);
-    if (st == BNNE_OK && e == hipSuccess && logits)
-        e = hipMemcpyAsync(r->pinned, r->logits_dev, (size_t)r->V * sizeof(float), hipMemcpyDeviceToHost, r->stream);
-    const uint64_t t1 = stats ? clock_ns() : 0;
-    const BNN_Status sync = BNNX_DeviceSynchronize(r->dev);
-    const uint64_t t2 = stats ? clock_ns() : 0;
+    uint64_t t1 = 0, t2 = 0;
+    BNN_Status sync = BNN_OK;
+    // enqueues the call's tokens, in blocks or one after another, and waits
+    const auto pass = [&](bool blocks) {
+        if (blocks)
+            st = enqueue_blocks(r, tokens, n, pos0, logits != nullptr);
+        for (uint32_t i = 0; i < n && st == BNNE_OK && !blocks; ++i)
+            st = enqueue_token(r, pos0 + i, (uint32_t)tokens[i], nullptr, nullptr, nullptr, logits && i + 1 == n,
+                               i == 0);
+        e = hipGetLastError();
+        // the error word and the logits come back behind the last launch, into pinned memory
+        if (st == BNNE_OK && e == hipSuccess)
+            e = hipMemcpyAsync(err_host, r->err, sizeof(int), hipMemcpyDeviceToHost, r->stream);
+        if (st == BNNE_OK && e == hipSuccess && logits)
+            e = hipMemcpyAsync(r->pinned, r->logits_dev, (size_t)r->V * sizeof(float), hipMemcpyDeviceToHost,
+                               r->stream);
+        t1 = stats ? clock_ns() : 0;
+        sync = BNNX_DeviceSynchronize(r->dev);
+        t2 = stats ? clock_ns() : 0;
+    };
+    bool blocks = st == BNNE_OK && n >= kBlockMinTokens && block_path(r);
+    if (st == BNNE_OK)
+        pass(blocks);
+    // A block that meets an error, or no memory for one: the tokens one after another, which
+    // is also what says which token's which check fails first (nothing of the failed pass
+    // remains: every cache row it wrote is written again before it is read).
+    if (blocks && e == hipSuccess && sync != BNN_EIO &&
+        (st == BNNE_ENOMEM || st == BNNE_ENOTSUP ||
+         (st == BNNE_OK && (sync != BNN_OK || *static_cast<volatile int*>(err_host) != kErrNone)))) {
+        forget_message();
+        st = ready_batches(r);
+        if (st == BNNE_OK)
+            pass(false);
+    }
     if (st != BNNE_OK)
         return st;
     if (e != hipSuccess)

@@ -163,6 +163,20 @@ BNN_Status BNNX_BatchCreateFusedPost(BNN_Device device, const BNN_Job* jobs, uin
                                      const BNNX_PostOp* post, BNNX_Batch* out_batch);
 
 /*
+ * A block of rows in one call: the jobs (at most 8, GEMM_F32 or GEMV_F32, all with the same
+ * rows <= 4096 and K = pre->width) run on one block of input rows produced by the
+ * pre-operation, as a fused batch's single row is: row r of a, b and a_out starts at
+ * r * width, the gain is shared, and with BNNX_PRE_ROW the rows are the jobs' input view
+ * (the same for every job).  Everything is checked, then enqueued on the device's stream;
+ * nothing is built or allocated and the call does not wait.  Results equal computing the
+ * rows on the host and calling BNN_Execute per job, bit for bit.  Statuses as
+ * BNNX_BatchCreateFused and BNNX_BatchLaunch; BNN_ENOTSUP for views that are not naturally
+ * aligned and for more rows than the device's 32 MiB scratch holds.  A block that holds an
+ * illegal row writes no job output, and the next BNNX_DeviceSynchronize reports it.
+ */
+BNN_Status BNNX_LaunchRows(BNN_Device device, const BNN_Job* jobs, uint32_t count, const BNNX_PreOp* pre);
+
+/*
  * Chained batches: GEMM_F32 layers applied in turn to every row of an input view.
  * Layer i computes, for each row, exactly what a GEMM_F32 job computes (check,
  * quantisation, group dots, FP32 accumulation in group order); when post_scale is

@@ -1,0 +1,163 @@
+"""Blocks of rows: BNNX_LaunchRows against the CPU oracle fed with host-computed rows, and the
+engine's prompt blocks against the same tokens decoded one call at a time (whose logits the
+fixtures of test_engine.py pin to the reference).  All comparisons bit for bit."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from bnn_cases import first_mismatch
+from conftest import load_pkg
+from test_engine import ERR, _engine_lib, write_error_model
+from test_fused import f32, host_rmsnorm, host_silu_mul
+
+pytestmark = pytest.mark.gpu
+PreOp = load_pkg().api.PreOp
+
+
+class Rows:
+    def __init__(self, pkg, dev, k, ns, rows, kind, with_b, seed=3):
+        self.pkg, self.dev, self.kind, self.k, self.rows, self.with_b = pkg, dev, kind, k, rows, with_b
+        rng = np.random.default_rng(seed + k + rows)
+        self.chunks = [pkg.synth.matrix(n, k, seed=seed, stream=i) for i, n in enumerate(ns)]
+        self.mats = [dev.matrix(b, s) for b, s in self.chunks]
+        self.a, self.b = f32(rng, (rows, k), 3.0), f32(rng, (rows, k), 0.5)
+        self.gain = (1.0 + 0.02 * rng.standard_normal(k)).astype(np.float32)
+        self.bufs = {name: dev.buffer(4 * rows * k) for name in ("a", "b", "gain", "x")}
+        self.outs = [dev.buffer(4 * rows * n) for n in ns]
+        self.err = dev.buffer(4)
+        self.write()
+        self.err.write(np.zeros(1, np.int32))
+        for o, n in zip(self.outs, ns):
+            o.write(np.full(rows * n, 5.0, np.float32))
+
+    def write(self):
+        for name in ("a", "b", "gain"):
+            self.bufs[name].write(getattr(self, name))
+
+    def launch(self):
+        pkg, T = self.pkg, self.pkg.Type.F32
+        jobs = (pkg.Job * len(self.mats))(*[
+            pkg.Job(int(pkg.Op.GEMM_F32), m.handle.value, self.bufs["a"].view(T), o.view(T), self.rows)
+            for m, o in zip(self.mats, self.outs)])
+        ptr = {name: b.device_pointer() for name, b in self.bufs.items()}
+        pre = PreOp(self.kind, self.k)
+        if self.kind != PreOp.ROW:
+            pre.a, pre.b = ptr["a"], ptr["b"] if self.with_b else None
+        if self.kind == PreOp.RMSNORM:
+            pre.gain, pre.a_out, pre.eps, pre.err, pre.err_code = ptr["gain"], ptr["x"], 1e-6, self.err.device_pointer(), 7
+        st = self.dev.api.BNNX_LaunchRows(self.dev.handle, jobs, len(self.mats), ctypes.byref(pre))
+        return st, self.dev.api.BNNX_DeviceSynchronize(self.dev.handle)
+
+    def row(self, r):
+        b = self.b[r] if self.with_b else None
+        if self.kind == PreOp.RMSNORM:
+            return host_rmsnorm(self.a[r], b, self.gain, 1e-6)[1]
+        return host_silu_mul(self.a[r], b) if self.kind == PreOp.SILU_MUL else self.a[r]
+
+    def free(self):
+        for m in self.mats:
+            m.destroy()
+        for b in self.outs + list(self.bufs.values()) + [self.err]:
+            b.free()
+
+
+@pytest.mark.parametrize("k,ns,rows,kind,with_b", [
+    (128, [70], 1, PreOp.RMSNORM, True),
+    (2048, [256, 100, 64], 3, PreOp.RMSNORM, True),
+    (2176, [65], 5, PreOp.RMSNORM, False),
+    (6144, [130], 2, PreOp.RMSNORM, True),
+    (8192, [64], 17, PreOp.RMSNORM, True),
+    (6144, [200], 9, PreOp.SILU_MUL, True),
+    (384, [1000], 66, PreOp.SILU_MUL, True),
+    (2048, [96, 33], 40, PreOp.ROW, False),
+])
+def test_launch_rows(pkg, hipdev, oracle, k, ns, rows, kind, with_b):
+    f = Rows(pkg, hipdev, k, ns, rows, kind, with_b)
+    try:
+        print(f"rows {rows} x {k}, kind {kind}", flush=True)
+        assert f.launch() == (0, 0)
+        x = np.stack([f.row(r) for r in range(rows)])
+        with pkg.Device(oracle, 0) as ref:
+            for (bits, scales), out in zip(f.chunks, f.outs):
+                m = ref.matrix(bits, scales)
+                want = ref.run(pkg.Op.GEMM_F32, m, x)
+                m.destroy()
+                got = out.read().view(np.float32).reshape(want.shape)
+                assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), first_mismatch(got, want)
+        if kind == PreOp.RMSNORM:
+            stored = f.bufs["x"].read().view(np.float32).reshape(rows, k)
+            assert np.array_equal(stored, f.a + f.b if with_b else f.a)
+    finally:
+        f.free()
+
+
+@pytest.mark.parametrize("kind", [PreOp.ROW, PreOp.RMSNORM, PreOp.SILU_MUL])
+def test_launch_rows_illegal_row(pkg, hipdev, kind):
+    """One non-finite row: nothing of the block is written, the next synchronisation says so."""
+    f = Rows(pkg, hipdev, 256, [70], 20, kind, True)
+    try:
+        f.a[13, 200] = np.inf
+        f.write()
+        assert f.launch() == (0, pkg.Status.ERANGE)
+        assert (f.outs[0].read().view(np.float32) == 5.0).all()
+        assert f.err.read().view(np.int32)[0] == (7 if kind == PreOp.RMSNORM else 0)
+        f.a[13, 200] = 1.0
+        f.write()
+        assert f.launch() == (0, 0)
+    finally:
+        f.free()
+
+
+TINY = {"layers": 2, "hidden": 256, "heads": 2, "kv_heads": 1, "ffn": 512, "vocab": 512, "context": 2816}
+
+
+@pytest.mark.parametrize("count,split", [
+    (3, 0), (7, 2), (16, 0), (33, 1), (64, 0), (65, 0), (127, 63), (200, 0),
+    (1025, 0),      # a second block of one token
+    (1300, 40),     # two blocks behind a started cache
+    (2500, 1400),   # softmax rows of more than one LDS chunk
+])
+def test_prompt_blocks_match_single_tokens(pkg, hip, tmp_path, count, split):
+    path = tmp_path / "m.gguf"
+    pkg.gguf.qwen3_random(path, **TINY)
+    ids = np.random.default_rng(count).integers(0, TINY["vocab"], count, dtype=np.int32)
+    with pkg.Device(hip, 0) as dev:
+        m = pkg.engine.Model(_engine_lib(pkg), dev, path)
+        one, block = (pkg.engine.Context(m, n_ctx=TINY["context"]) for _ in range(2))
+        print(f"prompt of {count} tokens, {split} of them before the block", flush=True)
+        for t in ids[:-1]:
+            one.decode([t], want_logits=False)
+        want = one.decode(ids[-1:])
+        if split:
+            block.decode(ids[:split], want_logits=False)
+        got = block.decode(ids[split:])
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        # the caches are the same too: the next steps read every row
+        nxt = int(want.argmax())
+        assert block.decode_greedy(nxt, 3) == one.decode_greedy(nxt, 3)
+        for c in (one, block):
+            c.free()
+        m.free()
+
+
+def test_prompt_block_error_then_prompt(pkg, hip, tmp_path):
+    """A prompt whose middle token fails: the status of the single-token step, the position
+    unchanged; afterwards the clean prompt gives the reference's tokens."""
+    model_path, _, _ = write_error_model(pkg, tmp_path)
+    prompt = list(ERR["prompt"])
+    bad = prompt[:2] + [ERR["error_token"]] + prompt[2:]
+    with pkg.Device(hip, 0) as dev:
+        m = pkg.engine.Model(_engine_lib(pkg), dev, model_path)
+        c = pkg.engine.Context(m, n_ctx=ERR["ctx"])
+        with pytest.raises(pkg.engine.EngineError) as e:
+            c.decode(bad)
+        assert e.value.status == -7 and "RMSNorm" in str(e.value)
+        assert c.pos() == 0
+        first = int(c.decode(prompt).argmax())
+        want = [row[1] for row in ERR["steps"]]
+        assert [first] + c.decode_greedy(first, len(want) - 1) == want
+        c.free()
+        m.free()
