@@ -1569,8 +1569,11 @@ EXPORT BNN_Status BNNX_LaunchRows(BNN_Device device, const BNN_Job* jobs, uint32
         ra.kind = pre->kind;
         return launch_rows(device->stream, ra, seq, device->flag_dev, device->status_host + 1);
     });
-    for (uint32_t i = 0; e == hipSuccess && i < count; ++i) {
-        const GemmJob gj = make_gemm(plans[i], pj, plans[i].out_base, plans[i].out_stride);
+    for (uint32_t i = 0; e == hipSuccess && i < count; i += kGemmParts) {
+        GemmJob gj = make_gemm(plans[i], pj, plans[i].out_base, plans[i].out_stride);
+        for (uint32_t p = i + 1u; p < count && p < i + kGemmParts; ++p)
+            gj.parts[gj.extra++] = GemmPart{plans[p].m->wbits,   plans[p].m->wscale, plans[p].out_base,
+                                            plans[p].out_stride, plans[p].m->n,      plans[p].m->tiles, 0, 0};
         e = timed(device, KK_GEMM,
                   [&] { return launch_gemm(device->stream, gj, device->cu_count, seq, device->flag_dev); });
     }

@@ -85,6 +85,28 @@ __device__ __forceinline__ TileRC gemm_tile_of_block(uint32_t b, uint32_t grid, 
     return TileRC{bi * band + rest % width, rest / width};
 }
 
+// The tile's column tile within its part of the job, whose matrix and output `j` then
+// describes (wave-uniform: the argument block's loads and a few scalar selects, once).
+__device__ __forceinline__ uint32_t select_part(GemmJob& j, uint32_t nt) {
+    uint32_t first = 0;
+    if (j.extra != 0u) {
+#pragma unroll
+        for (uint32_t i = 0; i < kGemmParts - 1u; ++i) {
+            if (i < j.extra && nt >= j.parts[i].first) {
+                const GemmPart& p = j.parts[i];
+                j.wbits = p.wbits;
+                j.wscale = p.wscale;
+                j.out = p.out;
+                j.out_stride = p.out_stride;
+                j.n = p.n;
+                j.tiles = p.tiles;
+                first = p.first;
+            }
+        }
+    }
+    return nt - first;
+}
+
 // 16 bytes per active lane from global memory into LDS at lds_addr + 16 * lane (the
 // wave's LDS base goes in M0).  Inline assembly, so that the compiler's own wait
 // insertion does not add a wait for every LDS DMA before each later LDS read: the
@@ -185,7 +207,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WGN, wn = wave % WGN;
-    const TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
     const uint32_t mt = tile.mt, nt = tile.nt;
     const uint32_t m0 = mt * TM, n0 = nt * TN;
     const uint32_t groups = j.groups;
@@ -525,7 +548,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WGN, wn = wave % WGN;
-    const TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
     const uint32_t m0 = tile.mt * TM, n0 = tile.nt * TN;
     const uint32_t groups = j.groups;
     unsigned char* const lds_a = smem;
@@ -753,10 +777,11 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
 }
 
 uint32_t gemm_band(const GemmJob& job, uint32_t mtiles);
+uint32_t gemm_ntiles(GemmJob& job, uint32_t tn);
 
 template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_co(hipStream_t stream, const GemmJob& job, uint64_t seq, const uint64_t* flag) {
-    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = (job.n + TN - 1u) / TN;
+hipError_t launch_co(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
     launch_kernel((k_gemm_co<TM, TN, WGM, WGN>), dim3(mtiles * ntiles), dim3(64 * WGM * WGN), 0, stream, job, mtiles,
                   ntiles, gemm_band(job, mtiles), seq, flag);
     return hipGetLastError();
@@ -801,7 +826,8 @@ __global__ __launch_bounds__(64 * W) void k_gemm_ks(GemmJob j, uint32_t mtiles, 
         return;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
     const uint32_t mt = tile.mt, nt = tile.nt;
     const uint32_t m0 = mt * TM, n0 = nt * TN;
     // the row scales of this thread's outputs (F32 jobs), requested now (see k_gemm_kr)
@@ -985,7 +1011,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wv(GemmJob j, uint32_t mt
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WN, wn = wave % WN;
-    const TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
     const uint32_t m0 = tile.mt * TM + 16u * MS * wm, n0 = tile.nt * TN + 16u * NS * wn;
     const uint32_t groups = j.groups;
     for (uint32_t i = tid; i < 256u; i += NT)
@@ -1201,7 +1228,8 @@ __global__ __launch_bounds__(64 * W) void k_gemm_kr(GemmJob j, uint32_t mtiles, 
     const uint64_t failed_seq = *flag;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
     const uint32_t m0 = tile.mt * T::TM, n0 = tile.nt * T::TN;
     const uint32_t groups = j.groups;
     // the row scales of this thread's outputs (F32 jobs; the prep launch wrote them),
@@ -1413,7 +1441,8 @@ __global__ __launch_bounds__(64 * WN * KS) void k_gemm_kc(GemmJob j, uint32_t mt
     const uint64_t failed_seq = *flag;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
     const uint32_t m0 = tile.mt * T::TM, n0 = tile.nt * T::TN;
     // the row scales of this thread's outputs (F32 jobs), requested now (see k_gemm_kr)
     float rs[TMS][4];
@@ -1654,7 +1683,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, chunk = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WGN, wn = wave % WGN;
-    const TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
     const uint32_t m0 = tile.mt * TM, n0 = tile.nt * TN;
     const uint32_t groups = j.groups;
     uint2* const lut_all = reinterpret_cast<uint2*>(smem + T::OFF_LUT);
@@ -1868,7 +1898,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t 
 // into about 8 * band / mtiles L2s and the weights (1.125 bits each) into
 // mtiles / band of them; the band minimising the sum.
 uint32_t gemm_band(const GemmJob& job, uint32_t mtiles) {
-    const double a = (double)job.rows * job.k, b = (double)job.n * job.k * 0.140625;
+    double n = job.n;
+    for (uint32_t i = 0; i < job.extra; ++i)
+        n += job.parts[i].n;
+    const double a = (double)job.rows * job.k, b = n * job.k * 0.140625;
     uint32_t best = 1;
     double best_cost = 0.0;
     for (uint32_t band = 1; band <= mtiles; ++band) {
@@ -1880,57 +1913,67 @@ uint32_t gemm_band(const GemmJob& job, uint32_t mtiles) {
     return best;
 }
 
+// Column tiles of `tn` columns of every part of the job, whose first tiles it fills in.
+uint32_t gemm_ntiles(GemmJob& job, uint32_t tn) {
+    uint32_t t = (job.n + tn - 1u) / tn;
+    for (uint32_t i = 0; i < job.extra; ++i) {
+        job.parts[i].first = t;
+        t += (job.parts[i].n + tn - 1u) / tn;
+    }
+    return t;
+}
+
 template <int TMS, int TNS, int W, int DEPTH>
-hipError_t launch_ks(hipStream_t stream, const GemmJob& job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_ks(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
     const uint32_t mtiles = (job.rows + 16u * TMS - 1u) / (16u * TMS);
-    const uint32_t ntiles = (job.n + 16u * TNS - 1u) / (16u * TNS);
+    const uint32_t ntiles = gemm_ntiles(job, 16u * TNS);
     launch_kernel((k_gemm_ks<TMS, TNS, W, DEPTH>), dim3(mtiles * ntiles), dim3(64 * W), 0, stream, job, mtiles, ntiles,
                   gemm_band(job, mtiles), seq, flag);
     return hipGetLastError();
 }
 
 template <int TMS, int TNS, int W, int R>
-hipError_t launch_kr(hipStream_t stream, const GemmJob& job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_kr(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
     if (job.groups > (uint32_t)(W * R) || job.mode == MODE_DOT_I16)
         return hipErrorInvalidValue;  // the selection below never asks for this
     const uint32_t mtiles = (job.rows + 16u * TMS - 1u) / (16u * TMS);
-    const uint32_t ntiles = (job.n + 16u * TNS - 1u) / (16u * TNS);
+    const uint32_t ntiles = gemm_ntiles(job, 16u * TNS);
     launch_kernel((k_gemm_kr<TMS, TNS, W, R>), dim3(mtiles * ntiles), dim3(64 * W), 0, stream, job, mtiles, ntiles,
                   gemm_band(job, mtiles), seq, flag);
     return hipGetLastError();
 }
 
 template <int TMS, int TNW, int WN, int KS, int G>
-hipError_t launch_kc(hipStream_t stream, const GemmJob& job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_kc(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
     if (job.groups > (uint32_t)G || job.mode == MODE_DOT_I16)
         return hipErrorInvalidValue;  // the selection below never asks for this
     const uint32_t mtiles = (job.rows + 16u * TMS - 1u) / (16u * TMS);
-    const uint32_t ntiles = (job.n + 16u * TNW * WN - 1u) / (16u * TNW * WN);
+    const uint32_t ntiles = gemm_ntiles(job, 16u * TNW * WN);
     launch_kernel((k_gemm_kc<TMS, TNW, WN, KS, G>), dim3(mtiles * ntiles), dim3(64 * WN * KS), 0, stream, job, mtiles,
                   ntiles, gemm_band(job, mtiles), seq, flag);
     return hipGetLastError();
 }
 
 template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_mx(hipStream_t stream, const GemmJob& job, uint64_t seq, const uint64_t* flag) {
-    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = (job.n + TN - 1u) / TN;
+hipError_t launch_mx(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
     launch_kernel((k_gemm_mx<TM, TN, WGM, WGN>), dim3(mtiles * ntiles), dim3(64 * WGM * WGN), 0, stream, job,
                   mtiles, ntiles, gemm_band(job, mtiles), seq, flag);
     return hipGetLastError();
 }
 
 template <int MS, int NS, int WM, int WN, int DEPTH>
-hipError_t launch_wv(hipStream_t stream, const GemmJob& job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_wv(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
     constexpr uint32_t TM = 16u * MS * WM, TN = 16u * NS * WN;
-    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = (job.n + TN - 1u) / TN;
+    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
     launch_kernel((k_gemm_wv<MS, NS, WM, WN, DEPTH>), dim3(mtiles * ntiles), dim3(64 * WM * WN), 0, stream, job,
                   mtiles, ntiles, gemm_band(job, mtiles), seq, flag);
     return hipGetLastError();
 }
 
 template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_bits(hipStream_t stream, const GemmJob& job, uint64_t seq, const uint64_t* flag) {
-    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = (job.n + TN - 1u) / TN;
+hipError_t launch_bits(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
     const dim3 grid(mtiles * ntiles), block(64 * WGM * WGN);
     const uint32_t band = gemm_band(job, mtiles);
     if (job.mode == MODE_DOT_I16)
@@ -1950,7 +1993,10 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
                        const uint64_t* flag) {
     const uint64_t cus = cu_count ? cu_count : 256u;
     auto blocks = [&](uint32_t tm, uint32_t tn) {
-        return (uint64_t)((job.rows + tm - 1u) / tm) * ((job.n + tn - 1u) / tn);
+        uint64_t cols = (job.n + tn - 1u) / tn;
+        for (uint32_t i = 0; i < job.extra; ++i)
+            cols += (job.parts[i].n + tn - 1u) / tn;
+        return (uint64_t)((job.rows + tm - 1u) / tm) * cols;
     };
 #ifndef BNN_GEMM_CO
 #define BNN_GEMM_CO 1  // F32-accumulating jobs with a 128 x 128 tile per CU: two workgroups per CU (k_gemm_co)

@@ -87,7 +87,19 @@ struct DotJob {
 };
 
 // One multi-row job on the matrix cores (rows >= kMfmaMinRows), read from the
-// matrix's resident layout (sign bits unpacked in LDS by the kernel).
+// matrix's resident layout (sign bits unpacked in LDS by the kernel).  Up to kGemmParts
+// matrices of one k may share the rows (the q, k and v projections of a block of tokens): the
+// job's own fields describe the first, parts[] the others, whose column tiles follow the
+// first's; column tile t of the launch belongs to the last part with first <= t (first is set
+// by the launcher, in column tiles of the kernel it picks).
+struct GemmPart {
+    const uint4* wbits;
+    const uint16_t* wscale;
+    unsigned char* out;
+    uint64_t out_stride;
+    uint32_t n, tiles, first, pad_;
+};
+constexpr uint32_t kGemmParts = 4;
 struct GemmJob {
     const uint4* wbits;       // matrix layout [tiles][groups][64] x 16 bytes
     const uint16_t* wscale;   // matrix layout [tiles][groups][64]
@@ -98,6 +110,8 @@ struct GemmJob {
     uint32_t n, k, groups, tiles;  // tiles of 64 features, as in the matrix layout
     uint32_t rows;
     int32_t mode;
+    uint32_t extra, pad_;          // parts in use
+    GemmPart parts[kGemmParts - 1];
 };
 
 // Rows from which a job runs on the matrix cores instead of the bit-plane kernel.
