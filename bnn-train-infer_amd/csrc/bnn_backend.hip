@@ -370,6 +370,7 @@ EXPORT BNN_Status BNN_DeviceClose(BNN_Device device) {
     if (device->table_dev)
         (void)hipFree(device->table_dev);
     free(device->batch_jobs);
+    free(device->batch_gemms);
     destroy_events(device);
     (void)hipHostFree(device->status_host);
     (void)hipFree(device->flag_dev);
@@ -767,6 +768,12 @@ GemmJob make_gemm(const JobPlan& p, const PrepJob& pj, unsigned char* out, size_
     return j;
 }
 
+// `more` as a further part of the launch of `j` (equal k, rows and mode).
+void add_part(GemmJob* j, const GemmJob& more) {
+    j->parts[j->extra++] =
+        GemmPart{more.wbits, more.wscale, more.q, more.rscale, more.out, more.out_stride, more.n, more.tiles, 0, 0};
+}
+
 // Completion of a single-row launch whose `grid` workgroups each store seq into their own
 // pinned word (status_host from kDoneFlagWord) once their results are visible to the host:
 // spin on those instead of waiting for the end of the kernel, which the runtime reports
@@ -1017,27 +1024,106 @@ BNN_Status ensure_tables(BNN_Device d, size_t bytes) {
     return BNN_OK;
 }
 
+// How a batch runs a job: with the dot launch, or as a part of matrix-core launch `gemm`.
+struct BatchPlace {
+    uint32_t gemm;  // kNoGemm: the dot launch
+    uint32_t prep;  // the job whose quantised rows it reads (itself, or one with the same input view)
+    size_t at;      // its own quantised rows' offset in the batch's scratch
+};
+constexpr uint32_t kNoGemm = 0xffffffffu;
+
 // All checks of a batch (per job as BNN_Execute, then the batch rules) and the
 // sizes of its scratch and job tables.
 struct BatchPlan {
     JobPlan* plans = nullptr;
-    uint32_t count = 0;
-    bool needs_nearest = false, uniform = true;
+    BatchPlace* places = nullptr;
+    uint32_t count = 0, gemm_count = 0;
+    bool needs_nearest = false, uniform = true, scales = false;
     uint64_t prep_blocks = 0, dot_items_total = 0;
+    uint32_t prep_jobs = 0, dot_jobs = 0;
     size_t scratch_bytes = 0;
-    uint32_t max_groups = 0;
-    // tables: PrepJob[count] | DotJob[count] | prep block->job (unless one row per job) |
+    uint32_t max_groups = 0;    // of every job (the prep launch)
+    uint32_t dot_groups = 0;    // of the jobs of the dot launch
+    uint32_t uniform_items = 0; // items of each of its jobs when they are equal, else 0
+    // tables: PrepJob[prep_jobs] | DotJob[dot_jobs] | prep block->job (unless one row per job) |
     // dot item->job (non-uniform only)
     size_t prep_tab = 0, dot_tab = 0, prep_map = 0, dot_map = 0, tables = 0;
-    ~BatchPlan() { free(plans); }
+    ~BatchPlan() {
+        free(plans);
+        free(places);
+    }
 };
+
+// Which jobs run on the matrix cores: groups of up to kGemmParts jobs of one k, one number of
+// rows (>= kBatchMfmaRows) and one mode, each group one launch of ~4 us and more, against
+// ~4 us for the one dot launch of every other job plus ~36 us per 10^9 weights times rows in
+// it (q/k/v of 8 / 64 / 256 rows 9.0 / 19.4 / 52 us a pass with dots, 7.9 / 8.4 / 15 us on
+// the matrix cores; 6144->6144 x 64 rows 60 against 22 us).  A group is worth its launch from
+// 0.11 * 10^9 on, or when it leaves the dot launch without work.
+constexpr uint32_t kBatchMfmaRows = 4;
+constexpr double kGemmGroupWork = 0.11e9;
+
+constexpr uint32_t kGemmLookAhead = 64;  // jobs behind its first that a group is filled from
+
+BNN_Status place_jobs(const BNN_Job* jobs, BatchPlan* bp) {
+    const uint32_t count = bp->count;
+    double* work = static_cast<double*>(malloc(sizeof(double) * count));  // of group g
+    if (work == nullptr)
+        return BNN_ENOMEM;
+    uint32_t groups = 0, small = 0, dots = 0;
+    for (uint32_t i = 0; i < count; ++i)
+        bp->places[i] = BatchPlace{kNoGemm, i, 0};
+    for (uint32_t i = 0; i < count; ++i) {
+        if (bp->places[i].gemm != kNoGemm)
+            continue;
+        if (jobs[i].rows < kBatchMfmaRows) {
+            ++dots;
+            continue;
+        }
+        const JobPlan& p = bp->plans[i];
+        work[groups] = 0.0;
+        for (uint32_t j = i, members = 0; j < count && j - i < kGemmLookAhead && members < kGemmParts; ++j) {
+            const JobPlan& o = bp->plans[j];
+            if (bp->places[j].gemm != kNoGemm || jobs[j].rows != jobs[i].rows || o.m->k != p.m->k || o.mode != p.mode)
+                continue;
+            bp->places[j].gemm = groups;
+            work[groups] += (double)jobs[j].rows * o.m->n * o.m->k;
+            ++members;
+        }
+        small += work[groups] < kGemmGroupWork;
+        ++groups;
+    }
+    // small groups go with the dots, unless the only one is all that the dots would have
+    const bool keep_small = small == 0 || (small == 1 && dots == 0);
+    uint32_t kept = 0;
+    for (uint32_t g = 0; g < groups; ++g)
+        work[g] = keep_small || work[g] >= kGemmGroupWork ? (double)kept++ : -1.0;  // the group's new number
+    for (uint32_t i = 0; i < count; ++i)
+        if (bp->places[i].gemm != kNoGemm) {
+            const double to = work[bp->places[i].gemm];
+            bp->places[i].gemm = to < 0.0 ? kNoGemm : (uint32_t)to;
+        }
+    bp->gemm_count = kept;
+    free(work);
+    return BNN_OK;
+}
+
+// Scratch of the quantised rows of job i of a batch: bit planes and sums for the dots, Q for
+// the matrix cores, and the row scales.
+size_t job_scratch_bytes(const BatchPlan& bp, uint32_t i, uint32_t rows) {
+    size_t a, b, c;
+    if (bp.places[i].gemm == kNoGemm)
+        return row_scratch_bytes(bp.plans[i], rows, &a, &b, &c);
+    return round_up((size_t)rows * bp.plans[i].m->k, 256) + round_up(rows * 4u, 256);
+}
 
 BNN_Status plan_batch(BNN_Device device, const BNN_Job* jobs, uint32_t count, BatchPlan* bp) {
     bp->plans = static_cast<JobPlan*>(malloc(sizeof(JobPlan) * count));
+    bp->places = static_cast<BatchPlace*>(malloc(sizeof(BatchPlace) * count));
     bp->count = count;
     Extent* outs = static_cast<Extent*>(malloc(sizeof(Extent) * count));
     const void** ins = static_cast<const void**>(malloc(sizeof(void*) * count));
-    BNN_Status st = bp->plans && outs && ins ? BNN_OK : BNN_ENOMEM;
+    BNN_Status st = bp->plans && bp->places && outs && ins ? BNN_OK : BNN_ENOMEM;
     for (uint32_t i = 0; st == BNN_OK && i < count; ++i) {
         st = plan_job(device, &jobs[i], &bp->plans[i]);
         if (st != BNN_OK)
@@ -1048,21 +1134,47 @@ BNN_Status plan_batch(BNN_Device device, const BNN_Job* jobs, uint32_t count, Ba
             break;
         }
         bp->needs_nearest = bp->needs_nearest || !p.dot_out;
-        size_t a, b, c;
-        bp->scratch_bytes += row_scratch_bytes(p, jobs[i].rows, &a, &b, &c);
-        bp->prep_blocks += jobs[i].rows;
         bp->max_groups = p.m->groups > bp->max_groups ? p.m->groups : bp->max_groups;
         outs[i].buffer = jobs[i].output.buffer;
         outs[i].begin = jobs[i].output.offset;
         outs[i].end = jobs[i].output.offset + (size_t)(jobs[i].rows - 1) * p.out_stride + p.out_row;
         ins[i] = jobs[i].input.buffer;
     }
-    // work items per job depend on the batch's largest group count
+    if (st == BNN_OK)
+        st = place_jobs(jobs, bp);
     for (uint32_t i = 0; st == BNN_OK && i < count; ++i) {
-        const uint64_t items = dot_items(bp->plans[i].m->tiles, jobs[i].rows, bp->max_groups);
-        bp->uniform = bp->uniform && items == dot_items(bp->plans[0].m->tiles, jobs[0].rows, bp->max_groups);
+        const JobPlan& p = bp->plans[i];
+        if (bp->places[i].gemm == kNoGemm) {
+            bp->dot_groups = p.m->groups > bp->dot_groups ? p.m->groups : bp->dot_groups;
+            bp->scales = bp->scales || !p.dot_out;
+            ++bp->dot_jobs;
+        } else {
+            // parts of one launch that read one view share its quantised rows
+            for (uint32_t j = i > kGemmLookAhead ? i - kGemmLookAhead : 0; j < i; ++j)
+                if (bp->places[j].gemm == bp->places[i].gemm && bp->plans[j].in_base == p.in_base &&
+                    bp->plans[j].in_stride == p.in_stride && bp->plans[j].f32_in == p.f32_in) {
+                    bp->places[i].prep = bp->places[j].prep;
+                    break;
+                }
+        }
+        if (bp->places[i].prep != i)
+            continue;
+        bp->places[i].at = bp->scratch_bytes;
+        bp->scratch_bytes += job_scratch_bytes(*bp, i, jobs[i].rows);
+        bp->prep_blocks += jobs[i].rows;
+        ++bp->prep_jobs;
+    }
+    // work items per job depend on the dot launch's largest group count
+    for (uint32_t i = 0; st == BNN_OK && i < count; ++i) {
+        if (bp->places[i].gemm != kNoGemm)
+            continue;
+        const uint32_t items = dot_items(bp->plans[i].m->tiles, jobs[i].rows, bp->dot_groups);
+        bp->uniform = bp->uniform && (bp->uniform_items == 0 || items == bp->uniform_items);
+        bp->uniform_items = items;
         bp->dot_items_total += items;
     }
+    if (!bp->uniform)
+        bp->uniform_items = 0;
     // the jobs run concurrently: no output buffer may be an input buffer, and
     // outputs sharing a buffer may not overlap
     if (st == BNN_OK) {
@@ -1080,9 +1192,9 @@ BNN_Status plan_batch(BNN_Device device, const BNN_Job* jobs, uint32_t count, Ba
     free(outs);
     free(ins);
     if (st == BNN_OK) {
-        bp->prep_tab = round_up(sizeof(PrepJob) * count, 256);
-        bp->dot_tab = round_up(sizeof(DotJob) * count, 256);
-        bp->prep_map = bp->prep_blocks == count ? 0 : round_up(4u * bp->prep_blocks, 256);
+        bp->prep_tab = round_up(sizeof(PrepJob) * bp->prep_jobs, 256);
+        bp->dot_tab = round_up(sizeof(DotJob) * bp->dot_jobs, 256);
+        bp->prep_map = bp->prep_blocks == bp->prep_jobs ? 0 : round_up(4u * bp->prep_blocks, 256);
         bp->dot_map = bp->uniform ? 0 : round_up(4u * bp->dot_items_total, 256);
         bp->tables = bp->prep_tab + bp->dot_tab + bp->prep_map + bp->dot_map;
     }
@@ -1090,38 +1202,62 @@ BNN_Status plan_batch(BNN_Device device, const BNN_Job* jobs, uint32_t count, Ba
 }
 
 // Writes the job tables of a planned batch into host memory, with the rows'
-// quantised forms placed consecutively from 'scratch' (a device address).
-void fill_batch_tables(const BatchPlan& bp, const BNN_Job* jobs, unsigned char* scratch, unsigned char* host) {
+// quantised forms placed consecutively from 'scratch' (a device address), and its
+// matrix-core launches into `gemms` [gemm_count].
+void fill_batch_tables(const BatchPlan& bp, const BNN_Job* jobs, unsigned char* scratch, unsigned char* host,
+                       GemmJob* gemms) {
     PrepJob* hp = reinterpret_cast<PrepJob*>(host);
     DotJob* hd = reinterpret_cast<DotJob*>(host + bp.prep_tab);
     uint32_t* hpm = reinterpret_cast<uint32_t*>(host + bp.prep_tab + bp.dot_tab);
     uint32_t* hdm = reinterpret_cast<uint32_t*>(host + bp.prep_tab + bp.dot_tab + bp.prep_map);
-    size_t soff = 0;
-    uint32_t pb = 0, di = 0;
+    uint32_t pj = 0, pb = 0, dj = 0, di = 0;
+    for (uint32_t g = 0; g < bp.gemm_count; ++g)
+        gemms[g] = GemmJob{};
     for (uint32_t i = 0; i < bp.count; ++i) {
         const JobPlan& p = bp.plans[i];
+        const BatchPlace& place = bp.places[i];
         const uint32_t rows = jobs[i].rows;
-        size_t a, b, c;
-        hp[i] = make_prep(p, p.in_base, rows, scratch + soff);
-        hp[i].first_block = pb;
-        soff += row_scratch_bytes(p, rows, &a, &b, &c);
-        hd[i] = make_dot(p, hp[i], p.out_base, p.out_stride);
-        hd[i].first_block = di;
-        for (uint32_t r = 0; r < rows; ++r, ++pb)
-            if (bp.prep_map)
-                hpm[pb] = i;
-        const uint32_t items = dot_items(p.m->tiles, rows, bp.max_groups);
+        const bool mfma = place.gemm != kNoGemm;
+        unsigned char* const at = scratch + bp.places[place.prep].at;
+        PrepJob prep = make_prep(p, p.in_base, rows, at);
+        if (mfma) {
+            prep.q = reinterpret_cast<int8_t*>(at);
+            prep.planes = nullptr;
+            prep.sums = nullptr;
+            prep.rscale = reinterpret_cast<float*>(at + round_up((size_t)rows * p.m->k, 256));
+        }
+        if (place.prep == i) {
+            prep.first_block = pb;
+            for (uint32_t r = 0; r < rows; ++r, ++pb)
+                if (bp.prep_map)
+                    hpm[pb] = pj;
+            hp[pj++] = prep;
+        }
+        if (mfma) {
+            const GemmJob part = make_gemm(p, prep, p.out_base, p.out_stride);
+            if (gemms[place.gemm].wbits == nullptr)
+                gemms[place.gemm] = part;
+            else
+                add_part(&gemms[place.gemm], part);
+            continue;
+        }
+        hd[dj] = make_dot(p, prep, p.out_base, p.out_stride);
+        hd[dj].first_block = di;
+        const uint32_t items = dot_items(p.m->tiles, rows, bp.dot_groups);
         if (!bp.uniform)
             for (uint32_t r = 0; r < items; ++r)
-                hdm[di + r] = i;
+                hdm[di + r] = dj;
         di += items;
+        ++dj;
     }
 }
 
-// The two launches of a batch whose tables start at 'tables' on the device.
+// The launches of a batch whose tables start at 'tables' on the device: every job's rows,
+// the dots, then the matrix-core launches.
 hipError_t launch_batch(BNN_Device device, const unsigned char* tables, size_t prep_tab, size_t dot_tab,
                         size_t prep_map, uint32_t prep_blocks, uint32_t items, uint32_t uniform_items,
-                        uint32_t max_groups, bool scales, uint64_t seq, uint64_t* status) {
+                        uint32_t max_groups, uint32_t dot_groups, bool scales, const GemmJob* gemms,
+                        uint32_t gemm_count, uint64_t seq, uint64_t* status) {
     const PrepJob* dp = reinterpret_cast<const PrepJob*>(tables);
     const DotJob* dd = reinterpret_cast<const DotJob*>(tables + prep_tab);
     // no map (prep_map == 0) when every job has one row: prep block b is job b
@@ -1131,10 +1267,14 @@ hipError_t launch_batch(BNN_Device device, const unsigned char* tables, size_t p
     hipError_t e = timed(device, KK_PREP, [&] {
         return launch_prep_batch(device->stream, dp, dpm, prep_blocks, max_groups, seq, device->flag_dev, status);
     });
-    if (e == hipSuccess)
+    if (e == hipSuccess && items != 0)
         e = timed(device, KK_DOT, [&] {
-            return launch_dot_batch(device->stream, dd, ddm, items, uniform_items, max_groups, scales,
+            return launch_dot_batch(device->stream, dd, ddm, items, uniform_items, dot_groups, scales,
                                     device->cu_count, seq, device->flag_dev);
+        });
+    for (uint32_t g = 0; e == hipSuccess && g < gemm_count; ++g)
+        e = timed(device, KK_GEMM, [&] {
+            return launch_gemm(device->stream, gemms[g], device->cu_count, seq, device->flag_dev);
         });
     return e;
 }
@@ -1178,6 +1318,12 @@ EXPORT BNN_Status BNNX_ExecuteBatch(BNN_Device device, const BNN_Job* jobs, uint
     st = ensure_scratch(device, bp.scratch_bytes);
     if (st == BNN_OK)
         st = ensure_tables(device, bp.tables);
+    GemmJob* gemms = nullptr;
+    if (st == BNN_OK && bp.gemm_count != 0) {
+        gemms = static_cast<GemmJob*>(malloc(sizeof(GemmJob) * bp.gemm_count));
+        if (gemms == nullptr)
+            st = BNN_ENOMEM;
+    }
     if (st == BNN_OK && count > device->batch_cap) {
         BNN_Job* copy = static_cast<BNN_Job*>(realloc(device->batch_jobs, sizeof(BNN_Job) * count));
         if (copy == nullptr) {
@@ -1189,9 +1335,13 @@ EXPORT BNN_Status BNNX_ExecuteBatch(BNN_Device device, const BNN_Job* jobs, uint
     }
     if (st != BNN_OK) {
         device->batch_count = 0;
+        free(gemms);
         return st;
     }
-    fill_batch_tables(bp, jobs, device->scratch, device->table_host);
+    free(device->batch_gemms);
+    device->batch_gemms = gemms;
+    device->batch_gemm_count = bp.gemm_count;
+    fill_batch_tables(bp, jobs, device->scratch, device->table_host, gemms);
     if (hipMemcpyAsync(device->table_dev, device->table_host, bp.tables, hipMemcpyHostToDevice, device->stream) !=
         hipSuccess) {
         (void)hipGetLastError();
@@ -1203,8 +1353,10 @@ EXPORT BNN_Status BNNX_ExecuteBatch(BNN_Device device, const BNN_Job* jobs, uint
     device->batch_generation = device->generation;
     device->batch_prep_blocks = (uint32_t)bp.prep_blocks;
     device->batch_items = (uint32_t)bp.dot_items_total;
-    device->batch_uniform_items = bp.uniform ? dot_items(bp.plans[0].m->tiles, jobs[0].rows, bp.max_groups) : 0u;
+    device->batch_uniform_items = bp.uniform_items;
     device->batch_max_groups = bp.max_groups;
+    device->batch_dot_groups = bp.dot_groups;
+    device->batch_scales = bp.scales;
     device->batch_prep_tab = bp.prep_tab;
     device->batch_dot_tab = bp.dot_tab;
     device->batch_prep_map = bp.prep_map;
@@ -1219,7 +1371,8 @@ static BNN_Status run_cached_batch(BNN_Device device) {
     const hipError_t e = launch_batch(device, device->table_dev, device->batch_prep_tab, device->batch_dot_tab,
                                       device->batch_prep_map, device->batch_prep_blocks, device->batch_items,
                                       device->batch_uniform_items, device->batch_max_groups,
-                                      device->batch_needs_nearest, seq, device->status_host);
+                                      device->batch_dot_groups, device->batch_scales, device->batch_gemms,
+                                      device->batch_gemm_count, seq, device->status_host);
     if (e != hipSuccess)
         device->batch_count = 0;
     return finish(device, e, seq);
@@ -1243,9 +1396,11 @@ EXPORT BNN_Status BNNX_BatchCreate(BNN_Device device, const BNN_Job* jobs, uint3
         return BNN_EIO;
     BNNX_Batch b = static_cast<BNNX_Batch>(calloc(1, sizeof(bnnx_batch)));
     unsigned char* host = static_cast<unsigned char*>(malloc(bp.tables));
-    if (b == nullptr || host == nullptr) {
+    GemmJob* gemms = bp.gemm_count ? static_cast<GemmJob*>(malloc(sizeof(GemmJob) * bp.gemm_count)) : nullptr;
+    if (b == nullptr || host == nullptr || (bp.gemm_count && gemms == nullptr)) {
         free(b);
         free(host);
+        free(gemms);
         return BNN_ENOMEM;
     }
     const size_t scratch_at = round_up(bp.tables, 256);
@@ -1254,23 +1409,29 @@ EXPORT BNN_Status BNNX_BatchCreate(BNN_Device device, const BNN_Job* jobs, uint3
         (void)hipGetLastError();
         free(b);
         free(host);
+        free(gemms);
         return BNN_ENOMEM;
     }
     b->mem = static_cast<unsigned char*>(mem);
-    fill_batch_tables(bp, jobs, b->mem + scratch_at, host);
+    fill_batch_tables(bp, jobs, b->mem + scratch_at, host, gemms);
     hipError_t e = hipMemcpy(b->mem, host, bp.tables, hipMemcpyHostToDevice);
     free(host);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         (void)hipFree(b->mem);
         free(b);
+        free(gemms);
         return BNN_EIO;
     }
     b->device = device;
     b->retired = device->retired;
+    b->gemms = gemms;
+    b->gemm_count = bp.gemm_count;
+    b->scales = bp.scales;
+    b->dot_groups = bp.dot_groups;
     b->prep_blocks = (uint32_t)bp.prep_blocks;
     b->items = (uint32_t)bp.dot_items_total;
-    b->uniform_items = bp.uniform ? dot_items(bp.plans[0].m->tiles, jobs[0].rows, bp.max_groups) : 0u;
+    b->uniform_items = bp.uniform_items;
     b->max_groups = bp.max_groups;
     b->prep_tab = bp.prep_tab;
     b->dot_tab = bp.dot_tab;
@@ -1572,8 +1733,7 @@ EXPORT BNN_Status BNNX_LaunchRows(BNN_Device device, const BNN_Job* jobs, uint32
     for (uint32_t i = 0; e == hipSuccess && i < count; i += kGemmParts) {
         GemmJob gj = make_gemm(plans[i], pj, plans[i].out_base, plans[i].out_stride);
         for (uint32_t p = i + 1u; p < count && p < i + kGemmParts; ++p)
-            gj.parts[gj.extra++] = GemmPart{plans[p].m->wbits,   plans[p].m->wscale, plans[p].out_base,
-                                            plans[p].out_stride, plans[p].m->n,      plans[p].m->tiles, 0, 0};
+            add_part(&gj, make_gemm(plans[p], pj, plans[p].out_base, plans[p].out_stride));
         e = timed(device, KK_GEMM,
                   [&] { return launch_gemm(device->stream, gj, device->cu_count, seq, device->flag_dev); });
     }
@@ -1615,7 +1775,8 @@ EXPORT BNN_Status BNNX_BatchLaunch(BNNX_Batch batch) {
                              })
                      : launch_batch(device, batch->mem, batch->prep_tab, batch->dot_tab, batch->prep_map,
                                     batch->prep_blocks, batch->items, batch->uniform_items, batch->max_groups,
-                                    batch->needs_nearest, seq, device->status_host + 1);
+                                    batch->dot_groups, batch->scales, batch->gemms, batch->gemm_count, seq,
+                                    device->status_host + 1);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return BNN_EIO;
@@ -1630,6 +1791,7 @@ EXPORT void BNNX_BatchDestroy(BNNX_Batch batch) {
     (void)hipStreamSynchronize(batch->device->stream);
     (void)hipFree(batch->mem);
     batch->device->live_batches--;
+    free(batch->gemms);
     free(batch);
 }
 

@@ -96,6 +96,8 @@ __device__ __forceinline__ uint32_t select_part(GemmJob& j, uint32_t nt) {
                 const GemmPart& p = j.parts[i];
                 j.wbits = p.wbits;
                 j.wscale = p.wscale;
+                j.q = p.q;
+                j.rscale = p.rscale;
                 j.out = p.out;
                 j.out_stride = p.out_stride;
                 j.n = p.n;

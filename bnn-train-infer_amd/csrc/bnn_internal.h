@@ -87,19 +87,22 @@ struct DotJob {
 };
 
 // One multi-row job on the matrix cores (rows >= kMfmaMinRows), read from the
-// matrix's resident layout (sign bits unpacked in LDS by the kernel).  Up to kGemmParts
-// matrices of one k may share the rows (the q, k and v projections of a block of tokens): the
-// job's own fields describe the first, parts[] the others, whose column tiles follow the
-// first's; column tile t of the launch belongs to the last part with first <= t (first is set
-// by the launcher, in column tiles of the kernel it picks).
+// matrix's resident layout (sign bits unpacked in LDS by the kernel).  Up to kGemmParts jobs
+// of one k, one number of rows and one mode (the q, k and v projections of a block of tokens,
+// jobs of a batch) may share a launch: the job's own fields describe the first, parts[] the
+// others, whose column tiles follow the first's; column tile t of the launch belongs to the
+// last part with first <= t (first is set by the launcher, in column tiles of the kernel it
+// picks).
 struct GemmPart {
     const uint4* wbits;
     const uint16_t* wscale;
+    const int8_t* q;
+    const float* rscale;
     unsigned char* out;
     uint64_t out_stride;
     uint32_t n, tiles, first, pad_;
 };
-constexpr uint32_t kGemmParts = 4;
+constexpr uint32_t kGemmParts = 8;
 struct GemmJob {
     const uint4* wbits;       // matrix layout [tiles][groups][64] x 16 bytes
     const uint16_t* wscale;   // matrix layout [tiles][groups][64]
@@ -316,9 +319,12 @@ struct bnn_accel_device {
     BNN_Job* batch_jobs;
     uint32_t batch_count, batch_cap;
     uint64_t batch_generation;
-    uint32_t batch_prep_blocks, batch_items, batch_uniform_items, batch_max_groups;
+    uint32_t batch_prep_blocks, batch_items, batch_uniform_items, batch_max_groups, batch_dot_groups;
     size_t batch_prep_tab, batch_dot_tab, batch_prep_map, batch_tables;
     bool batch_needs_nearest;  // some job of the cached batch is an FP32 operation
+    bool batch_scales;         // some job of its dot launch sums scaled products
+    bnnhip::GemmJob* batch_gemms;  // its matrix-core launches
+    uint32_t batch_gemm_count;
     // optional kernel timing (extension API): event pairs recorded around
     // launches, resolved after the call's synchronisation
     int timing;
@@ -339,14 +345,17 @@ struct bnn_accel_matrix {
 };
 
 // A prepared batch: job tables and the rows' scratch in one device allocation,
-// built once; every launch is two kernel launches and nothing else.
+// built once; every launch is the rows' kernel, the dots' kernel for the jobs it takes and
+// one per group of matrix-core jobs, and nothing else.
 struct bnnx_batch {
     BNN_Device device;
     uint64_t retired;  // device->retired when built: valid while no matrix or buffer was destroyed since
     unsigned char* mem;
-    uint32_t prep_blocks, items, uniform_items, max_groups;
+    uint32_t prep_blocks, items, uniform_items, max_groups, dot_groups;
     size_t prep_tab, dot_tab, prep_map;
-    bool needs_nearest;
+    bool needs_nearest, scales;
+    bnnhip::GemmJob* gemms;  // the launches of its matrix-core jobs
+    uint32_t gemm_count;
     // fused batch (BNNX_BatchCreateFused): one launch of `fused_tiles` workgroups
     bool fused;
     uint32_t fused_tiles, fused_grid;

@@ -161,3 +161,49 @@ def test_prompt_block_error_then_prompt(pkg, hip, tmp_path):
         assert [first] + c.decode_greedy(first, len(want) - 1) == want
         c.free()
         m.free()
+
+
+# Batches whose multi-row jobs run on the matrix cores: groups of up to eight alike jobs (one k,
+# rows and operation), shared and own input views, beside jobs that stay with the dots.
+@pytest.mark.parametrize("specs,shared", [
+    ([("GEMM_F32", 2048, 2048, 48), ("GEMM_F32", 2048, 1024, 48), ("GEMM_F32", 2048, 1030, 48)], True),
+    ([("GEMM_F32", 2048, 2048, 64)] * 9, False),                        # a second group of one
+    ([("GEMM_F32", 256, 70, 4)], False),                                # a small group alone
+    ([("GEMM_F32", 256, 70, 4), ("GEMM", 256, 70, 4)], False),          # two small groups: the dots
+    ([("GEMM_F32", 4096, 3000, 17), ("GEMV_F32", 512, 100, 1), ("GEMM", 4096, 200, 17),
+      ("DOT_GROUPS", 4096, 1000, 33), ("GEMM_F32", 128, 5, 3), ("GEMM_F32", 4096, 65, 17)], False),
+], ids=["shared", "nine", "small", "small-two", "mixed"])
+def test_batch_jobs_on_the_matrix_cores(pkg, hipdev, oracle_fast, specs, shared):
+    from test_hip_batch import _free, _mk_batch, _oracle, _outputs
+    mats, xs, bi, bo, jobs, out_off, layouts = _mk_batch(pkg, hipdev, specs, seed=11)
+    if shared:  # one view for all
+        for i in range(len(specs)):
+            jobs[i].input, xs[i] = jobs[0].input, xs[0]
+    wants = _oracle(pkg, oracle_fast, specs, mats, xs)
+    print(f"batch of {len(specs)} jobs", flush=True)
+
+    def check():
+        for i, (got, want) in enumerate(zip(_outputs(bo, out_off, layouts), wants)):
+            assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (i, specs[i], first_mismatch(got, want))
+        bo.write(np.zeros(bo.nbytes, np.uint8))
+
+    api = hipdev.api
+    for _ in range(2):  # planned, then from the cached tables
+        assert api.BNNX_ExecuteBatch(hipdev.handle, jobs, len(specs)) == pkg.Status.OK
+        check()
+    batch = ctypes.c_void_p()
+    assert api.BNNX_BatchCreate(hipdev.handle, jobs, len(specs), ctypes.byref(batch)) == pkg.Status.OK
+    for _ in range(2):
+        assert api.BNNX_BatchLaunch(batch) == pkg.Status.OK
+        assert api.BNNX_DeviceSynchronize(hipdev.handle) == pkg.Status.OK
+        check()
+    # an illegal value in the last job's last row: no job writes anything
+    t, at = pkg.Type.F32, jobs[len(specs) - 1].input.offset
+    row_bytes = specs[-1][1] * 4
+    if jobs[len(specs) - 1].input.type == int(t):
+        bi.write(np.full(1, np.nan, np.float32), at + (specs[-1][3] - 1) * row_bytes)
+        assert api.BNNX_BatchLaunch(batch) == pkg.Status.OK
+        assert api.BNNX_DeviceSynchronize(hipdev.handle) == pkg.Status.ERANGE
+        assert not bo.read().any()
+    api.BNNX_BatchDestroy(batch)
+    _free(mats, bi, bo)
