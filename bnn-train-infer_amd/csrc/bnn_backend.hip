@@ -1055,12 +1055,13 @@ struct BatchPlan {
 };
 
 // Which jobs run on the matrix cores: groups of up to kGemmParts jobs of one k, one number of
-// rows (>= kBatchMfmaRows) and one mode, each group one launch of ~4 us and more, against
+// rows and one mode, each group one launch of ~4 us and more, against
 // ~4 us for the one dot launch of every other job plus ~36 us per 10^9 weights times rows in
 // it (q/k/v of 8 / 64 / 256 rows 9.0 / 19.4 / 52 us a pass with dots, 7.9 / 8.4 / 15 us on
 // the matrix cores; 6144->6144 x 64 rows 60 against 22 us).  A group is worth its launch from
-// 0.11 * 10^9 on, or when it leaves the dot launch without work.
-constexpr uint32_t kBatchMfmaRows = 4;
+// 0.11 * 10^9 on, or when it leaves the dot launch without work.  Fewest rows: 8, or 4 for
+// K > 2048, where the dots run in longer chains (6144->2048 x 4 rows 15.1 against 11.8 us; at
+// K = 2048 both take the same time, and the dots share the chip better with other streams).
 constexpr double kGemmGroupWork = 0.11e9;
 
 constexpr uint32_t kGemmLookAhead = 64;  // jobs behind its first that a group is filled from
@@ -1076,11 +1077,11 @@ BNN_Status place_jobs(const BNN_Job* jobs, BatchPlan* bp) {
     for (uint32_t i = 0; i < count; ++i) {
         if (bp->places[i].gemm != kNoGemm)
             continue;
-        if (jobs[i].rows < kBatchMfmaRows) {
+        const JobPlan& p = bp->plans[i];
+        if (jobs[i].rows < (p.m->k > 2048u ? 4u : 8u)) {
             ++dots;
             continue;
         }
-        const JobPlan& p = bp->plans[i];
         work[groups] = 0.0;
         for (uint32_t j = i, members = 0; j < count && j - i < kGemmLookAhead && members < kGemmParts; ++j) {
             const JobPlan& o = bp->plans[j];

@@ -452,15 +452,13 @@ __device__ void set_error_first(int* err, int code) {
 //   the kv head's first query head, in the block that holds pos), then one score per
 //   lane, each an in-order dot over head_dim -- position pos from the wave's own new
 //   key, so no workgroup reads a row another is writing;
-//   k_attn_pv, workgroup (query head h, slice of 32 head dims), two waves: the maximum,
+//   k_attn_pv, workgroup (query head h, slice of 32 head dims), sixteen waves: the maximum,
 //   expf, the in-order sum and the probabilities over positions 0..pos, then
-//   value[i] = sum over t in order of p[t] * V[t][i] for the slice's i, the V rows
-//   moved into LDS by DMA by a second wave meanwhile.
+//   value[i] = sum over t in order of p[t] * V[t][i] for the slice's i.
 // Every sum runs in index / position order, as in the host step.
 constexpr uint32_t kAttnHD = 128;             // head_dim of the fused step
 constexpr uint32_t kScoreBlock = 64;          // positions per k_attn_scores workgroup
 constexpr uint32_t kPvSlice = 32;             // head dims per k_attn_pv workgroup
-constexpr uint32_t kPvLdsPositions = 4096;    // probabilities in LDS (16 KB); beyond, recomputed
 
 // Orders one wave's LDS writes before its later LDS reads of other lanes' data.
 __device__ __forceinline__ void wave_lds_sync() {
@@ -863,145 +861,267 @@ __global__ __launch_bounds__(256) void k_attn_one(
     }
 }
 
-constexpr uint32_t kPvRows = 1024;  // V slice rows in LDS per pass (128 KB)
-constexpr uint32_t kPvPad = 16;     // rows / probabilities read past the end by the pipelined loop
+// The softmax and the weighted values of one slice of 32 head dims of one head, positions
+// 0..pos, by sixteen waves:
+//   all waves: the maximum; expf(score - max) into LDS, 4096 positions (a span) at a time; their
+//   in-order sum -- segments of 128 terms, each run from 64 candidate starts at once (one per
+//   lane: the binary32 values around the binary64 prefix sum), then wave 0 walks the segments in
+//   order and takes the lane that started from exactly the running sum (or adds the segment
+//   term by term where none did), so the result is the sequential loop's whatever the data;
+//   then tiles of 128 positions: two waves the probabilities e / sum of the tile after next,
+//   eight waves the products p[t] * V[t][i] of the next tile into LDS, transposed, and wave 0
+//   value[i] = sum over t in order (lane i), four products per 16-byte read.
+// Bound by wave 0's chain: a wave alone on its SIMD issues an instruction every ~6.5 cycles, so
+// a position costs ~8 cycles (an add and a quarter of a read) -- the waves that feed it stay off
+// its SIMD.  Against one wave doing the softmax, the products and the sums of a slice with a
+// second one loading V rows: 300 positions 8.4 -> 8.4 us, 3000 positions 65 -> 23 us per layer.
+constexpr uint32_t kPvWaves = 16, kPvTile = 128, kPvSpan = 4096, kPvSegment = 128;
+constexpr uint32_t kPvHeld = 4 * kPvSpan;  // exponentials kept in LDS (64 KB); longer rows recompute theirs per tile
+constexpr uint32_t kPvSegments = kPvSpan / kPvSegment, kPvPitch4 = kPvTile / 4 + 1;
 
-__global__ __launch_bounds__(128) void k_attn_pv(const float* __restrict__ scores, const float* __restrict__ vc,
-                                                 uint32_t kv_mul, uint32_t pos, uint32_t kv_dim, uint32_t n_ctx,
-                                                 float* __restrict__ y, int* err, int code_base) {
+extern "C" __device__ double __ockl_wfred_add_f64(double);
+
+__global__ __launch_bounds__(64 * kPvWaves) void k_attn_pv(const float* __restrict__ scores,
+                                                           const float* __restrict__ vc, uint32_t kv_mul, uint32_t pos,
+                                                           uint32_t kv_dim, uint32_t n_ctx, float* __restrict__ y,
+                                                           int* err, int code_base) {
     constexpr uint32_t HD = kAttnHD;
-    constexpr uint32_t kBatch = 8;  // score loads per lane in flight
-    __shared__ float4 vs4[(kPvRows + kPvPad) * kPvSlice / 4];
-    __shared__ float4 p4[(kPvLdsPositions + 64u) / 4];  // probabilities (or one pass's), padded
-    __shared__ uint64_t exp_tab[32];                      // the expf table: its lookups are per-lane gathers
-    float* p = reinterpret_cast<float*>(p4);
-    const float* vs = reinterpret_cast<const float*>(vs4);
-    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t h = blockIdx.x, d0 = blockIdx.y * kPvSlice;
-    const size_t off = (size_t)(h / kv_mul) * HD + d0;
+    __shared__ float4 e4[kPvHeld / 4];                      // the exponentials, or one span's past kPvHeld
+    __shared__ float4 prod4[2][kPvSlice * kPvPitch4];       // a tile's products, [dim][position]
+    __shared__ float p_tile[2][kPvTile];
+    __shared__ double seg_sum[kPvSegments];
+    __shared__ float seg_end[kPvSegments * 64];
+    __shared__ int seg_base[kPvSegments];
+    __shared__ float red[kPvWaves];
+    __shared__ float sum_s;
+    __shared__ uint64_t exp_tab[32];                        // its lookups are per-lane gathers
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t h = blockIdx.x, d0 = blockIdx.y * kPvSlice, n = pos + 1u;
+    const bool held = n <= kPvHeld;
     const float* sc = scores + (size_t)h * n_ctx;
-    const bool in_lds = pos < kPvLdsPositions;  // every probability in LDS, else per pass of V rows
 
-    if (wave == 1) {
-        // the V rows of each pass into LDS, 8 rows of 128 bytes per instruction (lane l:
-        // piece l % 8 of row l / 8; rows past pos clamped), between the barriers that
-        // hand the rows to wave 0 and take them back
-        const uint32_t base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)vs4;
-        for (uint32_t t0 = 0; t0 <= pos; t0 += kPvRows) {
-            if (t0 > 0)
-                __builtin_amdgcn_s_barrier();  // wave 0 is done with the previous rows
-            const uint32_t rows = min(pos + 1u - t0, kPvRows);
-            for (uint32_t r0 = 0; r0 < rows; r0 += 8u) {
-                const uint32_t t = min(t0 + r0 + (lane >> 3), pos);
-                dma16(vc + (size_t)t * kv_dim + off + 4u * (lane & 7u), base + r0 * kPvSlice * 4u);
-            }
-            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-            __builtin_amdgcn_s_barrier();         // the rows are in LDS
-        }
-        return;
-    }
+    // producers: waves 1, 2, 3, 5, 6, 7, 9, 10 (not on wave 0's SIMD), 16-byte piece g of each
+    // half tile: position g / 8, dims 4 (g % 8) ..
+    const uint32_t pw = wave - 1u - wave / 4u;              // 0..7 for the producers
+    const bool producer = wave % 4u != 0u && pw < 8u;
+    const uint32_t piece = pw * 64u + lane;
+    const float* v = vc + (size_t)(h / kv_mul) * HD + d0 + 4u * (piece & 7u);
+    float4 vv[2];
+    const auto load_v = [&](uint32_t tile) {
+#pragma unroll
+        for (uint32_t f = 0; f < 2u; ++f)
+            vv[f] = *reinterpret_cast<const float4*>(
+                v + (size_t)min(tile * kPvTile + 64u * f + (piece >> 3), pos) * kv_dim);
+    };
 
-    // wave 0: the scores into LDS when they fit, and their maximum (order-free: finite
-    // or flagged)
-    if (lane < 32u)
-        exp_tab[lane] = kExp2Table[lane];
+    if (tid < 32u)
+        exp_tab[tid] = kExp2Table[tid];
     float mx = -INFINITY;
-    for (uint32_t t0 = 0; t0 <= pos; t0 += 64u * kBatch) {
-        float x[kBatch];
+    for (uint32_t t0 = 0; t0 < n; t0 += kPvSpan) {
+        float x[4];
 #pragma unroll
-        for (uint32_t c = 0; c < kBatch; ++c)
-            x[c] = sc[min(t0 + 64u * c + lane, pos)];
+        for (uint32_t c = 0; c < 4u; ++c)
+            x[c] = sc[min(t0 + 1024u * c + tid, pos)];
 #pragma unroll
-        for (uint32_t c = 0; c < kBatch; ++c) {
-            const uint32_t t = t0 + 64u * c + lane;
-            if (t <= pos) {
-                if (in_lds)
-                    p[t] = x[c];
-                mx = x[c] > mx ? x[c] : mx;
+        for (uint32_t c = 0; c < 4u; ++c)
+            mx = x[c] > mx ? x[c] : mx;
+    }
+    mx = __ockl_wfred_max_f32(mx);  // order-free: finite or flagged
+    if (lane == 0)
+        red[wave] = mx;
+    if (tid == 0)
+        sum_s = 0.0f;
+    block_lds_barrier();
+    float maximum = red[0];
+#pragma unroll
+    for (uint32_t w = 1; w < kPvWaves; ++w)
+        maximum = red[w] > maximum ? red[w] : maximum;
+
+    for (uint32_t t0 = 0; t0 < n; t0 += kPvSpan) {
+        const uint32_t m = min(kPvSpan, n - t0), segs = (m + kPvSegment - 1u) / kPvSegment;
+        float4* const span4 = e4 + (held ? t0 / 4u : 0u);
+        float* const e = reinterpret_cast<float*>(span4);
+        // +0 pads the last segment (adding +0 to this sum of non-negative terms changes nothing)
+#pragma unroll
+        for (uint32_t c = 0; c < 4u; ++c) {
+            const uint32_t i = 1024u * c + tid;
+            if (i < segs * kPvSegment)
+                e[i] = i < m ? bnne_expf_libc(sc[t0 + i] - maximum, exp_tab) : 0.0f;
+        }
+        block_lds_barrier();
+        // wave w: segments w and w + 16
+        const bool two = wave + kPvWaves < segs;
+        if (wave < segs) {
+            const double a = __ockl_wfred_add_f64((double)e[wave * kPvSegment + lane] +
+                                                  (double)e[wave * kPvSegment + 64u + lane]);
+            if (lane == 0)
+                seg_sum[wave] = a;
+        }
+        if (two) {
+            const uint32_t at = (wave + kPvWaves) * kPvSegment + lane;
+            const double a = __ockl_wfred_add_f64((double)e[at] + (double)e[at + 64u]);
+            if (lane == 0)
+                seg_sum[wave + kPvWaves] = a;
+        }
+        block_lds_barrier();
+        if (wave < segs) {
+            float c[2];
+            int base[2];
+#pragma unroll
+            for (uint32_t r = 0; r < 2u; ++r) {
+                const uint32_t j = wave + kPvWaves * r;
+                const double before = __ockl_wfred_add_f64(lane < min(j, segs) ? seg_sum[lane] : 0.0);
+                base[r] = __float_as_int((float)((double)sum_s + before)) - 32;
+                c[r] = __int_as_float(base[r] + (int)lane);
+            }
+            const float4* s0 = span4 + wave * (kPvSegment / 4u);
+            const float4* s1 = span4 + (two ? wave + kPvWaves : wave) * (kPvSegment / 4u);
+#pragma unroll 2
+            for (uint32_t i = 0; i < kPvSegment / 4u; i += 4u) {
+                float4 a[4], b[4];
+#pragma unroll
+                for (uint32_t q = 0; q < 4u; ++q)
+                    a[q] = s0[i + q], b[q] = s1[i + q];
+#pragma unroll
+                for (uint32_t q = 0; q < 4u; ++q) {
+                    c[0] = c[0] + a[q].x;
+                    c[1] = c[1] + b[q].x;
+                    c[0] = c[0] + a[q].y;
+                    c[1] = c[1] + b[q].y;
+                    c[0] = c[0] + a[q].z;
+                    c[1] = c[1] + b[q].z;
+                    c[0] = c[0] + a[q].w;
+                    c[1] = c[1] + b[q].w;
+                }
+            }
+            seg_end[wave * 64u + lane] = c[0];
+            if (lane == 0)
+                seg_base[wave] = base[0];
+            if (two) {
+                seg_end[(wave + kPvWaves) * 64u + lane] = c[1];
+                if (lane == 0)
+                    seg_base[wave + kPvWaves] = base[1];
             }
         }
-    }
-    const float maximum = __ockl_wfred_max_f32(mx);
-    wave_lds_sync();
-
-    // expf(score - max) and their sum in position order; +0 pads the terms to a
-    // multiple of 64 (adding +0 to this sum of non-negative terms changes nothing)
-    float sum = 0.0f;
-    if (in_lds) {
-        const uint32_t padded = (pos + 64u) & ~63u;
-        for (uint32_t t = lane; t < padded; t += 64u)
-            p[t] = t <= pos ? bnne_expf_libc(p[t] - maximum, exp_tab) : 0.0f;
-        wave_lds_sync();
-        sum = sum_lds_in_order(p, padded);
-    } else {
-        for (uint32_t t0 = 0; t0 <= pos; t0 += 64u) {
-            p[lane] = t0 + lane <= pos ? bnne_expf_libc(sc[t0 + lane] - maximum, exp_tab) : 0.0f;
-            wave_lds_sync();
-            sum = sum_lds_in_order(p, 64u, sum);
-            wave_lds_sync();
+        block_lds_barrier();
+        if (wave == 0) {
+            // the running sum's bits, uniform across the wave; lane j holds segment j's first
+            // candidate, ends[j] its candidates' end values
+            const int bases = seg_base[min(lane, segs - 1u)];
+            float ends[kPvSegments];
+#pragma unroll
+            for (uint32_t j = 0; j < kPvSegments; ++j)
+                ends[j] = seg_end[min(j, segs - 1u) * 64u + lane];
+            uint32_t run = __builtin_amdgcn_readfirstlane(__float_as_int(sum_s));
+#pragma unroll
+            for (uint32_t j = 0; j < kPvSegments; ++j) {
+                if (j < segs) {
+                    const uint32_t idx = run - (uint32_t)__builtin_amdgcn_readlane(bases, (int)j);
+                    if (idx < 64u)
+                        run = (uint32_t)__builtin_amdgcn_readlane(__float_as_int(ends[j]), (int)idx);
+                    else
+                        run = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(
+                            sum_lds_in_order(e + j * kPvSegment, kPvSegment, __uint_as_float(run))));
+                }
+            }
+            if (lane == 0)
+                sum_s = __uint_as_float(run);
         }
+        block_lds_barrier();
     }
-    // a failed softmax is flagged; the wave still runs its barriers (y is then unused)
+    const float sum = sum_s;
+    // a failed softmax is flagged; the waves still run their barriers (y is then unused)
     if (!(sum > 0.0f) || !isfinite(sum)) {
-        if (lane == 0)
+        if (tid == 0)
             set_error_first(err, code_base + 4 + 2 * (int)h);
     }
-    if (in_lds) {
-        for (uint32_t t = lane; t <= pos; t += 64u)
-            p[t] = p[t] / sum;
-    }
 
-    // value[i] = sum over t in order of p[t] * V[t][i] (lane i < 32 of the slice) per
-    // pass of V rows; the next 8 rows' reads are issued before the current 8 are added
-    float acc = 0.0f;
-    for (uint32_t t0 = 0; t0 <= pos; t0 += kPvRows) {
-        const uint32_t n = min(kPvRows, pos + 1u - t0);
-        if (t0 > 0)
-            __builtin_amdgcn_s_barrier();  // the previous rows are read: wave 1 may reload
-        if (!in_lds) {                     // this pass's probabilities
-            for (uint32_t r = lane; r < n; r += 64u)
-                p[r] = bnne_expf_libc(sc[t0 + r] - maximum, exp_tab) / sum;
+    // tiles of 128 positions.  Step k: wave 0 adds tile k's products, the producers form tile
+    // k + 1's (their V values requested a step ago) and request tile k + 2's, and waves 11 and
+    // 13 form tile k + 2's probabilities.
+    const uint32_t tiles = (n + kPvTile - 1u) / kPvTile;
+    const float* const e = reinterpret_cast<const float*>(e4);
+    const uint32_t pt = wave == 11u ? lane : 64u + lane;
+    const auto probabilities = [&](uint32_t tile) {
+        const uint32_t t = tile * kPvTile + pt;
+        if ((wave == 11u || wave == 13u) && t < n) {
+            const float x = held ? e[t] : bnne_expf_libc(sc[t] - maximum, exp_tab);
+            p_tile[tile & 1u][pt] = x / sum;
         }
-        wave_lds_sync();
-        __builtin_amdgcn_s_barrier();  // the rows are in LDS
-        if (lane < kPvSlice) {
-            const float4* pp = reinterpret_cast<const float4*>(in_lds ? p + t0 : p);
-            const float* vl = vs + lane;
-            float4 pa0 = pp[0], pa1 = pp[1];
-            float va[8];
+    };
+    const auto products = [&](uint32_t tile) {  // positions past pos: never added
+        float* out = reinterpret_cast<float*>(prod4[tile & 1u]) + 4u * (piece & 7u) * (4u * kPvPitch4);
 #pragma unroll
-            for (uint32_t c = 0; c < 8; ++c)
-                va[c] = vl[c * kPvSlice];
-            uint32_t r = 0;
-#pragma unroll 2
-            for (; r + 8u <= n; r += 8u) {
-                const float4 pb0 = pp[(r + 8u) / 4u], pb1 = pp[(r + 8u) / 4u + 1u];
-                float vb[8];
-#pragma unroll
-                for (uint32_t c = 0; c < 8; ++c)
-                    vb[c] = vl[(r + 8u + c) * kPvSlice];
-                acc = acc + pa0.x * va[0];
-                acc = acc + pa0.y * va[1];
-                acc = acc + pa0.z * va[2];
-                acc = acc + pa0.w * va[3];
-                acc = acc + pa1.x * va[4];
-                acc = acc + pa1.y * va[5];
-                acc = acc + pa1.z * va[6];
-                acc = acc + pa1.w * va[7];
-                pa0 = pb0;
-                pa1 = pb1;
-#pragma unroll
-                for (uint32_t c = 0; c < 8; ++c)
-                    va[c] = vb[c];
-            }
-            const float pr[8] = {pa0.x, pa0.y, pa0.z, pa0.w, pa1.x, pa1.y, pa1.z, pa1.w};
-#pragma unroll
-            for (uint32_t c = 0; c < 7; ++c)
-                if (r + c < n)
-                    acc = acc + pr[c] * va[c];
+        for (uint32_t f = 0; f < 2u; ++f) {
+            const uint32_t t = 64u * f + (piece >> 3);
+            const float p = p_tile[tile & 1u][t];
+            out[t] = p * vv[f].x;
+            out[4u * kPvPitch4 + t] = p * vv[f].y;
+            out[8u * kPvPitch4 + t] = p * vv[f].z;
+            out[12u * kPvPitch4 + t] = p * vv[f].w;
         }
+    };
+    if (producer)
+        load_v(0);
+    probabilities(0);
+    block_lds_barrier();
+    if (producer) {
+        products(0);
+        load_v(1);
     }
-    if (lane < kPvSlice)
+    probabilities(1);
+    block_lds_barrier();
+    float acc = 0.0f;
+    for (uint32_t k = 0; k < tiles; ++k) {
+        if (wave == 0) {
+            const uint32_t count = min(kPvTile, n - k * kPvTile);
+            const f32x4* row = reinterpret_cast<const f32x4*>(prod4[k & 1u]) + (lane & (kPvSlice - 1u)) * kPvPitch4;
+            if (count == kPvTile) {
+                // stages of 8 reads, the next stage's in flight during the additions
+                f32x4 r[2][8];
+#pragma unroll
+                for (uint32_t c = 0; c < 8u; ++c)
+                    r[0][c] = row[c];
+#pragma unroll
+                for (uint32_t i = 0; i < kPvTile / 4u; i += 8u) {
+                    const uint32_t cur = (i / 8u) & 1u;
+                    if (i + 8u < kPvTile / 4u) {
+#pragma unroll
+                        for (uint32_t c = 0; c < 8u; ++c)
+                            r[cur ^ 1u][c] = row[i + 8u + c];
+                    }
+                    lds_stage_ready(r[cur]);
+#pragma unroll
+                    for (uint32_t c = 0; c < 8u; ++c) {
+                        acc = acc + r[cur][c].x;
+                        acc = acc + r[cur][c].y;
+                        acc = acc + r[cur][c].z;
+                        acc = acc + r[cur][c].w;
+                    }
+                }
+            } else {
+                const float* f = reinterpret_cast<const float*>(row);
+                uint32_t t = 0;
+                for (; t + 4u <= count; t += 4u) {
+                    const f32x4 x = row[t / 4u];
+                    acc = acc + x.x;
+                    acc = acc + x.y;
+                    acc = acc + x.z;
+                    acc = acc + x.w;
+                }
+                for (; t < count; ++t)
+                    acc = acc + f[t];
+            }
+        } else if (k + 1u < tiles) {
+            if (producer) {
+                products(k + 1u);
+                load_v(k + 2u);
+            }
+            probabilities(k + 2u);
+        }
+        block_lds_barrier();
+    }
+    if (wave == 0 && lane < kPvSlice)
         y[(size_t)h * HD + d0 + lane] = acc;
 }
 
@@ -1488,7 +1608,7 @@ BNNE_Status enqueue_token(Resident* r, uint32_t pos, uint32_t token, const unsig
                                k_norm + (size_t)l * HD, r->rope_cos + (size_t)pos * half,
                                r->rope_sin + (size_t)pos * half, r->kc + cache_layer, r->vc + cache_layer, pos,
                                r->kv_dim, scale, r->scores, r->n_ctx, r->err, (int)l * code_span(r));
-            hipLaunchKernelGGL(k_attn_pv, dim3(r->H, HD / kPvSlice), dim3(128), 0, r->stream, r->scores,
+            hipLaunchKernelGGL(k_attn_pv, dim3(r->H, HD / kPvSlice), dim3(64 * kPvWaves), 0, r->stream, r->scores,
                                r->vc + cache_layer, r->H / r->Hk, pos, r->kv_dim, r->n_ctx, r->y, r->err,
                                (int)l * code_span(r));
         }

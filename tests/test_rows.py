@@ -111,7 +111,7 @@ def test_launch_rows_illegal_row(pkg, hipdev, kind):
         f.free()
 
 
-TINY = {"layers": 2, "hidden": 256, "heads": 2, "kv_heads": 1, "ffn": 512, "vocab": 512, "context": 2816}
+TINY = {"layers": 2, "hidden": 256, "heads": 2, "kv_heads": 1, "ffn": 512, "vocab": 512, "context": 4352}
 
 
 @pytest.mark.parametrize("count,split", [
@@ -119,6 +119,7 @@ TINY = {"layers": 2, "hidden": 256, "heads": 2, "kv_heads": 1, "ffn": 512, "voca
     (1025, 0),      # a second block of one token
     (1300, 40),     # two blocks behind a started cache
     (2500, 1400),   # softmax rows of more than one LDS chunk
+    (4200, 4150),   # single tokens whose in-order softmax sum spans two rounds of segments
 ])
 def test_prompt_blocks_match_single_tokens(pkg, hip, tmp_path, count, split):
     path = tmp_path / "m.gguf"
