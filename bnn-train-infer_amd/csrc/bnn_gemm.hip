@@ -16,7 +16,7 @@
 //     increasing order, one rounding per add.  A zero product comes out as +0
 //     where the reference may form -0; the accumulator starts at +0 and never
 //     becomes -0 (x + -x == +0 in round-to-nearest), so the sums agree bit for bit.
-// DOT_GROUPS restarts the accumulator at 0 and stores D itself as int16.
+// DOT_GROUPS stores D itself as int16 (k_gemm_dots).
 //
 // k_gemm_bits<TM, TN, WGM, WGN>: workgroup tile TM x TN, WGM x WGN waves of
 // (TM/WGM) x (TN/WGN).  Everything a group needs reaches LDS by DMA
@@ -198,7 +198,7 @@ struct Tiling {
     static_assert(TM * TN / 4 % THREADS == 0, "output chunks per thread");
 };
 
-template <int TM, int TN, int WGM, int WGN, bool DOT>
+template <int TM, int TN, int WGM, int WGN>
 __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_t mtiles, uint32_t ntiles, uint32_t band,
                                                               uint64_t seq, const uint64_t* __restrict__ flag) {
     using T = Tiling<TM, TN, WGM, WGN>;
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
 
     float acc[MS][NS][4];
     v4i d[MS][NS];
-    const v4i c_init = {DOT ? 0 : kMagicBits, DOT ? 0 : kMagicBits, DOT ? 0 : kMagicBits, DOT ? 0 : kMagicBits};
+    const v4i c_init = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
 #pragma unroll
     for (int mi = 0; mi < MS; ++mi)
 #pragma unroll
@@ -338,8 +338,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
             for (int r = 0; r < 4; ++r)
                 acc[mi][ni][r] = 0.0f;
         }
-    const uint32_t row_base = m0 + wm * T::WTM + 4u * (lane >> 4);
-    const uint32_t col_base = n0 + wn * T::WTN + (lane & 15u);
     float sc_prev[NS];
 #pragma unroll
     for (int ni = 0; ni < NS; ++ni)
@@ -370,7 +368,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
         const uint16_t* scl = reinterpret_cast<const uint16_t*>(lds_sc + (g & 3u) * T::SC_SLOT);
 #pragma unroll
         for (int ni = 0; ni < NS; ++ni)
-            sc_cur[ni] = DOT ? 0.0f : __half2float(__ushort_as_half(scl[wn * T::WTN + 16u * ni + (lane & 15u)]));
+            sc_cur[ni] = __half2float(__ushort_as_half(scl[wn * T::WTN + 16u * ni + (lane & 15u)]));
         __builtin_amdgcn_sched_barrier(0);
         // first half: the epilogue of group g-1 on each subtile, then restart it
 #pragma unroll
@@ -379,34 +377,18 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
             const float cneg = sc * -kMagicValue;  // exact
 #pragma unroll
             for (int mi = 0; mi < MS; ++mi) {
-                if constexpr (DOT) {
-                    // D of group g-1 as int16 at [m][n][g-1]
-                    const uint32_t n = col_base + 16u * ni;
-                    if (g > 0 && n < j.n) {
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const uint32_t m = row_base + 16u * mi + r;
-                            if (m < j.rows)
-                                reinterpret_cast<int16_t*>(j.out + (size_t)m * j.out_stride)[(size_t)n * groups + g - 1u] =
-                                    (int16_t)d[mi][ni][r];
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        acc[mi][ni][r] = acc[mi][ni][r] + __builtin_fmaf(sc, __int_as_float(d[mi][ni][r]), cneg);
-                }
+                for (int r = 0; r < 4; ++r)
+                    acc[mi][ni][r] = acc[mi][ni][r] + __builtin_fmaf(sc, __int_as_float(d[mi][ni][r]), cneg);
                 d[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ca[0][mi], cb[0][ni], c_init, 0, 0, 0);
             }
         }
-        if constexpr (!DOT) {
-            // per subtile its 8 epilogue VALU ops, then its restarting MFMA: the matrix
-            // pipe runs while the next subtile's VALU ops issue
+        // per subtile its 8 epilogue VALU ops, then its restarting MFMA: the matrix
+        // pipe runs while the next subtile's VALU ops issue
 #pragma unroll
-            for (int i = 0; i < MS * NS; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            }
+        for (int i = 0; i < MS * NS; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
         unpack_store(ex, g + 2u);
@@ -452,25 +434,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
 
     // no DMA may still be writing LDS when it is reused or the workgroup ends
     wait_dma<0>();
-    if constexpr (DOT) {
-        // D of the last group
-#pragma unroll
-        for (int mi = 0; mi < MS; ++mi)
-#pragma unroll
-            for (int ni = 0; ni < NS; ++ni) {
-                const uint32_t n = col_base + 16u * ni;
-                if (n >= j.n)
-                    continue;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t m = row_base + 16u * mi + r;
-                    if (m < j.rows)
-                        reinterpret_cast<int16_t*>(j.out + (size_t)m * j.out_stride)[(size_t)n * groups + groups - 1u] =
-                            (int16_t)d[mi][ni][r];
-                }
-            }
-        return;
-    }
     // epilogue of the last group
 #pragma unroll
     for (int ni = 0; ni < NS; ++ni) {
@@ -1140,6 +1103,152 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wv(GemmJob j, uint32_t mt
                                             orow + n);
             }
         }
+}
+
+// k_gemm_dots<TNS, GB, WAVES>: DOT_GROUPS.  Every group's dots stand alone (no sum over groups), so a
+// workgroup takes a 16 x (16 TNS) tile over the whole K, wave w the blocks of four
+// groups w, w + WAVES, ... (at most GB blocks in all): a block's rows and sign bits are requested at
+// once, straight into registers, expanded through the byte table, and each output's four dots
+// go to LDS as 8 bytes.  A row's part of the tile, [column][group] int16, is one contiguous run
+// of the output, so the tile leaves in 16- or 8-byte pieces of that run (2-byte ones for
+// odd-aligned views).  Bound by the launch for small jobs, by the stores for large ones; against
+// the accumulating kernels' tiles storing 2 bytes per output and group from the loop: 896->1000
+// x 37 rows 7.3 -> 5.3 us, 2048->2048 x 256 rows 27.7 -> 10.2, 8192->1000 x 64 rows 89.7 -> 11.3.
+template <int TNS, int GB, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_gemm_dots(GemmJob j, uint32_t mtiles, uint32_t ntiles, uint32_t band,
+                                                   uint64_t seq, const uint64_t* __restrict__ flag) {
+    constexpr uint32_t TN = 16u * TNS, THREADS = 64u * WAVES;
+    static_assert(THREADS >= 256u, "one thread per table entry");
+    static_assert(64 % TN == 0, "the tile's columns lie in one 64-feature tile");
+    // an output's dots: GB blocks of 8 bytes and 8 bytes that shift the next column's banks; for
+    // group counts that are no multiple of 4, a row's run as it leaves instead (no gaps)
+    constexpr uint32_t PITCH = 8u * GB + 8u, ROW = TN * PITCH;
+    __shared__ __attribute__((aligned(16))) unsigned char dots[16u * ROW];
+    __shared__ uint2 lut[256];
+    if (*flag == seq)
+        return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, chunk = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
+    const uint32_t m0 = tile.mt * 16u, n0 = tile.nt * TN, groups = j.groups, blocks = (groups + 3u) / 4u;
+    // rows past the end are clamped (never stored); so is the matrix tile of columns past the
+    // last one.  The K order inside a group is that of k_gemm_ks / k_gemm_wv.
+    const uint8_t* a_ptr = reinterpret_cast<const uint8_t*>(j.q) +
+                           (size_t)min(m0 + (lane & 15u), j.rows - 1u) * j.k + 32u * chunk;
+    const uint8_t* b_ptr[TNS];
+#pragma unroll
+    for (int ni = 0; ni < TNS; ++ni) {
+        const uint32_t n = n0 + 16u * ni + (lane & 15u), st = min(n >> 6, j.tiles - 1u);
+        b_ptr[ni] = reinterpret_cast<const uint8_t*>(j.wbits) + ((size_t)st * groups * kTile + (n & 63u)) * 16u +
+                    4u * chunk;
+    }
+    v4i a[4][2];
+    uint32_t bits[4][TNS];
+    const auto load = [&](uint32_t b) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+            const uint32_t g = min(4u * b + i, groups - 1u);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                a[i][h] = gload_v4i(a_ptr + (size_t)g * kGroup + 16u * h);
+#pragma unroll
+            for (int ni = 0; ni < TNS; ++ni)
+                bits[i][ni] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(
+                    (uintptr_t)(b_ptr[ni] + (size_t)g * kTile * 16u));
+        }
+    };
+    load(min(wave, blocks - 1u));
+    if (tid < 256u)
+        lut[tid] = make_uint2(pm1_nibble(tid & 15u), pm1_nibble(tid >> 4));
+    __syncthreads();
+    const v4i zero = {0, 0, 0, 0};
+    const bool gaps = groups % 4u == 0;
+    for (uint32_t b = wave; b < blocks; b += WAVES) {
+        v4i d[4][TNS];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+#pragma unroll
+            for (int ni = 0; ni < TNS; ++ni) {
+                const uint32_t w = bits[i][ni];
+                const uint2 e0 = lut[w & 0xffu], e1 = lut[(w >> 8) & 0xffu], e2 = lut[(w >> 16) & 0xffu], e3 = lut[w >> 24];
+                const v4i b0 = {(int)e0.x, (int)e0.y, (int)e1.x, (int)e1.y}, b1 = {(int)e2.x, (int)e2.y, (int)e3.x, (int)e3.y};
+                const v4i x = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][0], b0, zero, 0, 0, 0);
+                d[i][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][1], b1, x, 0, 0, 0);
+            }
+        if (b + WAVES < blocks)
+            load(b + WAVES);  // the next block's operands, in flight during the stores
+#pragma unroll
+        for (int ni = 0; ni < TNS; ++ni)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t row = 4u * chunk + r, col = 16u * ni + (lane & 15u);
+                if (gaps) {
+                    uint2 v;
+                    v.x = ((uint32_t)d[0][ni][r] & 0xffffu) | ((uint32_t)d[1][ni][r] << 16);
+                    v.y = ((uint32_t)d[2][ni][r] & 0xffffu) | ((uint32_t)d[3][ni][r] << 16);
+                    *reinterpret_cast<uint2*>(dots + row * ROW + col * PITCH + 8u * b) = v;
+                } else {
+                    uint16_t* run = reinterpret_cast<uint16_t*>(dots + row * ROW) + col * groups + 4u * b;
+#pragma unroll
+                    for (uint32_t i = 0; i < 4u; ++i)
+                        if (4u * b + i < groups)
+                            run[i] = (uint16_t)d[i][ni][r];
+                }
+            }
+    }
+    __syncthreads();
+    // the rows' runs: row r of the tile holds cols x groups int16 from out + r * stride + 2 n0 groups
+    const uint32_t cols = min(TN, j.n - n0), rows = min(16u, j.rows - m0);
+    unsigned char* const out = j.out + (size_t)m0 * j.out_stride + (size_t)n0 * groups * 2u;
+    const uint64_t align = j.out_stride | (uint64_t)(uintptr_t)out;
+    // piece p of the tile: elements of `per` groups each, `pieces` per row
+    const auto each = [&](uint32_t pieces, auto&& store) {
+        for (uint32_t i = tid; i < rows * pieces; i += THREADS) {
+            const uint32_t row = i / pieces, p = i - row * pieces;
+            store(row, p, out + (size_t)row * j.out_stride);
+        }
+    };
+    if (groups % 8u == 0 && (align & 15u) == 0) {
+        const uint32_t per = groups / 8u;
+        each(cols * per, [&](uint32_t row, uint32_t p, unsigned char* run) {
+            const uint32_t col = p / per, g = p - col * per;
+            const uint2* src = reinterpret_cast<const uint2*>(dots + row * ROW + col * PITCH + 16u * g);
+            const uint2 lo = src[0], hi = src[1];
+            const v4i v = {(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+            __builtin_nontemporal_store(v, (__attribute__((address_space(1))) v4i*)(uintptr_t)(run + 16u * p));
+        });
+    } else if (groups % 4u == 0 && (align & 7u) == 0) {
+        const uint32_t per = groups / 4u;
+        each(cols * per, [&](uint32_t row, uint32_t p, unsigned char* run) {
+            const uint32_t col = p / per, g = p - col * per;
+            *(__attribute__((address_space(1))) uint64_t*)(uintptr_t)(run + 8u * p) =
+                *reinterpret_cast<const uint64_t*>(dots + row * ROW + col * PITCH + 8u * g);
+        });
+    } else if (!gaps && (align & 15u) == 0) {
+        const uint32_t bytes = cols * groups * 2u;
+        each((bytes + 15u) / 16u, [&](uint32_t row, uint32_t p, unsigned char* run) {
+            const unsigned char* src = dots + row * ROW + 16u * p;
+            if (16u * p + 16u <= bytes) {
+                const v4i v = *reinterpret_cast<const v4i*>(src);
+                __builtin_nontemporal_store(v, (__attribute__((address_space(1))) v4i*)(uintptr_t)(run + 16u * p));
+            } else {
+                for (uint32_t i = 16u * p; i < bytes; i += 2u)
+                    *(__attribute__((address_space(1))) uint16_t*)(uintptr_t)(run + i) =
+                        *reinterpret_cast<const uint16_t*>(dots + row * ROW + i);
+            }
+        });
+    } else {  // any other alignment: value by value
+        each(cols * groups, [&](uint32_t row, uint32_t p, unsigned char* run) {
+            uint32_t at = 2u * p;
+            if (gaps) {
+                const uint32_t col = p / groups;
+                at = col * PITCH + 2u * (p - col * groups);
+            }
+            *(__attribute__((address_space(1))) uint16_t*)(uintptr_t)(run + 2u * p) =
+                *reinterpret_cast<const uint16_t*>(dots + row * ROW + at);
+        });
+    }
 }
 
 // k_gemm_kr<TMS, TNS, W, R>: F32-accumulating jobs with few rows, whose tiles are too
@@ -1973,17 +2082,21 @@ hipError_t launch_wv(hipStream_t stream, GemmJob job, uint64_t seq, const uint64
     return hipGetLastError();
 }
 
+template <int TNS, int GB, int WAVES>
+hipError_t launch_dots(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+    if (job.groups > 4u * GB || job.mode != MODE_DOT_I16)
+        return hipErrorInvalidValue;  // the selection below never asks for this
+    const uint32_t mtiles = (job.rows + 15u) / 16u, ntiles = gemm_ntiles(job, 16u * TNS);
+    launch_kernel((k_gemm_dots<TNS, GB, WAVES>), dim3(mtiles * ntiles), dim3(64 * WAVES), 0, stream, job, mtiles, ntiles,
+                  gemm_band(job, mtiles), seq, flag);
+    return hipGetLastError();
+}
+
 template <int TM, int TN, int WGM, int WGN>
 hipError_t launch_bits(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
     const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
-    const dim3 grid(mtiles * ntiles), block(64 * WGM * WGN);
-    const uint32_t band = gemm_band(job, mtiles);
-    if (job.mode == MODE_DOT_I16)
-        launch_kernel((k_gemm_bits<TM, TN, WGM, WGN, true>), grid, block, 0, stream, job, mtiles, ntiles, band, seq,
-                      flag);
-    else
-        launch_kernel((k_gemm_bits<TM, TN, WGM, WGN, false>), grid, block, 0, stream, job, mtiles, ntiles, band, seq,
-                      flag);
+    launch_kernel((k_gemm_bits<TM, TN, WGM, WGN>), dim3(mtiles * ntiles), dim3(64 * WGM * WGN), 0, stream, job, mtiles,
+                  ntiles, gemm_band(job, mtiles), seq, flag);
     return hipGetLastError();
 }
 
@@ -2016,7 +2129,15 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // tiles in one round, then 32 x 32 up to three rounds; 33..48 groups: 16 x 32 tiles, then
     // 16 x 64 tiles with the slices' running sums handed on (k_gemm_kc), each in one round;
     // 49..64 groups: 16 x 16 tiles in one round.
-    if (job.mode != MODE_DOT_I16) {
+    if (job.mode == MODE_DOT_I16) {
+        // 32-column tiles up to two per CU, and past 16 groups, whose tiles of 64 columns would
+        // not fit two workgroups' LDS
+        if (job.groups > 16u)
+            return launch_dots<2, 16, 8>(stream, job, seq, flag);
+        return blocks(16, 32) <= 2u * cus ? launch_dots<2, 4, 4>(stream, job, seq, flag)
+                                          : launch_dots<4, 4, 4>(stream, job, seq, flag);
+    }
+    {
         const uint32_t g = job.groups;
         if (g <= 16u) {
             if (job.rows <= 16u && blocks(16, 32) <= cus)
@@ -2048,7 +2169,7 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // tiles): one wave per 16 x 16 output block with its operands straight in registers,
     // while that makes at most three waves per CU (the blocks of 16 columns each load their
     // rows, and more of them outrun the loads a CU keeps in flight)
-    if (job.mode != MODE_DOT_I16 && job.rows <= 64u && (job.rows <= 32u || job.groups <= 16u) &&
+    if (job.rows <= 64u && (job.rows <= 32u || job.groups <= 16u) &&
         blocks(16, 16) <= 3u * cus)
         return launch_wv<1, 1, 1, 1, 8>(stream, job, seq, flag);
     // K >= 6144 with between half a round and one round of 32 x 64 tiles: eight waves
@@ -2056,7 +2177,7 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // 32 x 32 block, 8192->2048 x 256 21.6 against 23.3, 8192->1024 x 320-512 21.7-22.2
     // against 24.2-28.4; forced-choice sweep, bit-identical outputs; it loses at K = 4096,
     // below half a round and from a second round on)
-    if (job.mode != MODE_DOT_I16 && job.groups >= 48u && blocks(32, 64) > cus / 2u && blocks(32, 64) <= cus)
+    if (job.groups >= 48u && blocks(32, 64) > cus / 2u && blocks(32, 64) <= cus)
         return launch_ks<2, 4, 8, 3>(stream, job, seq, flag);
     // K split over four waves per 32 x 64 tile: 17..47 groups with between half a round and
     // one round of tiles (4096->2048 x 192 rows 14.0 us against 15.9 for 32 x 64
@@ -2065,20 +2186,20 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // rounds (6144->2048 x 384-512 rows 24.7-25.4 against 26.3-26.8, 6144->6144 x
     // 96-128 rows 23.8-24.4 against 26.1-26.5; forced-choice sweeps, bit-identical
     // outputs; at 16 groups and from a third round on the tiled kernels win)
-    if (job.mode != MODE_DOT_I16 && job.groups > 16u && job.groups < 48u && blocks(32, 64) > cus / 2u &&
+    if (job.groups > 16u && job.groups < 48u && blocks(32, 64) > cus / 2u &&
         blocks(32, 64) <= cus)
         return launch_ks<2, 4, 4, 3>(stream, job, seq, flag);
-    if (job.mode != MODE_DOT_I16 && job.groups >= 48u && blocks(32, 64) > cus && blocks(32, 64) <= 2u * cus)
+    if (job.groups >= 48u && blocks(32, 64) > cus && blocks(32, 64) <= 2u * cus)
         return launch_ks<2, 4, 4, 3>(stream, job, seq, flag);
     // a long K (>= 32 groups) with two to three 32 x 32 blocks per CU: a wave per block
     // beats the tiled kernels, whose per-group steps serialise over the long K
-    if (job.mode != MODE_DOT_I16 && job.groups >= 32u && blocks(32, 32) >= 2u * cus && blocks(32, 32) <= 3u * cus)
+    if (job.groups >= 32u && blocks(32, 32) >= 2u * cus && blocks(32, 32) <= 3u * cus)
         return launch_wv<2, 2, 1, 1, 4>(stream, job, seq, flag);
-    if (job.mode != MODE_DOT_I16 && blocks(128, 192) >= cus)
+    if (blocks(128, 192) >= cus)
         return launch_mx<128, 192, 2, 4>(stream, job, seq, flag);
-    if (job.mode != MODE_DOT_I16 && blocks(64, 128) >= cus && job.groups >= 32u)
+    if (blocks(64, 128) >= cus && job.groups >= 32u)
         return launch_mx<64, 128, 2, 4>(stream, job, seq, flag);
-    if (BNN_GEMM_CO && job.mode != MODE_DOT_I16 && blocks(128, 128) >= cus)
+    if (BNN_GEMM_CO && blocks(128, 128) >= cus)
         return launch_co<128, 128, 2, 2>(stream, job, seq, flag);
     // 128 x 128 tiles also where 64 x 128 ones would need a second round of workgroups
     // (one 8-wave 64 x 128 workgroup per CU fits the registers): 1.26-1.43x measured at
@@ -2090,7 +2211,7 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     if (blocks(64, 64) >= cus)
         return launch_bits<64, 64, 2, 2>(stream, job, seq, flag);
     const uint64_t enough = cus * 3u / 4u;
-    if (job.mode != MODE_DOT_I16 && blocks(32, 64) < enough && blocks(32, 32) <= cus) {
+    if (blocks(32, 64) < enough && blocks(32, 32) <= cus) {
         // too few tiles for the CUs (jobs of more than 48 groups get here): K split across
         // eight waves of a workgroup with 32 x 32 tiles while those fit one round, else four
         // waves with 32 x 16 tiles

@@ -208,3 +208,39 @@ def test_batch_jobs_on_the_matrix_cores(pkg, hipdev, oracle_fast, specs, shared)
         assert not bo.read().any()
     api.BNNX_BatchDestroy(batch)
     _free(mats, bi, bo)
+
+
+@pytest.mark.parametrize("k,n,rows,off,pad", [
+    (896, 1000, 37, 0, 0),      # 7 groups, 16-byte rows
+    (896, 1001, 20, 0, 0),      # rows that start at odd multiples of 2 bytes
+    (128, 33, 17, 2, 0),        # one group, a view at offset 2
+    (2048, 100, 16, 0, 0),      # 16 groups: 16-byte pieces, a partial column tile
+    (512, 70, 49, 8, 8),        # 4 groups, 8-byte aligned rows
+    (2048, 70, 9, 2, 6),        # 16 groups from an odd address: value by value
+    (2176, 65, 18, 0, 0),       # 17 groups
+    (8192, 40, 33, 0, 16),      # 64 groups
+    (1024, 5000, 130, 0, 0),    # more than two tiles per CU: 64-column tiles
+])
+def test_dot_groups_rows(pkg, hipdev, oracle_fast, k, n, rows, off, pad):
+    """DOT_GROUPS of many rows: every store width; padding and neighbours untouched."""
+    from bnn_cases import fast_oracle
+    host = pkg.synth.matrix(n, k, seed=k + n)
+    x = pkg.synth.int8_uniform(rows, k, seed=3)
+    m = hipdev.matrix(*host)
+    row = n * (k // 128) * 2
+    bi, bo = hipdev.buffer(x.nbytes), hipdev.buffer(off + rows * (row + pad) + 64)
+    bi.write(x)
+    bo.write(np.full(bo.nbytes, 0x5a, np.uint8))
+    T = pkg.Type
+    job = pkg.Job(int(pkg.Op.DOT_GROUPS), m.handle.value, bi.view(T.I8), bo.view(T.I16, off, row + pad), rows)
+    print(f"dots {k}->{n} x {rows}", flush=True)
+    assert hipdev.execute(job) == pkg.Status.OK
+    raw = bo.read()
+    want = np.full(bo.nbytes, 0x5a, np.uint8)
+    dots = fast_oracle(pkg, oracle_fast, "DOT_GROUPS", *host, x).reshape(rows, -1).view(np.uint8)
+    for r in range(rows):
+        want[off + r * (row + pad):off + r * (row + pad) + row] = dots[r]
+    assert np.array_equal(raw, want)
+    bi.free()
+    bo.free()
+    m.destroy()
