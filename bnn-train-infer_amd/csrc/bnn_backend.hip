@@ -770,14 +770,13 @@ GemmJob make_gemm(const JobPlan& p, const PrepJob& pj, unsigned char* out, size_
 
 // `more` as a further part of the launch of `j` (equal k, rows and mode).
 void add_part(GemmJob* j, const GemmJob& more) {
-    j->parts[j->extra++] =
-        GemmPart{more.wbits, more.wscale, more.q, more.rscale, more.out, more.out_stride, more.n, more.tiles, 0, 0};
+    j->parts[j->extra++] = GemmPart{more.wbits, more.q, more.rscale, more.out, more.out_stride, more.n, 0};
 }
 
-// Completion of a single-row launch whose `grid` workgroups each store seq into their own
-// pinned word (status_host from kDoneFlagWord) once their results are visible to the host:
+// Completion of a call whose last launch's `grid` workgroups each store seq into their own
+// pinned word (status_host from kDoneFlagWord) once their results are written to memory:
 // spin on those instead of waiting for the end of the kernel, which the runtime reports
-// several microseconds later.  Past a bound far above any single-row kernel (or with
+// several microseconds later.  Past a bound above the calls this pays for (or with
 // kernel timing on, whose events are resolved at a stream synchronisation) the ordinary
 // stream wait takes over; it also reports device errors.
 BNN_Status finish(BNN_Device device, hipError_t e, uint64_t seq);
@@ -884,12 +883,15 @@ BNN_Status run_single_row(BNN_Device device, const BNN_Job* job, const JobPlan& 
 // A multi-row job (or a single row the fused kernel does not take) in chunks of
 // `chunk` rows whose quantised forms occupy the first `rows_bytes` of `scratch`,
 // followed by the chunk's staging rows when the output view is not aligned.
-// mfma: the rows run on the matrix cores (the matrix's +1/-1 copy must exist).
+// mfma: the rows run on the matrix cores.
 BNN_Status run_rows(BNN_Device device, const BNN_Job* job, const JobPlan& p, bool mfma, unsigned char* scratch,
                     size_t chunk, size_t rows_bytes, hipError_t e) {
     const uint32_t rows = job->rows;
     unsigned char* staging = scratch + rows_bytes;
     const uint64_t seq = ++device->seq;
+    // a job that is one matrix-core launch signals its end itself
+    const bool signal = mfma && chunk >= rows && p.out_aligned && !device->timing;
+    uint32_t signals = 0;
     if (e == hipSuccess && chunk < rows) {
         // every row is checked before any chunk writes output
         const PrepJob all = make_prep(p, p.in_base, rows, scratch);
@@ -908,9 +910,11 @@ BNN_Status run_rows(BNN_Device device, const BNN_Job* job, const JobPlan& p, boo
         unsigned char* dst = p.out_aligned ? p.out_base + r0 * p.out_stride : staging;
         const size_t dst_stride = p.out_aligned ? p.out_stride : p.out_row;
         if (mfma) {
-            const GemmJob gj = make_gemm(p, pj, dst, dst_stride);
-            e = timed(device, KK_GEMM,
-                      [&] { return launch_gemm(device->stream, gj, device->cu_count, seq, device->flag_dev); });
+            GemmJob gj = make_gemm(p, pj, dst, dst_stride);
+            gj.done = signal ? device->status_host + kDoneFlagWord : nullptr;
+            e = timed(device, KK_GEMM, [&] {
+                return launch_gemm(device->stream, gj, device->cu_count, seq, device->flag_dev, &signals);
+            });
         } else {
             const DotJob dj = make_dot(p, pj, dst, dst_stride);
             e = timed(device, KK_DOT,
@@ -922,7 +926,7 @@ BNN_Status run_rows(BNN_Device device, const BNN_Job* job, const JobPlan& p, boo
                                       p.out_stride, p.out_row, rc, seq, device->flag_dev);
             });
     }
-    return finish(device, e, seq);
+    return signals && e == hipSuccess ? finish_signalled(device, e, seq, signals) : finish(device, e, seq);
 }
 
 bool single_row_path(const BNN_Job* job, const JobPlan& p) {

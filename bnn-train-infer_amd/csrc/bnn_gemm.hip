@@ -86,7 +86,7 @@ __device__ __forceinline__ TileRC gemm_tile_of_block(uint32_t b, uint32_t grid, 
 }
 
 // The tile's column tile within its part of the job, whose matrix and output `j` then
-// describes (wave-uniform: the argument block's loads and a few scalar selects, once).
+// describes (wave-uniform; as selects without the branch it measured the same or slower).
 __device__ __forceinline__ uint32_t select_part(GemmJob& j, uint32_t nt) {
     uint32_t first = 0;
     if (j.extra != 0u) {
@@ -95,13 +95,13 @@ __device__ __forceinline__ uint32_t select_part(GemmJob& j, uint32_t nt) {
             if (i < j.extra && nt >= j.parts[i].first) {
                 const GemmPart& p = j.parts[i];
                 j.wbits = p.wbits;
-                j.wscale = p.wscale;
                 j.q = p.q;
                 j.rscale = p.rscale;
                 j.out = p.out;
                 j.out_stride = p.out_stride;
                 j.n = p.n;
-                j.tiles = p.tiles;
+                j.tiles = (p.n + kTile - 1u) / kTile;
+                j.wscale = reinterpret_cast<const uint16_t*>(p.wbits + (size_t)j.tiles * j.groups * kTile);
                 first = p.first;
             }
         }
@@ -166,6 +166,49 @@ __device__ __forceinline__ float row_scale(const GemmJob& j, uint32_t m) {
     return *(const __attribute__((address_space(1))) float*)(j.rscale + m);
 }
 
+// Output stores: nontemporal, or written through to memory (system-coherent, sc0 sc1) in a
+// launch that signals its end itself (gemm_signal).
+__device__ __forceinline__ void put(float* p, float v, bool through) {
+    if (through)
+        __hip_atomic_store((__attribute__((address_space(1))) float*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    else
+        __builtin_nontemporal_store(v, (__attribute__((address_space(1))) float*)p);
+}
+__device__ __forceinline__ void put4(void* p, v4i v, bool through) {
+    if (through)
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+    else
+        __builtin_nontemporal_store(v, (__attribute__((address_space(1))) v4i*)p);
+}
+
+__device__ __forceinline__ void put8(void* p, uint64_t v, bool through) {
+    if (through)
+        __hip_atomic_store((__attribute__((address_space(1))) uint64_t*)p, v, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    else
+        *(__attribute__((address_space(1))) uint64_t*)p = v;
+}
+__device__ __forceinline__ void put2(void* p, uint16_t v, bool through) {
+    if (through)
+        asm volatile("global_store_short %0, %1, off sc0 sc1" ::"v"(p), "v"((uint32_t)v) : "memory");
+    else
+        *(__attribute__((address_space(1))) uint16_t*)p = v;
+}
+
+// The end of a workgroup in a launch whose caller waits for it (GemmJob::done): once the
+// stores of all its waves are complete (vmcnt), the workgroup stores seq into its own pinned
+// host word; the host spins on those words instead of waiting for the end of the kernel, which
+// the runtime reports several microseconds later (a call of 2048->6144 x 64 rows 20.6 -> 17.5
+// us, 384->278 x 33 rows 19.0 -> 14.0).  Every thread of the workgroup comes here.
+__device__ __forceinline__ void gemm_signal(const GemmJob& j, uint64_t seq) {
+    if (j.done == nullptr)
+        return;
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(j.done + blockIdx.x, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ void barrier() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");  // no LDS access moves across it
@@ -204,8 +247,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
     using T = Tiling<TM, TN, WGM, WGN>;
     constexpr int MS = T::MS, NS = T::NS, THREADS = T::THREADS;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[T::SMEM];
-    if (*flag == seq)
+    if (*flag == seq) {
+        gemm_signal(j, seq);
         return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WGN, wn = wave % WGN;
@@ -459,36 +504,43 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_
                    (lane & 15u)] = acc[mi][ni][r];
     wait_dma<0>();
     barrier();
-    const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
-    const bool scaled = j.mode == MODE_SUM_SCALED;
+    // stored in one of two forms, each without a branch per value
+    const auto store = [&](auto through) {
+        const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
+        const bool scaled = j.mode == MODE_SUM_SCALED;
 #pragma unroll
-    for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
-        const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
-        const uint32_t m = m0 + row, n = n0 + col;
-        if (m >= j.rows || n >= j.n)
-            continue;
-        float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
-        if (scaled) {
-            const float s = row_scale(j, m);
-            v.x = v.x * s;
-            v.y = v.y * s;
-            v.z = v.z * s;
-            v.w = v.w * s;
+        for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
+            const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
+            const uint32_t m = m0 + row, n = n0 + col;
+            if (m >= j.rows || n >= j.n)
+                continue;
+            float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
+            if (scaled) {
+                const float s = row_scale(j, m);
+                v.x = v.x * s;
+                v.y = v.y * s;
+                v.z = v.z * s;
+                v.w = v.w * s;
+            }
+            float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
+            if (vec && n + 4u <= j.n) {
+                put4(dst, v4i{__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)}, through);
+            } else {
+                put(dst, v.x, through);
+                if (n + 1u < j.n)
+                    put(dst + 1, v.y, through);
+                if (n + 2u < j.n)
+                    put(dst + 2, v.z, through);
+                if (n + 3u < j.n)
+                    put(dst + 3, v.w, through);
+            }
         }
-        float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
-        if (vec && n + 4u <= j.n) {
-            const v4f w = {v.x, v.y, v.z, v.w};
-            __builtin_nontemporal_store(w, reinterpret_cast<v4f*>(dst));
-        } else {
-            dst[0] = v.x;
-            if (n + 1u < j.n)
-                dst[1] = v.y;
-            if (n + 2u < j.n)
-                dst[2] = v.z;
-            if (n + 3u < j.n)
-                dst[3] = v.w;
-        }
-    }
+    };
+    if (j.done)
+        store(std::true_type{});
+    else
+        store(std::false_type{});
+    gemm_signal(j, seq);
 }
 
 // k_gemm_co<TM, TN, WGM, WGN>: GEMM / GEMM_F32 with two workgroups per CU.  The
@@ -508,8 +560,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
     using T = Tiling<TM, TN, WGM, WGN, 2>;
     constexpr int MS = T::MS, NS = T::NS, THREADS = T::THREADS;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[T::SMEM];
-    if (*flag == seq)
+    if (*flag == seq) {
+        gemm_signal(j, seq);
         return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WGN, wn = wave % WGN;
@@ -709,47 +763,78 @@ __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(
                    (lane & 15u)] = acc[mi][ni][r];
     wait_dma<0>();
     barrier();
-    const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
-    const bool scaled = j.mode == MODE_SUM_SCALED;
+    // stored in one of two forms, each without a branch per value
+    const auto store = [&](auto through) {
+        const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
+        const bool scaled = j.mode == MODE_SUM_SCALED;
 #pragma unroll
-    for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
-        const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
-        const uint32_t m = m0 + row, n = n0 + col;
-        if (m >= j.rows || n >= j.n)
-            continue;
-        float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
-        if (scaled) {
-            const float s = row_scale(j, m);
-            v.x = v.x * s;
-            v.y = v.y * s;
-            v.z = v.z * s;
-            v.w = v.w * s;
+        for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
+            const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
+            const uint32_t m = m0 + row, n = n0 + col;
+            if (m >= j.rows || n >= j.n)
+                continue;
+            float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
+            if (scaled) {
+                const float s = row_scale(j, m);
+                v.x = v.x * s;
+                v.y = v.y * s;
+                v.z = v.z * s;
+                v.w = v.w * s;
+            }
+            float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
+            if (vec && n + 4u <= j.n) {
+                put4(dst, v4i{__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)}, through);
+            } else {
+                put(dst, v.x, through);
+                if (n + 1u < j.n)
+                    put(dst + 1, v.y, through);
+                if (n + 2u < j.n)
+                    put(dst + 2, v.z, through);
+                if (n + 3u < j.n)
+                    put(dst + 3, v.w, through);
+            }
         }
-        float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
-        if (vec && n + 4u <= j.n) {
-            const v4f w = {v.x, v.y, v.z, v.w};
-            __builtin_nontemporal_store(w, reinterpret_cast<v4f*>(dst));
-        } else {
-            dst[0] = v.x;
-            if (n + 1u < j.n)
-                dst[1] = v.y;
-            if (n + 2u < j.n)
-                dst[2] = v.z;
-            if (n + 3u < j.n)
-                dst[3] = v.w;
-        }
-    }
+    };
+    if (j.done)
+        store(std::true_type{});
+    else
+        store(std::false_type{});
+    gemm_signal(j, seq);
 }
 
 uint32_t gemm_band(const GemmJob& job, uint32_t mtiles);
 uint32_t gemm_ntiles(GemmJob& job, uint32_t tn);
 
-template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_co(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
-    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
-    launch_kernel((k_gemm_co<TM, TN, WGM, WGN>), dim3(mtiles * ntiles), dim3(64 * WGM * WGN), 0, stream, job, mtiles,
-                  ntiles, gemm_band(job, mtiles), seq, flag);
+// What every launcher passes on.
+struct GemmLaunch {
+    hipStream_t stream;
+    uint64_t seq;
+    const uint64_t* flag;
+    uint32_t* signals;  // with job.done: receives the workgroups that signal
+};
+
+// One workgroup per tile.  Launches of more than kDoneWords workgroups do not signal: from a
+// second round of workgroups on, stores written through cost what the earlier word to the
+// host saves (2048->6144 x 128 rows, 768 workgroups, 23.6 us either way; 2048->4213 x 250
+// rows, 1056 of them counted on a device word, 28.0 -> 30.0).
+template <class Kernel>
+hipError_t launch_tiles(const GemmLaunch& at, Kernel kernel, uint32_t threads, GemmJob& job, uint32_t mtiles,
+                        uint32_t ntiles) {
+    const uint32_t grid = mtiles * ntiles;
+    if (grid > kDoneWords)
+        job.done = nullptr;
+    if (job.done)
+        *at.signals = grid;
+    launch_kernel(kernel, dim3(grid), dim3(threads), 0, at.stream, job, mtiles, ntiles, gemm_band(job, mtiles), at.seq,
+                  at.flag);
     return hipGetLastError();
+}
+
+
+template <int TM, int TN, int WGM, int WGN>
+hipError_t launch_co(const GemmLaunch& at, GemmJob job) {
+    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
+    return launch_tiles(at, k_gemm_co<TM, TN, WGM, WGN>, 64 * WGM * WGN, job, mtiles, ntiles);
 }
 
 // k_gemm_ks: F32-accumulating jobs with too few tiles to give every CU a workgroup.
@@ -787,8 +872,10 @@ __global__ __launch_bounds__(64 * W) void k_gemm_ks(GemmJob j, uint32_t mtiles, 
     static_assert(TN <= 64, "a tile's columns lie in one 64-feature tile of the matrix layout");
     __shared__ __attribute__((aligned(16))) float prod[W][BLOCKS * 4u];  // [wave][subtile][lane][4]
     __shared__ uint2 lut[256];
-    if (*flag == seq)
+    if (*flag == seq) {
+        gemm_signal(j, seq);
         return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
@@ -925,23 +1012,31 @@ __global__ __launch_bounds__(64 * W) void k_gemm_ks(GemmJob j, uint32_t mtiles, 
         for (int d = 0; d < DEPTH; ++d)
             round(d, r + d);
     }
-    // block NT*i + tid is subtile W*i + wave, lane `lane`
+    // stored in one of two forms, each without a branch per value
+    const auto store = [&](auto through) {
+        // block NT*i + tid is subtile W*i + wave, lane `lane`
 #pragma unroll
-    for (int i = 0; i < (int)PER_THREAD; ++i) {
-        const uint32_t sub = W * i + wave;
-        if (sub >= SUBS)
-            continue;
-        const uint32_t mi = sub / TNS, ni = sub % TNS;
-        const uint32_t n = n0 + 16u * ni + (lane & 15u);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t m = m0 + 16u * mi + 4u * (lane >> 4) + r;
-            if (m >= j.rows || n >= j.n)
+        for (int i = 0; i < (int)PER_THREAD; ++i) {
+            const uint32_t sub = W * i + wave;
+            if (sub >= SUBS)
                 continue;
-            float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
-            __builtin_nontemporal_store(j.mode == MODE_SUM_SCALED ? acc[i][r] * rs[i][r] : acc[i][r], orow + n);
+            const uint32_t mi = sub / TNS, ni = sub % TNS;
+            const uint32_t n = n0 + 16u * ni + (lane & 15u);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t m = m0 + 16u * mi + 4u * (lane >> 4) + r;
+                if (m >= j.rows || n >= j.n)
+                    continue;
+                float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
+                put(orow + n, j.mode == MODE_SUM_SCALED ? acc[i][r] * rs[i][r] : acc[i][r], through);
+            }
         }
-    }
+    };
+    if (j.done)
+        store(std::true_type{});
+    else
+        store(std::false_type{});
+    gemm_signal(j, seq);
 }
 
 // k_gemm_wv: F32-accumulating jobs with few rows.  Every wave computes a (16*MS) x
@@ -971,8 +1066,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wv(GemmJob j, uint32_t mt
     static_assert(DEPTH >= 2 && DEPTH % 2 == 0, "two D sets alternate with the ring slots");
     static_assert(16 * NS <= 64 && 64 % (16 * NS) == 0, "a wave's columns lie in one 64-feature tile");
     __shared__ uint2 lut[256];
-    if (*flag == seq)
+    if (*flag == seq) {
+        gemm_signal(j, seq);
         return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WN, wn = wave % WN;
@@ -1086,23 +1183,30 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wv(GemmJob j, uint32_t mt
     }
     epilogue(dd[(DEPTH - 1) & 1]);  // the last step's group
 
+    // stored in one of two forms, each without a branch per value
+    const auto store = [&](auto through) {
 #pragma unroll
-    for (int mi = 0; mi < MS; ++mi)
+        for (int mi = 0; mi < MS; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < NS; ++ni) {
-            const uint32_t n = n0 + 16u * ni + (lane & 15u);
-            if (n >= j.n)
-                continue;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t m = m0 + 16u * mi + 4u * (lane >> 4) + r;
-                if (m >= j.rows)
+            for (int ni = 0; ni < NS; ++ni) {
+                const uint32_t n = n0 + 16u * ni + (lane & 15u);
+                if (n >= j.n)
                     continue;
-                float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
-                __builtin_nontemporal_store(j.mode == MODE_SUM_SCALED ? acc[mi][ni][r] * j.rscale[m] : acc[mi][ni][r],
-                                            orow + n);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t m = m0 + 16u * mi + 4u * (lane >> 4) + r;
+                    if (m >= j.rows)
+                        continue;
+                    float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
+                    put(orow + n, j.mode == MODE_SUM_SCALED ? acc[mi][ni][r] * j.rscale[m] : acc[mi][ni][r], through);
+                }
             }
-        }
+    };
+    if (j.done)
+        store(std::true_type{});
+    else
+        store(std::false_type{});
+    gemm_signal(j, seq);
 }
 
 // k_gemm_dots<TNS, GB, WAVES>: DOT_GROUPS.  Every group's dots stand alone (no sum over groups), so a
@@ -1125,12 +1229,15 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_dots(GemmJob j, uint32_t mt
     constexpr uint32_t PITCH = 8u * GB + 8u, ROW = TN * PITCH;
     __shared__ __attribute__((aligned(16))) unsigned char dots[16u * ROW];
     __shared__ uint2 lut[256];
-    if (*flag == seq)
+    if (*flag == seq) {
+        gemm_signal(j, seq);
         return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u, chunk = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
     tile.nt = select_part(j, tile.nt);
+    const bool through = j.done != nullptr;
     const uint32_t m0 = tile.mt * 16u, n0 = tile.nt * TN, groups = j.groups, blocks = (groups + 3u) / 4u;
     // rows past the end are clamped (never stored); so is the matrix tile of columns past the
     // last one.  The K order inside a group is that of k_gemm_ks / k_gemm_wv.
@@ -1216,14 +1323,13 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_dots(GemmJob j, uint32_t mt
             const uint2* src = reinterpret_cast<const uint2*>(dots + row * ROW + col * PITCH + 16u * g);
             const uint2 lo = src[0], hi = src[1];
             const v4i v = {(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
-            __builtin_nontemporal_store(v, (__attribute__((address_space(1))) v4i*)(uintptr_t)(run + 16u * p));
+            put4(run + 16u * p, v, through);
         });
     } else if (groups % 4u == 0 && (align & 7u) == 0) {
         const uint32_t per = groups / 4u;
         each(cols * per, [&](uint32_t row, uint32_t p, unsigned char* run) {
             const uint32_t col = p / per, g = p - col * per;
-            *(__attribute__((address_space(1))) uint64_t*)(uintptr_t)(run + 8u * p) =
-                *reinterpret_cast<const uint64_t*>(dots + row * ROW + col * PITCH + 8u * g);
+            put8(run + 8u * p, *reinterpret_cast<const uint64_t*>(dots + row * ROW + col * PITCH + 8u * g), through);
         });
     } else if (!gaps && (align & 15u) == 0) {
         const uint32_t bytes = cols * groups * 2u;
@@ -1231,11 +1337,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_dots(GemmJob j, uint32_t mt
             const unsigned char* src = dots + row * ROW + 16u * p;
             if (16u * p + 16u <= bytes) {
                 const v4i v = *reinterpret_cast<const v4i*>(src);
-                __builtin_nontemporal_store(v, (__attribute__((address_space(1))) v4i*)(uintptr_t)(run + 16u * p));
+                put4(run + 16u * p, v, through);
             } else {
                 for (uint32_t i = 16u * p; i < bytes; i += 2u)
-                    *(__attribute__((address_space(1))) uint16_t*)(uintptr_t)(run + i) =
-                        *reinterpret_cast<const uint16_t*>(dots + row * ROW + i);
+                    put2(run + i, *reinterpret_cast<const uint16_t*>(dots + row * ROW + i), through);
             }
         });
     } else {  // any other alignment: value by value
@@ -1245,10 +1350,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_dots(GemmJob j, uint32_t mt
                 const uint32_t col = p / groups;
                 at = col * PITCH + 2u * (p - col * groups);
             }
-            *(__attribute__((address_space(1))) uint16_t*)(uintptr_t)(run + 2u * p) =
-                *reinterpret_cast<const uint16_t*>(dots + row * ROW + at);
+            put2(run + 2u * p, *reinterpret_cast<const uint16_t*>(dots + row * ROW + at), through);
         });
     }
+    gemm_signal(j, seq);
 }
 
 // k_gemm_kr<TMS, TNS, W, R>: F32-accumulating jobs with few rows, whose tiles are too
@@ -1455,8 +1560,10 @@ __global__ __launch_bounds__(64 * W) void k_gemm_kr(GemmJob j, uint32_t mtiles, 
             mma(std::integral_constant<uint32_t, i - 2u>{});
     });
 
-    if (failed_seq == seq)
-        return;  // an illegal input row in this job: write nothing (the whole workgroup)
+    if (failed_seq == seq) {  // an illegal input row in this job: write nothing (the whole workgroup)
+        gemm_signal(j, seq);
+        return;
+    }
 
     // 3. the products by group into LDS (over the operands: every wave has read its own
     // by the barrier), then the in-order sums
@@ -1500,17 +1607,25 @@ __global__ __launch_bounds__(64 * W) void k_gemm_kr(GemmJob j, uint32_t mtiles, 
     }
     for (; g < groups; ++g)
         add_group(g);
+    // stored in one of two forms, each without a branch per value
+    const auto store = [&](auto through) {
 #pragma unroll
-    for (uint32_t it = 0; it < ITEMS; ++it) {
-        const uint32_t idx = T::NT * it + tid;
-        const uint32_t blk = idx >> 2, e = idx & 3u, sub = blk >> 6, l = blk & 63u;
-        const uint32_t mi = sub / TNS, ni = sub % TNS;
-        const uint32_t n = n0 + 16u * ni + (l & 15u), m = m0 + 16u * mi + 4u * (l >> 4) + e;
-        if (idx >= ELEMS || n >= j.n || m >= j.rows)
-            continue;
-        float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
-        __builtin_nontemporal_store(scaled ? acc[it] * rs[it] : acc[it], orow + n);
-    }
+        for (uint32_t it = 0; it < ITEMS; ++it) {
+            const uint32_t idx = T::NT * it + tid;
+            const uint32_t blk = idx >> 2, e = idx & 3u, sub = blk >> 6, l = blk & 63u;
+            const uint32_t mi = sub / TNS, ni = sub % TNS;
+            const uint32_t n = n0 + 16u * ni + (l & 15u), m = m0 + 16u * mi + 4u * (l >> 4) + e;
+            if (idx >= ELEMS || n >= j.n || m >= j.rows)
+                continue;
+            float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
+            put(orow + n, scaled ? acc[it] * rs[it] : acc[it], through);
+        }
+    };
+    if (j.done)
+        store(std::true_type{});
+    else
+        store(std::false_type{});
+    gemm_signal(j, seq);
 }
 
 // k_gemm_kc<TMS, TNW, WN, KS, G>: F32-accumulating jobs with few rows and at most G
@@ -1658,8 +1773,10 @@ __global__ __launch_bounds__(64 * WN * KS) void k_gemm_kc(GemmJob j, uint32_t mt
         if constexpr (i >= 2u)
             mma(std::integral_constant<uint32_t, i - 2u>{});
     });
-    if (failed_seq == seq)
-        return;  // an illegal input row in this job: write nothing (the whole workgroup)
+    if (failed_seq == seq) {  // an illegal input row in this job: write nothing (the whole workgroup)
+        gemm_signal(j, seq);
+        return;
+    }
 
     // 3. the running sums along the slices: slice 0 from +0, slice t after barrier t
     v4f acc[TMS][TNW];
@@ -1705,25 +1822,31 @@ __global__ __launch_bounds__(64 * WN * KS) void k_gemm_kc(GemmJob j, uint32_t mt
             add_slice();
         }
     }
-    if (s != (uint32_t)KS - 1u)
-        return;
-    const bool scaled = j.mode == MODE_SUM_SCALED;
+    // stored in one of two forms, each without a branch per value
+    const auto store = [&](auto through) {
+        const bool scaled = j.mode == MODE_SUM_SCALED;
 #pragma unroll
-    for (uint32_t mi = 0; mi < (uint32_t)TMS; ++mi)
+        for (uint32_t mi = 0; mi < (uint32_t)TMS; ++mi)
 #pragma unroll
-        for (uint32_t ni = 0; ni < (uint32_t)TNW; ++ni) {
-            const uint32_t n = n0 + 16u * (nn * TNW + ni) + lrow;
-            if (n >= j.n)
-                continue;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t m = m0 + 16u * mi + 4u * chunk + e;
-                if (m >= j.rows)
+            for (uint32_t ni = 0; ni < (uint32_t)TNW; ++ni) {
+                const uint32_t n = n0 + 16u * (nn * TNW + ni) + lrow;
+                if (n >= j.n || s != (uint32_t)KS - 1u)  // the last slice holds the sums
                     continue;
-                float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
-                __builtin_nontemporal_store(scaled ? acc[mi][ni][e] * rs[mi][e] : acc[mi][ni][e], orow + n);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t m = m0 + 16u * mi + 4u * chunk + e;
+                    if (m >= j.rows)
+                        continue;
+                    float* orow = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride);
+                    put(orow + n, scaled ? acc[mi][ni][e] * rs[mi][e] : acc[mi][ni][e], through);
+                }
             }
-        }
+    };
+    if (j.done)
+        store(std::true_type{});
+    else
+        store(std::false_type{});
+    gemm_signal(j, seq);
 }
 
 // k_gemm_mx<TM, TN, WGM, WGN>: GEMM / GEMM_F32 with a chip's worth of TM x TN tiles,
@@ -1789,8 +1912,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t 
     using T = MxTiling<TM, TN, WGM, WGN>;
     constexpr uint32_t MS = T::MS, NS = T::NS, THREADS = T::THREADS, DEPTH = T::DEPTH;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[T::SMEM];
-    if (*flag == seq)
+    if (*flag == seq) {
+        gemm_signal(j, seq);
         return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u, chunk = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave / WGN, wn = wave % WGN;
@@ -1972,36 +2097,43 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t 
                 so[(wm * T::WTM + 16u * mi + 4u * chunk + r) * T::OUT_STRIDE + wn * T::WTN + 16u * ni + (lane & 15u)] =
                     acc[mi][ni][r];
     barrier();
-    const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
-    const bool scaled = j.mode == MODE_SUM_SCALED;
+    // stored in one of two forms, each without a branch per value
+    const auto store = [&](auto through) {
+        const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
+        const bool scaled = j.mode == MODE_SUM_SCALED;
 #pragma unroll
-    for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
-        const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
-        const uint32_t m = m0 + row, n = n0 + col;
-        if (m >= j.rows || n >= j.n)
-            continue;
-        float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
-        if (scaled) {
-            const float s = row_scale(j, m);
-            v.x = v.x * s;
-            v.y = v.y * s;
-            v.z = v.z * s;
-            v.w = v.w * s;
+        for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
+            const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
+            const uint32_t m = m0 + row, n = n0 + col;
+            if (m >= j.rows || n >= j.n)
+                continue;
+            float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
+            if (scaled) {
+                const float s = row_scale(j, m);
+                v.x = v.x * s;
+                v.y = v.y * s;
+                v.z = v.z * s;
+                v.w = v.w * s;
+            }
+            float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
+            if (vec && n + 4u <= j.n) {
+                put4(dst, v4i{__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)}, through);
+            } else {
+                put(dst, v.x, through);
+                if (n + 1u < j.n)
+                    put(dst + 1, v.y, through);
+                if (n + 2u < j.n)
+                    put(dst + 2, v.z, through);
+                if (n + 3u < j.n)
+                    put(dst + 3, v.w, through);
+            }
         }
-        float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
-        if (vec && n + 4u <= j.n) {
-            const v4f w = {v.x, v.y, v.z, v.w};
-            __builtin_nontemporal_store(w, reinterpret_cast<v4f*>(dst));
-        } else {
-            dst[0] = v.x;
-            if (n + 1u < j.n)
-                dst[1] = v.y;
-            if (n + 2u < j.n)
-                dst[2] = v.z;
-            if (n + 3u < j.n)
-                dst[3] = v.w;
-        }
-    }
+    };
+    if (j.done)
+        store(std::true_type{});
+    else
+        store(std::false_type{});
+    gemm_signal(j, seq);
 }
 
 // The band width (in M tiles) of gemm_tile_of_block: an XCD covering band M tiles of
@@ -2035,69 +2167,55 @@ uint32_t gemm_ntiles(GemmJob& job, uint32_t tn) {
 }
 
 template <int TMS, int TNS, int W, int DEPTH>
-hipError_t launch_ks(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_ks(const GemmLaunch& at, GemmJob job) {
     const uint32_t mtiles = (job.rows + 16u * TMS - 1u) / (16u * TMS);
     const uint32_t ntiles = gemm_ntiles(job, 16u * TNS);
-    launch_kernel((k_gemm_ks<TMS, TNS, W, DEPTH>), dim3(mtiles * ntiles), dim3(64 * W), 0, stream, job, mtiles, ntiles,
-                  gemm_band(job, mtiles), seq, flag);
-    return hipGetLastError();
+    return launch_tiles(at, k_gemm_ks<TMS, TNS, W, DEPTH>, 64 * W, job, mtiles, ntiles);
 }
 
 template <int TMS, int TNS, int W, int R>
-hipError_t launch_kr(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_kr(const GemmLaunch& at, GemmJob job) {
     if (job.groups > (uint32_t)(W * R) || job.mode == MODE_DOT_I16)
         return hipErrorInvalidValue;  // the selection below never asks for this
     const uint32_t mtiles = (job.rows + 16u * TMS - 1u) / (16u * TMS);
     const uint32_t ntiles = gemm_ntiles(job, 16u * TNS);
-    launch_kernel((k_gemm_kr<TMS, TNS, W, R>), dim3(mtiles * ntiles), dim3(64 * W), 0, stream, job, mtiles, ntiles,
-                  gemm_band(job, mtiles), seq, flag);
-    return hipGetLastError();
+    return launch_tiles(at, k_gemm_kr<TMS, TNS, W, R>, 64 * W, job, mtiles, ntiles);
 }
 
 template <int TMS, int TNW, int WN, int KS, int G>
-hipError_t launch_kc(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_kc(const GemmLaunch& at, GemmJob job) {
     if (job.groups > (uint32_t)G || job.mode == MODE_DOT_I16)
         return hipErrorInvalidValue;  // the selection below never asks for this
     const uint32_t mtiles = (job.rows + 16u * TMS - 1u) / (16u * TMS);
     const uint32_t ntiles = gemm_ntiles(job, 16u * TNW * WN);
-    launch_kernel((k_gemm_kc<TMS, TNW, WN, KS, G>), dim3(mtiles * ntiles), dim3(64 * WN * KS), 0, stream, job, mtiles,
-                  ntiles, gemm_band(job, mtiles), seq, flag);
-    return hipGetLastError();
+    return launch_tiles(at, k_gemm_kc<TMS, TNW, WN, KS, G>, 64 * WN * KS, job, mtiles, ntiles);
 }
 
 template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_mx(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_mx(const GemmLaunch& at, GemmJob job) {
     const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
-    launch_kernel((k_gemm_mx<TM, TN, WGM, WGN>), dim3(mtiles * ntiles), dim3(64 * WGM * WGN), 0, stream, job,
-                  mtiles, ntiles, gemm_band(job, mtiles), seq, flag);
-    return hipGetLastError();
+    return launch_tiles(at, k_gemm_mx<TM, TN, WGM, WGN>, 64 * WGM * WGN, job, mtiles, ntiles);
 }
 
 template <int MS, int NS, int WM, int WN, int DEPTH>
-hipError_t launch_wv(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_wv(const GemmLaunch& at, GemmJob job) {
     constexpr uint32_t TM = 16u * MS * WM, TN = 16u * NS * WN;
     const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
-    launch_kernel((k_gemm_wv<MS, NS, WM, WN, DEPTH>), dim3(mtiles * ntiles), dim3(64 * WM * WN), 0, stream, job,
-                  mtiles, ntiles, gemm_band(job, mtiles), seq, flag);
-    return hipGetLastError();
+    return launch_tiles(at, k_gemm_wv<MS, NS, WM, WN, DEPTH>, 64 * WM * WN, job, mtiles, ntiles);
 }
 
 template <int TNS, int GB, int WAVES>
-hipError_t launch_dots(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_dots(const GemmLaunch& at, GemmJob job) {
     if (job.groups > 4u * GB || job.mode != MODE_DOT_I16)
         return hipErrorInvalidValue;  // the selection below never asks for this
     const uint32_t mtiles = (job.rows + 15u) / 16u, ntiles = gemm_ntiles(job, 16u * TNS);
-    launch_kernel((k_gemm_dots<TNS, GB, WAVES>), dim3(mtiles * ntiles), dim3(64 * WAVES), 0, stream, job, mtiles, ntiles,
-                  gemm_band(job, mtiles), seq, flag);
-    return hipGetLastError();
+    return launch_tiles(at, k_gemm_dots<TNS, GB, WAVES>, 64 * WAVES, job, mtiles, ntiles);
 }
 
 template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_bits(hipStream_t stream, GemmJob job, uint64_t seq, const uint64_t* flag) {
+hipError_t launch_bits(const GemmLaunch& at, GemmJob job) {
     const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
-    launch_kernel((k_gemm_bits<TM, TN, WGM, WGN>), dim3(mtiles * ntiles), dim3(64 * WGM * WGN), 0, stream, job, mtiles,
-                  ntiles, gemm_band(job, mtiles), seq, flag);
-    return hipGetLastError();
+    return launch_tiles(at, k_gemm_bits<TM, TN, WGM, WGN>, 64 * WGM * WGN, job, mtiles, ntiles);
 }
 
 }  // namespace
@@ -2105,7 +2223,8 @@ hipError_t launch_bits(hipStream_t stream, GemmJob job, uint64_t seq, const uint
 // The largest workgroup tile that still gives every CU a workgroup, else the tile
 // with the most workgroups.
 hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count, uint64_t seq,
-                       const uint64_t* flag) {
+                       const uint64_t* flag, uint32_t* signals) {
+    const GemmLaunch at{stream, seq, flag, signals};
     const uint64_t cus = cu_count ? cu_count : 256u;
     auto blocks = [&](uint32_t tm, uint32_t tn) {
         uint64_t cols = (job.n + tn - 1u) / tn;
@@ -2133,36 +2252,36 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
         // 32-column tiles up to two per CU, and past 16 groups, whose tiles of 64 columns would
         // not fit two workgroups' LDS
         if (job.groups > 16u)
-            return launch_dots<2, 16, 8>(stream, job, seq, flag);
-        return blocks(16, 32) <= 2u * cus ? launch_dots<2, 4, 4>(stream, job, seq, flag)
-                                          : launch_dots<4, 4, 4>(stream, job, seq, flag);
+            return launch_dots<2, 16, 8>(at, job);
+        return blocks(16, 32) <= 2u * cus ? launch_dots<2, 4, 4>(at, job)
+                                          : launch_dots<4, 4, 4>(at, job);
     }
     {
         const uint32_t g = job.groups;
         if (g <= 16u) {
             if (job.rows <= 16u && blocks(16, 32) <= cus)
-                return launch_kr<1, 2, 4, 4>(stream, job, seq, flag);
+                return launch_kr<1, 2, 4, 4>(at, job);
             if (blocks(32, 32) <= cus)
-                return launch_kr<2, 2, 8, 2>(stream, job, seq, flag);
+                return launch_kr<2, 2, 8, 2>(at, job);
             if (blocks(32, 64) <= cus && g > 8u)
-                return launch_kr<2, 4, 16, 1>(stream, job, seq, flag);  // 2048->6144 x 64 rows 6.2 -> 5.7 us
+                return launch_kr<2, 4, 16, 1>(at, job);  // 2048->6144 x 64 rows 6.2 -> 5.7 us
             if (blocks(32, 64) <= cus)
-                return launch_kr<2, 4, 8, 2>(stream, job, seq, flag);
+                return launch_kr<2, 4, 8, 2>(at, job);
             if (g > 8u && blocks(32, 32) <= 9u * cus / 2u)
-                return launch_kr<2, 2, 8, 2>(stream, job, seq, flag);
+                return launch_kr<2, 2, 8, 2>(at, job);
         } else if (g <= 32u) {
             if (blocks(16, 32) <= cus)
-                return launch_kr<1, 2, 8, 4>(stream, job, seq, flag);
+                return launch_kr<1, 2, 8, 4>(at, job);
             if (blocks(32, 32) <= 3u * cus)
-                return launch_kr<2, 2, 8, 4>(stream, job, seq, flag);
+                return launch_kr<2, 2, 8, 4>(at, job);
         } else if (g <= 48u) {
             if (blocks(16, 32) <= cus)
-                return launch_kr<1, 2, 8, 6>(stream, job, seq, flag);
+                return launch_kr<1, 2, 8, 6>(at, job);
             if (blocks(16, 64) <= cus)
-                return launch_kc<1, 1, 4, 2, 48>(stream, job, seq, flag);
+                return launch_kc<1, 1, 4, 2, 48>(at, job);
         } else if (g <= 64u) {
             if (blocks(16, 16) <= cus)
-                return launch_kc<1, 1, 1, 8, 64>(stream, job, seq, flag);
+                return launch_kc<1, 1, 1, 8, 64>(at, job);
         }
     }
     // few rows past the rules above (more than 48 groups and more than a round of 16 x 16
@@ -2171,14 +2290,14 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // rows, and more of them outrun the loads a CU keeps in flight)
     if (job.rows <= 64u && (job.rows <= 32u || job.groups <= 16u) &&
         blocks(16, 16) <= 3u * cus)
-        return launch_wv<1, 1, 1, 1, 8>(stream, job, seq, flag);
+        return launch_wv<1, 1, 1, 1, 8>(at, job);
     // K >= 6144 with between half a round and one round of 32 x 64 tiles: eight waves
     // splitting K per tile (6144->2048 x 256 rows 17.1 us against 19.1 us for a wave per
     // 32 x 32 block, 8192->2048 x 256 21.6 against 23.3, 8192->1024 x 320-512 21.7-22.2
     // against 24.2-28.4; forced-choice sweep, bit-identical outputs; it loses at K = 4096,
     // below half a round and from a second round on)
     if (job.groups >= 48u && blocks(32, 64) > cus / 2u && blocks(32, 64) <= cus)
-        return launch_ks<2, 4, 8, 3>(stream, job, seq, flag);
+        return launch_ks<2, 4, 8, 3>(at, job);
     // K split over four waves per 32 x 64 tile: 17..47 groups with between half a round and
     // one round of tiles (4096->2048 x 192 rows 14.0 us against 15.9 for 32 x 64
     // workgroup tiles, 4096->6144 x 48-64 rows 13.9-14.2 against 15.7-15.9,
@@ -2188,43 +2307,43 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // outputs; at 16 groups and from a third round on the tiled kernels win)
     if (job.groups > 16u && job.groups < 48u && blocks(32, 64) > cus / 2u &&
         blocks(32, 64) <= cus)
-        return launch_ks<2, 4, 4, 3>(stream, job, seq, flag);
+        return launch_ks<2, 4, 4, 3>(at, job);
     if (job.groups >= 48u && blocks(32, 64) > cus && blocks(32, 64) <= 2u * cus)
-        return launch_ks<2, 4, 4, 3>(stream, job, seq, flag);
+        return launch_ks<2, 4, 4, 3>(at, job);
     // a long K (>= 32 groups) with two to three 32 x 32 blocks per CU: a wave per block
     // beats the tiled kernels, whose per-group steps serialise over the long K
     if (job.groups >= 32u && blocks(32, 32) >= 2u * cus && blocks(32, 32) <= 3u * cus)
-        return launch_wv<2, 2, 1, 1, 4>(stream, job, seq, flag);
+        return launch_wv<2, 2, 1, 1, 4>(at, job);
     if (blocks(128, 192) >= cus)
-        return launch_mx<128, 192, 2, 4>(stream, job, seq, flag);
+        return launch_mx<128, 192, 2, 4>(at, job);
     if (blocks(64, 128) >= cus && job.groups >= 32u)
-        return launch_mx<64, 128, 2, 4>(stream, job, seq, flag);
+        return launch_mx<64, 128, 2, 4>(at, job);
     if (BNN_GEMM_CO && blocks(128, 128) >= cus)
-        return launch_co<128, 128, 2, 2>(stream, job, seq, flag);
+        return launch_co<128, 128, 2, 2>(at, job);
     // 128 x 128 tiles also where 64 x 128 ones would need a second round of workgroups
     // (one 8-wave 64 x 128 workgroup per CU fits the registers): 1.26-1.43x measured at
     // 144-192 tiles of 128 x 128
     if (blocks(128, 128) >= cus || blocks(64, 128) > cus)
-        return launch_bits<128, 128, 2, 4>(stream, job, seq, flag);
+        return launch_bits<128, 128, 2, 4>(at, job);
     if (blocks(64, 128) >= cus)
-        return launch_bits<64, 128, 2, 4>(stream, job, seq, flag);
+        return launch_bits<64, 128, 2, 4>(at, job);
     if (blocks(64, 64) >= cus)
-        return launch_bits<64, 64, 2, 2>(stream, job, seq, flag);
+        return launch_bits<64, 64, 2, 2>(at, job);
     const uint64_t enough = cus * 3u / 4u;
     if (blocks(32, 64) < enough && blocks(32, 32) <= cus) {
         // too few tiles for the CUs (jobs of more than 48 groups get here): K split across
         // eight waves of a workgroup with 32 x 32 tiles while those fit one round, else four
         // waves with 32 x 16 tiles
         if (blocks(32, 32) >= enough)
-            return launch_ks<2, 2, 8, 3>(stream, job, seq, flag);
-        return launch_ks<2, 1, 4, 3>(stream, job, seq, flag);
+            return launch_ks<2, 2, 8, 3>(at, job);
+        return launch_ks<2, 1, 4, 3>(at, job);
     }
     // three quarters of a round of 64 x 64 tiles: those beat a round and more of 32 x 64
     // ones (2048->2048 x 384 rows 11.7 us against 12.6, 2048->6144 x 96-128 rows 11.6-11.7
     // against 12.0-12.4)
     if (blocks(64, 64) >= enough)
-        return launch_bits<64, 64, 2, 2>(stream, job, seq, flag);
-    return launch_bits<32, 64, 2, 2>(stream, job, seq, flag);
+        return launch_bits<64, 64, 2, 2>(at, job);
+    return launch_bits<32, 64, 2, 2>(at, job);
 }
 
 }  // namespace bnnhip

@@ -93,16 +93,18 @@ struct DotJob {
 // others, whose column tiles follow the first's; column tile t of the launch belongs to the
 // last part with first <= t (first is set by the launcher, in column tiles of the kernel it
 // picks).
+// The arguments of a launch are written for each one, so a part holds no more than it must
+// (sixteen fields more in the arguments cost a call ~0.3 us): the scales lie behind the
+// matrix's bits, the tiles follow from n.
 struct GemmPart {
     const uint4* wbits;
-    const uint16_t* wscale;
     const int8_t* q;
     const float* rscale;
     unsigned char* out;
     uint64_t out_stride;
-    uint32_t n, tiles, first, pad_;
+    uint32_t n, first;
 };
-constexpr uint32_t kGemmParts = 8;
+constexpr uint32_t kGemmParts = 4;
 struct GemmJob {
     const uint4* wbits;       // matrix layout [tiles][groups][64] x 16 bytes
     const uint16_t* wscale;   // matrix layout [tiles][groups][64]
@@ -114,12 +116,16 @@ struct GemmJob {
     uint32_t rows;
     int32_t mode;
     uint32_t extra, pad_;          // parts in use
+    uint64_t* done;  // a launch whose caller waits for it: pinned host words, one per workgroup, that receive seq
     GemmPart parts[kGemmParts - 1];
 };
 
-// Rows from which a job runs on the matrix cores instead of the bit-plane kernel.
+// Rows from which a job of BNN_Execute that is not one fused launch runs on the matrix cores
+// instead of the bit-plane kernels: all of them (a call of 2048->6144 x 2 rows 19.3 us with
+// dots, 15.7 on the matrix cores with their own completion words; 6144->2048 x 2 rows 25.4 and
+// 18.3).
 #ifndef BNN_MFMA_MIN_ROWS
-#define BNN_MFMA_MIN_ROWS 8
+#define BNN_MFMA_MIN_ROWS 1
 #endif
 constexpr uint32_t kMfmaMinRows = BNN_MFMA_MIN_ROWS;
 
@@ -176,9 +182,10 @@ struct FusedArgs {
 
 // Pinned host words of a device (bnn_accel_device::status_host): [0] seq of the last
 // synchronous call that met an illegal input, [1] the same for asynchronous launches,
-// then from kDoneFlagWord one completion word per workgroup of a single-row launch.
+// then from kDoneFlagWord one completion word per workgroup of a launch that signals.
 constexpr uint32_t kDoneFlagWord = 32;     // 256 bytes in
-constexpr uint32_t kDoneFlagSlots = 1024;  // workgroups a single-row launch may signal with
+constexpr uint32_t kDoneFlagSlots = 1024;  // workgroups a launch may signal with
+constexpr uint32_t kDoneWords = 256;       // workgroups of a matrix-core launch that signals (one per CU)
 constexpr size_t kStatusHostBytes = (kDoneFlagWord + kDoneFlagSlots) * sizeof(uint64_t);
 
 // Kernel timing: when `start` is set, the next kernel launched through launch_kernel
@@ -221,8 +228,10 @@ hipError_t launch_prep_batch(hipStream_t stream, const PrepJob* jobs, const uint
 hipError_t launch_dot_batch(hipStream_t stream, const DotJob* jobs, const uint32_t* item_job, uint32_t items,
                             uint32_t uniform_items, uint32_t max_groups, bool scales, uint32_t cu_count,
                             uint64_t seq, const uint64_t* flag);
+// With job.done set, *signals receives the number of workgroups that signal, 0 when the
+// launch has too many for that.
 hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count, uint64_t seq,
-                       const uint64_t* flag);
+                       const uint64_t* flag, uint32_t* signals = nullptr);
 // One launch of a fused batch of `tiles` 64-feature tiles on `grid` workgroups
 // (bnn_fused.hip).
 hipError_t launch_fused(hipStream_t stream, const FusedArgs& args, uint32_t tiles, uint32_t grid, uint64_t seq,

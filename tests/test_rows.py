@@ -164,11 +164,11 @@ def test_prompt_block_error_then_prompt(pkg, hip, tmp_path):
         m.free()
 
 
-# Batches whose multi-row jobs run on the matrix cores: groups of up to eight alike jobs (one k,
+# Batches whose multi-row jobs run on the matrix cores: groups of up to four alike jobs (one k,
 # rows and operation), shared and own input views, beside jobs that stay with the dots.
 @pytest.mark.parametrize("specs,shared", [
     ([("GEMM_F32", 2048, 2048, 48), ("GEMM_F32", 2048, 1024, 48), ("GEMM_F32", 2048, 1030, 48)], True),
-    ([("GEMM_F32", 2048, 2048, 64)] * 9, False),                        # a second group of one
+    ([("GEMM_F32", 2048, 2048, 64)] * 9, False),                        # groups of four, four and one
     ([("GEMM_F32", 256, 70, 4)], False),                                # a small group alone
     ([("GEMM_F32", 256, 70, 4), ("GEMM", 256, 70, 4)], False),          # two small groups: the dots
     ([("GEMM_F32", 4096, 3000, 17), ("GEMV_F32", 512, 100, 1), ("GEMM", 4096, 200, 17),
