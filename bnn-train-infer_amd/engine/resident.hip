@@ -1137,6 +1137,8 @@ __global__ __launch_bounds__(256) void k_silu_mul(float* __restrict__ gate, cons
 
 }  // namespace
 
+constexpr uint32_t kMaxOutgrown = 8;
+
 struct Resident {
     BNN_Device dev;
     hipStream_t stream;
@@ -1176,6 +1178,8 @@ struct Resident {
     float *block_out, *block_in, *block_x;
     float* block_scores;
     size_t block_score_floats;
+    BNN_Buffer outgrown[kMaxOutgrown];  // smaller block buffers, given back with the context
+    uint32_t outgrown_count;
     const SignLinear** lin;  // [7 * L + 1]: per layer q, k, v, o, gate, up, down; then lm_head
     uint64_t jobs_per_token, macs_per_token, lm_jobs, lm_macs;
 };
@@ -1546,6 +1550,8 @@ void resident_free(Resident* r) {
     for (BNN_Buffer b : {r->b_norm, r->b_q, r->b_k, r->b_v, r->b_y, r->b_o, r->b_gate, r->b_up, r->b_h, r->b_logits,
                          r->b_block_out, r->b_block_in})
         BNN_BufferFree(b);
+    for (uint32_t i = 0; i < r->outgrown_count; ++i)
+        BNN_BufferFree(r->outgrown[i]);
     for (void* p : {(void*)r->x, (void*)r->x2, (void*)r->kc, (void*)r->vc, (void*)r->scores, (void*)r->gains, (void*)r->rope_cos,
                     (void*)r->rope_sin, (void*)r->emb_bits, (void*)r->emb_scales, (void*)r->err, (void*)r->keys,
                     (void*)r->block_x, (void*)r->block_scores})
@@ -1670,6 +1676,8 @@ BNNE_Status step_error(Resident* r, int err) {
 // operations in its own step's order, so the cache rows and the logits are the same bits.
 constexpr uint32_t kBlockMinTokens = 3;             // two tokens: 2.1 ms as a block, 2.0 ms one after the other
 constexpr uint32_t kBlockRows = 1024;               // most tokens of a block
+constexpr uint32_t kBlockFirstRows = 64;            // tokens that the first block memory holds, at least
+static_assert(kBlockRows <= (kBlockFirstRows << (kMaxOutgrown / 2u)), "every doubling's two buffers are kept");
 constexpr size_t kBlockScoreFloats = 128u << 20;    // most scores of a block (512 MB)
 
 // Where the parts of a block live, in floats.
@@ -1692,36 +1700,35 @@ uint32_t block_rows_for(const Resident* r, uint32_t n, uint32_t pos0) {
     return n <= rows ? n : (uint32_t)(rows >= 64u ? rows & ~(size_t)63u : rows);
 }
 
-void release_block(Resident* r) {
-    (void)hipStreamSynchronize(r->stream);
-    BNN_BufferFree(r->b_block_out);
-    BNN_BufferFree(r->b_block_in);
-    if (r->block_x)
-        (void)hipFree(r->block_x);
-    r->b_block_out = r->b_block_in = nullptr;
-    r->block_x = nullptr;
-    r->block_rows = 0;
-}
-
-// Memory for blocks of `rows` tokens and `scores` scores; grown by doubling, since giving
-// buffers back makes every prepared batch of the device stale.
+// Memory for blocks of `rows` tokens and `scores` scores.  Rows grow by doubling from
+// kBlockFirstRows, and outgrown buffers stay with the context: giving a buffer back makes every
+// prepared batch of the device stale, a caller's own ones too.
 BNNE_Status ready_block(Resident* r, uint32_t rows, size_t scores) {
     BNNE_Status st = BNNE_OK;
     if (rows > r->block_rows) {
-        rows = std::min(std::max(rows, 2u * r->block_rows), kBlockRows);
-        if (r->block_rows)
-            release_block(r);
+        rows = std::min(std::max({rows, 2u * r->block_rows, kBlockFirstRows}), kBlockRows);
         const BlockLayout at(r, rows);
-        st = alloc_buffer(r, at.out_floats, &r->b_block_out, &r->block_out);
+        BNN_Buffer b_out = nullptr, b_in = nullptr;
+        float *out = nullptr, *in = nullptr, *x = nullptr;
+        st = alloc_buffer(r, at.out_floats, &b_out, &out);
         if (st == BNNE_OK)
-            st = alloc_buffer(r, at.in_floats, &r->b_block_in, &r->block_in);
+            st = alloc_buffer(r, at.in_floats, &b_in, &in);
         if (st == BNNE_OK)
-            st = upload(&r->block_x, nullptr, 2u * (size_t)rows * r->C * sizeof(float));
+            st = upload(&x, nullptr, 2u * (size_t)rows * r->C * sizeof(float));
         if (st != BNNE_OK) {
-            r->block_x = nullptr;
-            release_block(r);
+            BNN_BufferFree(b_out);
+            BNN_BufferFree(b_in);
             return st;
         }
+        if (r->block_rows) {
+            (void)hipStreamSynchronize(r->stream);
+            (void)hipFree(r->block_x);
+            r->outgrown[r->outgrown_count++] = r->b_block_out;
+            r->outgrown[r->outgrown_count++] = r->b_block_in;
+        }
+        r->b_block_out = b_out, r->block_out = out;
+        r->b_block_in = b_in, r->block_in = in;
+        r->block_x = x;
         r->block_rows = rows;
     }
     if (scores > r->block_score_floats) {
@@ -1847,7 +1854,7 @@ BNNE_Status enqueue_blocks(Resident* r, const int32_t* tokens, uint32_t n, uint3
     const size_t pitch = ((size_t)pos0 + n + 63u) & ~(size_t)63u;
     BNNE_Status st = ready_block(r, rows, pitch * r->H * rows);
     if (st == BNNE_OK)
-        st = ready_batches(r);  // growing the block frees buffers, which makes batches stale
+        st = ready_batches(r);  // a failed growth frees buffers, which makes batches stale
     if (st != BNNE_OK)
         return st;
     std::memcpy(r->pinned_tokens, tokens, (size_t)n * sizeof(int32_t));

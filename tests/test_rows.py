@@ -164,6 +164,34 @@ def test_prompt_block_error_then_prompt(pkg, hip, tmp_path):
         m.free()
 
 
+def test_growing_block_keeps_batches(pkg, hip, tmp_path):
+    """Longer and longer prompts grow the context's block memory; a program's own prepared batch
+    on the same device stays valid."""
+    path = tmp_path / "m.gguf"
+    pkg.gguf.qwen3_random(path, **TINY)
+    bits, scales = pkg.synth.matrix(70, 256, seed=2)
+    with pkg.Device(hip, 0) as dev:
+        m = pkg.engine.Model(_engine_lib(pkg), dev, path)
+        c = pkg.engine.Context(m, n_ctx=TINY["context"])
+        mat, bi, bo = dev.matrix(bits, scales), dev.buffer(4 * 256), dev.buffer(4 * 70)
+        bi.write(np.ones(256, np.float32))
+        T = pkg.Type.F32
+        jobs = (pkg.Job * 1)(pkg.Job(int(pkg.Op.GEMV_F32), mat.handle.value, bi.view(T), bo.view(T), 1))
+        batch = ctypes.c_void_p()
+        assert dev.api.BNNX_BatchCreate(dev.handle, jobs, 1, ctypes.byref(batch)) == pkg.Status.OK
+        for count in (5, 65, 130, 600, 1100):
+            print(f"prompt of {count} tokens", flush=True)
+            c.decode(np.arange(count, dtype=np.int32) % TINY["vocab"], want_logits=False)
+            assert dev.api.BNNX_BatchLaunch(batch) == pkg.Status.OK
+        assert dev.api.BNNX_DeviceSynchronize(dev.handle) == pkg.Status.OK
+        dev.api.BNNX_BatchDestroy(batch)
+        c.free()
+        m.free()
+        mat.destroy()
+        bi.free()
+        bo.free()
+
+
 # Batches whose multi-row jobs run on the matrix cores: groups of up to four alike jobs (one k,
 # rows and operation), shared and own input views, beside jobs that stay with the dots.
 @pytest.mark.parametrize("specs,shared", [
