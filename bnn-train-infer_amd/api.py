@@ -194,6 +194,7 @@ class Api:
             "BNNX_BatchCreateFused": (S, [V, P(Job), U32, P(PreOp), P(V)]),
             "BNNX_BatchCreateFusedPost": (S, [V, P(Job), U32, P(PreOp), P(PostOp), P(V)]),
             "BNNX_BatchCreateChain": (S, [V, P(ChainLayer), U32, BufferView, BufferView, U32, P(V)]),
+            "BNNX_ChainRunHost": (S, [V, V, V]),
             "BNNX_LaunchRows": (S, [V, P(Job), U32, P(PreOp)]),
             "BNNX_BatchLaunch": (S, [V]),
             "BNNX_BatchCheck": (S, [V]),

@@ -1899,9 +1899,34 @@ EXPORT BNN_Status BNNX_BatchCreateChain(BNN_Device device, const BNNX_ChainLayer
     args.rows = rows;
     args.k0 = layers[0].matrix->k;
     b->chain_args = args;
+    b->chain_out = layers[count - 1].matrix->n;
     device->live_batches++;
     *out_batch = b;
     return BNN_OK;
+}
+
+EXPORT BNN_Status BNNX_ChainRunHost(BNNX_Batch batch, const float* input, float* output) {
+    const BNN_Status st = BNNX_BatchCheck(batch);
+    if (st != BNN_OK)
+        return st;
+    if (!batch->chain || input == nullptr || output == nullptr || (((uintptr_t)input | (uintptr_t)output) & 3u) != 0)
+        return BNN_EINVAL;
+    BNN_Device device = batch->device;
+    // an outstanding asynchronous launch's report belongs to BNNX_DeviceSynchronize
+    if (batch->chain_args.rows > kDoneFlagSlots || device->timing || device->async_first_seq != 0)
+        return BNN_ENOTSUP;
+    device->mirror_buf = nullptr;
+    if (hipSetDevice(device->ordinal) != hipSuccess)
+        return BNN_EIO;
+    ChainArgs args = batch->chain_args;
+    args.in = reinterpret_cast<const unsigned char*>(input);
+    args.in_stride = (uint64_t)args.k0 * 4u;
+    args.out = reinterpret_cast<unsigned char*>(output);
+    args.out_stride = (uint64_t)batch->chain_out * 4u;
+    args.done = device->status_host + kDoneFlagWord;
+    const uint64_t seq = ++device->seq;
+    const hipError_t e = launch_chain(device->stream, args, seq, device->flag_dev, device->status_host);
+    return finish_signalled(device, e, seq, args.rows);
 }
 
 EXPORT BNN_Status BNNX_BufferDevicePointer(BNN_Buffer buffer, void** out_pointer) {

@@ -277,6 +277,9 @@ struct ChainArgs {
     uint64_t in_stride;
     unsigned char* out;        // row 0 of the output view (F32, 4-byte aligned)
     uint64_t out_stride;
+    // rows in host memory: workgroup r writes its results through and stores seq into the
+    // pinned host word done[r] once they are complete (may be null)
+    uint64_t* done;
 };
 // One launch of a chained batch: a workgroup per row (bnn_chain.hip).
 hipError_t launch_chain(hipStream_t stream, const ChainArgs& args, uint64_t seq, uint64_t* flag,
@@ -372,6 +375,7 @@ struct bnnx_batch {
     // chained batch (BNNX_BatchCreateChain): one launch of a workgroup per row
     bool chain;
     bnnhip::ChainArgs chain_args;  // layers points into mem
+    uint32_t chain_out;            // the last layer's outputs
 };
 
 struct bnn_accel_buffer {

@@ -225,6 +225,32 @@ BNNE_Status mlp_device_create(bnne_context* c, const MlpDeviceBlock* blocks, uin
     return BNNE_OK;
 }
 
+// A chunk's launches on the copied rows and the copy of the logits, without the wait.
+static BNNE_Status mlp_device_enqueue(MlpDevice* d, const MlpDevice::Plan& plan, uint32_t rows) {
+    BNNE_Status st = BNNE_OK;
+    if (plan.chain)
+        st = accel_status(BNNX_BatchLaunch(plan.batches[0]), "BNNX_BatchLaunch");
+    for (size_t i = 0; i < d->blocks.size() && st == BNNE_OK && !plan.chain; ++i) {
+        const MlpDevice::Block& b = d->blocks[i];
+        st = accel_status(BNNX_BatchLaunch(plan.batches[i]), "BNNX_BatchLaunch");
+        if (st != BNNE_OK)
+            break;
+        const uint32_t n = rows * b.out;
+        hipLaunchKernelGGL(k_mlp_post, dim3((n + 255u) / 256u), dim3(256), 0, d->stream, d->output_ptr(i), n, b.out,
+                           b.scale, b.scale + b.out, b.relu ? 1 : 0);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            st = hip_failure(e, "post-operation launch");
+    }
+    if (st == BNNE_OK) {
+        const size_t out_bytes = (size_t)rows * d->classes * sizeof(float);
+        const hipError_t e = hipMemcpyAsync(d->pinned_out, d->out, out_bytes, hipMemcpyDeviceToHost, d->stream);
+        if (e != hipSuccess)
+            st = hip_failure(e, "logits to the host");
+    }
+    return st;
+}
+
 BNNE_Status mlp_device_classify(bnne_context* c, MlpDevice* d, const float* input, uint32_t rows, float* logits) {
     if (rows == 0 || rows > d->rows)
         return complain(BNNE_EINVAL, "%u rows at once; the device path stages %u", rows, d->rows);
@@ -265,30 +291,23 @@ BNNE_Status mlp_device_classify(bnne_context* c, MlpDevice* d, const float* inpu
     const size_t out_bytes = (size_t)rows * d->classes * sizeof(float);
     const uint64_t t0 = stats ? clock_ns() : 0;
     std::memcpy(d->pinned_in, input, in_bytes);
-    e = hipMemcpyAsync(d->in, d->pinned_in, in_bytes, hipMemcpyHostToDevice, d->stream);
-    BNNE_Status st = e == hipSuccess ? BNNE_OK : hip_failure(e, "input rows to the device");
-    const uint64_t t_in = stats ? clock_ns() : 0;
-    if (st == BNNE_OK && plan.chain)
-        st = accel_status(BNNX_BatchLaunch(plan.batches[0]), "BNNX_BatchLaunch");
-    for (size_t i = 0; i < d->blocks.size() && st == BNNE_OK && !plan.chain; ++i) {
-        const MlpDevice::Block& b = d->blocks[i];
-        st = accel_status(BNNX_BatchLaunch(plan.batches[i]), "BNNX_BatchLaunch");
-        if (st != BNNE_OK)
-            break;
-        const uint32_t n = rows * b.out;
-        hipLaunchKernelGGL(k_mlp_post, dim3((n + 255u) / 256u), dim3(256), 0, d->stream, d->output_ptr(i), n, b.out,
-                           b.scale, b.scale + b.out, b.relu ? 1 : 0);
-        e = hipGetLastError();
+    BNN_Status sync = BNN_ENOTSUP;
+    BNNE_Status st = BNNE_OK;
+    uint64_t t_in = stats ? clock_ns() : 0, t1 = t_in;
+    // a chain reads the staged rows and writes the logits itself: one launch, and the end
+    // signalled by its workgroups, against a copy, a launch, a copy and a stream wait
+    if (plan.chain)
+        sync = BNNX_ChainRunHost(plan.batches[0], d->pinned_in, d->pinned_out);
+    if (sync == BNN_ENOTSUP) {
+        e = hipMemcpyAsync(d->in, d->pinned_in, in_bytes, hipMemcpyHostToDevice, d->stream);
         if (e != hipSuccess)
-            st = hip_failure(e, "post-operation launch");
+            st = hip_failure(e, "input rows to the device");
+        t_in = stats ? clock_ns() : 0;
+        if (st == BNNE_OK)
+            st = mlp_device_enqueue(d, plan, rows);
+        t1 = stats ? clock_ns() : 0;
+        sync = BNNX_DeviceSynchronize(d->dev);
     }
-    if (st == BNNE_OK) {
-        e = hipMemcpyAsync(d->pinned_out, d->out, out_bytes, hipMemcpyDeviceToHost, d->stream);
-        if (e != hipSuccess)
-            st = hip_failure(e, "logits to the host");
-    }
-    const uint64_t t1 = stats ? clock_ns() : 0;
-    const BNN_Status sync = BNNX_DeviceSynchronize(d->dev);
     const uint64_t t2 = stats ? clock_ns() : 0;
     if (st != BNNE_OK)
         return st;

@@ -207,6 +207,17 @@ BNN_Status BNNX_BatchCreateChain(BNN_Device device, const BNNX_ChainLayer* layer
                                  BNN_BufferView input, BNN_BufferView output, uint32_t rows,
                                  BNNX_Batch* out_batch);
 
+/* Runs a chained batch on rows in host memory and waits for it: the batch's rows are read
+ * from `input` (rows x K_0 floats) and the last layer's results written to `output` (rows x
+ * N_last floats), both tight, in page-locked memory that the device addresses as the host
+ * does (hipHostMalloc), in place of the batch's views.  The kernel reads and writes that
+ * memory itself and signals its end, so the call is one launch with no copies.  BNN_OK, or
+ * BNN_ERANGE when a row met a non-finite value (`output` is then unspecified);
+ * BNN_EINVAL for a batch that is not chained, is stale, or NULL or misaligned addresses;
+ * BNN_ENOTSUP, with nothing enqueued, for batches of more than 1024 rows, with kernel timing
+ * on, or while launches of the device wait for a BNNX_DeviceSynchronize. */
+BNN_Status BNNX_ChainRunHost(BNNX_Batch batch, const float* input, float* output);
+
 /* Device address of a buffer's memory, for kernels a caller runs on the device's
  * stream between batch launches.  Valid until BNN_BufferFree. */
 BNN_Status BNNX_BufferDevicePointer(BNN_Buffer buffer, void** out_pointer);

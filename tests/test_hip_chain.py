@@ -209,3 +209,52 @@ def test_chain_argument_checks(pkg, hipdev):
     m_other.destroy()
     m_wide.destroy()
     c.free()
+
+
+class PinnedRows:
+    """A page-locked F32 array [rows][width] that the device addresses."""
+
+    def __init__(self, dev, rows, width):
+        self.hip = dev.api.lib  # resolves its HIP runtime's symbols too
+        self.ptr = ctypes.c_void_p()
+        assert self.hip.hipHostMalloc(ctypes.byref(self.ptr), ctypes.c_size_t(4 * rows * width), 0) == 0
+        buf = (ctypes.c_float * (rows * width)).from_address(self.ptr.value)
+        self.array = np.frombuffer(buf, np.float32).reshape(rows, width)
+
+    def free(self):
+        assert self.hip.hipHostFree(self.ptr) == 0
+
+
+@pytest.mark.parametrize("dims,rows", [([128, 64], 1), ([896, 512, 512, 10], 64), ([4096, 200], 3),
+                                       ([256, 70], 256), ([128, 33], 1024)])
+def test_chain_on_host_rows(pkg, hipdev, oracle_fast, dims, rows):
+    """The kernel reads and writes page-locked host rows itself; new rows on every call."""
+    c = Chain(pkg, hipdev, dims, [(1, 1)] * (len(dims) - 2) + [(1, 0)], rows, seed=rows)
+    st, b = c.create()
+    assert st == pkg.Status.OK
+    run = hipdev.api.BNNX_ChainRunHost
+    px, py = PinnedRows(hipdev, rows, dims[0]), PinnedRows(hipdev, rows, dims[-1])
+    tx, ty = px.array, py.array
+    print(f"host rows {rows} x {dims}", flush=True)
+    for seed in range(3):
+        x = pkg.synth.normal_f32(rows, dims[0], seed=seed + 1)
+        tx[:] = x
+        assert run(b, px.ptr, py.ptr) == pkg.Status.OK
+        assert np.array_equal(ty.view(np.uint32), c.expected(oracle_fast, x).view(np.uint32))
+    tx[rows - 1, 5] = float("nan")
+    assert run(b, px.ptr, py.ptr) == pkg.Status.ERANGE
+    tx[rows - 1, 5] = 1.0
+    assert run(b, px.ptr, py.ptr) == pkg.Status.OK
+    # a launch that waits for its synchronisation keeps its report
+    c.write_input(tx)
+    assert hipdev.api.BNNX_BatchLaunch(b) == pkg.Status.OK
+    assert run(b, px.ptr, py.ptr) == pkg.Status.ENOTSUP
+    assert hipdev.api.BNNX_DeviceSynchronize(hipdev.handle) == pkg.Status.OK
+    assert run(b, px.ptr, py.ptr) == pkg.Status.OK
+    assert np.array_equal(c.output().view(np.uint32), ty.view(np.uint32))
+    assert run(b, None, py.ptr) == pkg.Status.EINVAL
+    assert run(b, px.ptr.value + 2, py.ptr) == pkg.Status.EINVAL
+    hipdev.api.BNNX_BatchDestroy(b)
+    px.free()
+    py.free()
+    c.free()

@@ -111,6 +111,33 @@ def test_launch_rows_illegal_row(pkg, hipdev, kind):
         f.free()
 
 
+@pytest.mark.parametrize("k", [128, 384, 640, 2048, 2176, 4096, 8192])
+def test_launch_rows_sum_of_squares(pkg, hipdev, oracle, k):
+    """RMSNorm rows whose running sums leave the speculative windows: the sequential loop's bits."""
+    f = Rows(pkg, hipdev, k, [65], 6, PreOp.RMSNORM, False)
+    try:
+        ramp = np.exp2(np.linspace(-60, 40, k)).astype(np.float32)
+        f.a[0] = 1.1
+        f.a[1], f.a[2] = ramp, ramp[::-1]
+        f.a[3] = 0
+        f.a[3, k - 1] = 3
+        f.a[4] = np.where(np.arange(k) % 2, np.float32(1e-20), np.float32(777.7))
+        f.a[5] = np.float32(1e-22)
+        f.a[5, k // 2] = 1
+        f.write()
+        print(f"sum of squares, {k}", flush=True)
+        assert f.launch() == (0, 0)
+        x = np.stack([f.row(r) for r in range(6)])
+        with pkg.Device(oracle, 0) as ref:
+            m = ref.matrix(*f.chunks[0])
+            want = ref.run(pkg.Op.GEMM_F32, m, x)
+            m.destroy()
+        got = f.outs[0].read().view(np.float32).reshape(want.shape)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), first_mismatch(got, want)
+    finally:
+        f.free()
+
+
 TINY = {"layers": 2, "hidden": 256, "heads": 2, "kv_heads": 1, "ffn": 512, "vocab": 512, "context": 4352}
 
 
