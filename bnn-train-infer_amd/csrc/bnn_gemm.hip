@@ -1,7 +1,7 @@
 // Multi-row jobs (GEMM, GEMM_F32, DOT_GROUPS with rows >= kMfmaMinRows) on the
 // gfx950 matrix cores (v_mfma_i32_16x16x64_i8), fed from the matrix's resident
-// 1.125-bit layout: the sign bits of each 128-weight group are unpacked to +1/-1
-// bytes in LDS, per workgroup tile and group, two groups before the MFMAs use them.
+// 1.125-bit layout: a byte table in LDS turns the sign bits of each 128-weight group into
+// the MFMAs' +1/-1 operands.
 //
 // Numeric contract (reference bnn-accelerator.h:133-149, soft-bnn-accelerator.c:219-276),
 // per 128-weight group g:
@@ -17,25 +17,6 @@
 //     where the reference may form -0; the accumulator starts at +0 and never
 //     becomes -0 (x + -x == +0 in round-to-nearest), so the sums agree bit for bit.
 // DOT_GROUPS stores D itself as int16 (k_gemm_dots).
-//
-// k_gemm_bits<TM, TN, WGM, WGN>: workgroup tile TM x TN, WGM x WGN waves of
-// (TM/WGM) x (TN/WGN).  Everything a group needs reaches LDS by DMA
-// (global_load_lds, 16 bytes per lane, no registers): the TM rows' 128 quantised
-// bytes, the TN features' 16-byte sign-bit chunks (1 KiB per 64-feature tile of the
-// matrix layout) and their column scales.  One barrier per group; iteration g:
-//   * issue the DMAs of group g+3's rows, group g+5's bits and group g+2's scales
-//     (each has two iterations to land);
-//   * look up group g+2's bits (read into registers one iteration ago) in a
-//     256-entry table (2 KiB, built at start): one 8-byte lookup turns a byte of
-//     bits into 8 bytes of +1/-1;
-//   * read group g+3's bits, and group g+1's MFMA operands into the second
-//     register set (the loop is unrolled by two, so the two sets alternate without
-//     copies);
-//   * group g's first-half MFMAs (operands read one iteration ago), each subtile
-//     interleaved with group g-1's epilogue on it;
-//   * store group g+2's +1/-1 tile; group g's second-half MFMAs.
-// At the end every wave writes its accumulators into LDS and the workgroup stores
-// the tile row by row, 16 bytes per lane.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -214,594 +195,6 @@ __device__ __forceinline__ void barrier() {
     asm volatile("" ::: "memory");  // no LDS access moves across it
 }
 
-template <int TM, int TN, int WGM, int WGN, int ASLOTS = 4>
-struct Tiling {
-    static constexpr int WAVES = WGM * WGN, THREADS = 64 * WAVES;
-    static constexpr int WTM = TM / WGM, WTN = TN / WGN, MS = WTM / 16, NS = WTN / 16;
-    // DMA work per wave and group: every wave issues exactly A_INS + 2 DMAs, each
-    // with at least one active lane, so that the vmcnt bookkeeping is uniform
-    static constexpr uint32_t A_CHUNKS = TM * 8 / WAVES;  // 16-byte row chunks
-    static constexpr uint32_t A_INS = A_CHUNKS >= 64 ? A_CHUNKS / 64 : 1;
-    static constexpr uint32_t A_LANES = A_CHUNKS >= 64 ? 64 : A_CHUNKS;
-    static constexpr uint32_t BIT_LANES = TN / WAVES;     // one 16-byte chunk per feature
-    static constexpr uint32_t SC_CHUNKS = TN / 8;         // 8 fp16 scales per chunk
-    static constexpr uint32_t SC_CPW = SC_CHUNKS >= (uint32_t)WAVES ? SC_CHUNKS / WAVES : 1;
-    // LDS carve-up (bytes)
-    static constexpr uint32_t A_SLOT = TM * 128, B_SLOT = TN * 128, BITS_SLOT = TN * 16, SC_SLOT = TN * 2;
-    static constexpr uint32_t OFF_B = ASLOTS * A_SLOT, OFF_BITS = OFF_B + 2 * B_SLOT, OFF_SC = OFF_BITS + 4 * BITS_SLOT,
-                              OFF_LUT = (OFF_SC + 4 * SC_SLOT + 15u) & ~15u, LOOP_BYTES = OFF_LUT + 2048;
-    static constexpr uint32_t OUT_STRIDE = TN + 16;  // floats per staged output row
-    static constexpr uint32_t OUT_BYTES = TM * OUT_STRIDE * 4;
-    static constexpr uint32_t SMEM = LOOP_BYTES > OUT_BYTES ? LOOP_BYTES : OUT_BYTES;
-    static_assert(TM % (16 * WGM) == 0 && TN % (16 * WGN) == 0, "wave tiles of 16 x 16 subtiles");
-    static_assert(A_CHUNKS % 64 == 0 || A_CHUNKS < 64, "row DMA split");
-    static_assert(TN % WAVES == 0 && BIT_LANES <= 64, "bits DMA split");
-    static_assert(SC_CHUNKS < (uint32_t)WAVES || SC_CHUNKS % WAVES == 0, "scales DMA split");
-    static_assert(SMEM <= 160 * 1024, "LDS");
-    static_assert(TM * TN / 4 % THREADS == 0, "output chunks per thread");
-};
-
-template <int TM, int TN, int WGM, int WGN>
-__global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bits(GemmJob j, uint32_t mtiles, uint32_t ntiles, uint32_t band,
-                                                              uint64_t seq, const uint64_t* __restrict__ flag) {
-    using T = Tiling<TM, TN, WGM, WGN>;
-    constexpr int MS = T::MS, NS = T::NS, THREADS = T::THREADS;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[T::SMEM];
-    if (*flag == seq) {
-        gemm_signal(j, seq);
-        return;
-    }
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave / WGN, wn = wave % WGN;
-    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
-    tile.nt = select_part(j, tile.nt);
-    const uint32_t mt = tile.mt, nt = tile.nt;
-    const uint32_t m0 = mt * TM, n0 = nt * TN;
-    const uint32_t groups = j.groups;
-    unsigned char* const lds_a = smem;
-    unsigned char* const lds_b = smem + T::OFF_B;
-    unsigned char* const lds_bits = smem + T::OFF_BITS;
-    unsigned char* const lds_sc = smem + T::OFF_SC;
-    uint2* const lut = reinterpret_cast<uint2*>(smem + T::OFF_LUT);
-
-    // byte b of sign bits -> 8 bytes of +1/-1 (bit i -> byte i)
-    if (tid < 256u)
-        lut[tid] = make_uint2(pm1_nibble(tid & 15u), pm1_nibble(tid >> 4));
-
-    // this lane's DMA sources (without the group offset)
-    const uint8_t* a_src[T::A_INS];
-#pragma unroll
-    for (uint32_t i = 0; i < T::A_INS; ++i) {
-        const uint32_t p = wave * T::A_CHUNKS + i * 64u + lane, r = p >> 3;
-        const uint32_t c = (p & 7u) ^ ((r >> 1) & 7u);
-        a_src[i] = reinterpret_cast<const uint8_t*>(j.q) + (size_t)min(m0 + min(r, TM - 1u), j.rows - 1u) * j.k +
-                   16u * c;
-    }
-    // bits: feature f of the tile; its 64-feature matrix tile is clamped into the
-    // array (features past the last tile are never stored)
-    const uint32_t f = T::BIT_LANES * wave + min(lane, T::BIT_LANES - 1u);
-    const uint8_t* bit_src = reinterpret_cast<const uint8_t*>(j.wbits) +
-                             ((size_t)min((n0 + f) >> 6, j.tiles - 1u) * groups * kTile + ((n0 + f) & 63u)) * 16u;
-    // scales: chunks of 8 columns, SC_CPW consecutive ones per wave (with fewer
-    // chunks than waves, the waves past the last chunk repeat one, writing the same
-    // bytes)
-    const uint32_t sc_first = (wave * T::SC_CPW) % T::SC_CHUNKS;
-    const uint32_t sc_col = n0 + 8u * (sc_first + min(lane, T::SC_CPW - 1u));
-    const uint8_t* sc_src = reinterpret_cast<const uint8_t*>(j.wscale) +
-                            ((size_t)min(sc_col >> 6, j.tiles - 1u) * groups * kTile + (sc_col & 63u)) * 2u;
-    const uint32_t la0 = lds_offset(lds_a), lbits0 = lds_offset(lds_bits), lsc0 = lds_offset(lds_sc);
-    const size_t bit_step = (size_t)kTile * 16u, sc_step = (size_t)kTile * 2u;  // bytes per group
-    auto issue_rows = [&](uint32_t g) {
-        const uint32_t gg = min(g, groups - 1u);
-#pragma unroll
-        for (uint32_t i = 0; i < T::A_INS; ++i)
-            dma16_lanes<lane_mask<T::A_LANES>()>(a_src[i] + (size_t)gg * kGroup,
-                                                 la0 + (g & 3u) * T::A_SLOT + (wave * T::A_CHUNKS + i * 64u) * 16u);
-    };
-    auto issue_bits = [&](uint32_t g) {
-        const uint32_t gg = min(g, groups - 1u);
-        dma16_lanes<lane_mask<T::BIT_LANES>()>(bit_src + gg * bit_step,
-                                               lbits0 + (g & 3u) * T::BITS_SLOT + wave * (T::BIT_LANES * 16u));
-    };
-    auto issue_scales = [&](uint32_t g) {
-        const uint32_t gg = min(g, groups - 1u);
-        dma16_lanes<lane_mask<T::SC_CPW>()>(sc_src + gg * sc_step, lsc0 + (g & 3u) * T::SC_SLOT + 16u * sc_first);
-    };
-    // unpacks group g's bits (slot g % 4) into the +1/-1 tile lds_b[g % 2], in two
-    // parts so that the read of the bits can be issued long before its use: unit u =
-    // feature u / 4, bytes 4 * (u % 4) .. +3 of its 16 bytes of bits -> chunks
-    // 2 * (u % 4) and 2 * (u % 4) + 1 of its 128-byte row
-    constexpr uint32_t UNITS = TN * 4u, UPT = (UNITS + THREADS - 1u) / THREADS;  // units per thread
-    // a thread's i-th unit; past the last unit a thread repeats one (same bytes to the
-    // same place), so that no branch splits the loop body
-    auto unit = [&](uint32_t i) {
-        const uint32_t u = i * THREADS + tid;
-        return UNITS % THREADS == 0 || u < UNITS ? u : u - THREADS;
-    };
-    auto unpack_read = [&](uint32_t (&w)[UPT], uint32_t g) {
-        const unsigned char* bits = lds_bits + (g & 3u) * T::BITS_SLOT;
-#pragma unroll
-        for (uint32_t i = 0; i < UPT; ++i) {
-            const uint32_t u = unit(i);
-            w[i] = *reinterpret_cast<const uint32_t*>(bits + (u >> 2) * 16u + (u & 3u) * 4u);
-        }
-    };
-    auto unpack_lut = [&](uint2 (&e)[UPT][4], const uint32_t (&w)[UPT]) {
-#pragma unroll
-        for (uint32_t i = 0; i < UPT; ++i) {
-#pragma unroll
-            for (uint32_t b = 0; b < 4; ++b)
-                e[i][b] = lut[(w[i] >> (8u * b)) & 0xffu];
-        }
-    };
-    auto unpack_store = [&](const uint2 (&e)[UPT][4], uint32_t g) {
-        unsigned char* dst = lds_b + (g & 1u) * T::B_SLOT;
-#pragma unroll
-        for (uint32_t i = 0; i < UPT; ++i) {
-            const uint32_t u = unit(i), row = u >> 2, part = u & 3u;
-            *reinterpret_cast<uint4*>(dst + swz128(row, 2u * part)) =
-                make_uint4(e[i][0].x, e[i][0].y, e[i][1].x, e[i][1].y);
-            *reinterpret_cast<uint4*>(dst + swz128(row, 2u * part + 1u)) =
-                make_uint4(e[i][2].x, e[i][2].y, e[i][3].x, e[i][3].y);
-        }
-    };
-    auto unpack = [&](uint32_t g) {
-        uint32_t w[UPT];
-        uint2 e[UPT][4];
-        unpack_read(w, g);
-        unpack_lut(e, w);
-        unpack_store(e, g);
-    };
-
-    const uint32_t arow0 = wm * T::WTM + (lane & 15u), brow0 = wn * T::WTN + (lane & 15u);
-    const uint32_t chunk = lane >> 4;
-    // MFMA operands of group g: [half][subtile]
-    auto load_frags = [&](v4i (&a)[2][MS], v4i (&b)[2][NS], uint32_t g) {
-        const unsigned char* la = lds_a + (g & 3u) * T::A_SLOT;
-        const unsigned char* lb = lds_b + (g & 1u) * T::B_SLOT;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int mi = 0; mi < MS; ++mi)
-                a[h][mi] = *reinterpret_cast<const v4i*>(la + swz128(arow0 + 16u * mi, 4u * h + chunk));
-#pragma unroll
-            for (int ni = 0; ni < NS; ++ni)
-                b[h][ni] = *reinterpret_cast<const v4i*>(lb + swz128(brow0 + 16u * ni, 4u * h + chunk));
-        }
-    };
-
-    float acc[MS][NS][4];
-    v4i d[MS][NS];
-    const v4i c_init = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
-#pragma unroll
-    for (int mi = 0; mi < MS; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni) {
-            d[mi][ni] = c_init;  // with scale 0 the first epilogue adds +0
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                acc[mi][ni][r] = 0.0f;
-        }
-    float sc_prev[NS];
-#pragma unroll
-    for (int ni = 0; ni < NS; ++ni)
-        sc_prev[ni] = 0.0f;
-
-    // One group: see the header.  At entry (after the barrier) LDS holds group g+1's
-    // rows and +1/-1 tile, group g+3's bits and group g's scales (the DMAs of the
-    // previous step may still be landing); ubits holds group g+2's bits, read in the
-    // previous step.
-    uint32_t ubits[UPT];
-    auto step = [&](uint32_t g, v4i (&ca)[2][MS], v4i (&cb)[2][NS], v4i (&na)[2][MS], v4i (&nb)[2][NS]) {
-        // this wave's DMAs but the previous step's have landed, its LDS accesses are
-        // done; after the barrier the same holds for every wave
-        wait_dma<T::A_INS + 2>();
-        barrier();
-        issue_rows(g + 3u);
-        issue_bits(g + 5u);
-        issue_scales(g + 2u);
-        // LDS reads in this order: the table lookups of group g+2 (first, so that the
-        // unpack does not queue behind the operand reads), group g+3's bits, group
-        // g+1's operands, group g's scales
-        uint2 ex[UPT][4];
-        unpack_lut(ex, ubits);
-        __builtin_amdgcn_sched_barrier(0);
-        unpack_read(ubits, g + 3u);
-        load_frags(na, nb, g + 1u);
-        float sc_cur[NS];
-        const uint16_t* scl = reinterpret_cast<const uint16_t*>(lds_sc + (g & 3u) * T::SC_SLOT);
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-            sc_cur[ni] = __half2float(__ushort_as_half(scl[wn * T::WTN + 16u * ni + (lane & 15u)]));
-        __builtin_amdgcn_sched_barrier(0);
-        // first half: the epilogue of group g-1 on each subtile, then restart it
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni) {
-            const float sc = sc_prev[ni];
-            const float cneg = sc * -kMagicValue;  // exact
-#pragma unroll
-            for (int mi = 0; mi < MS; ++mi) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    acc[mi][ni][r] = acc[mi][ni][r] + __builtin_fmaf(sc, __int_as_float(d[mi][ni][r]), cneg);
-                d[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ca[0][mi], cb[0][ni], c_init, 0, 0, 0);
-            }
-        }
-        // per subtile its 8 epilogue VALU ops, then its restarting MFMA: the matrix
-        // pipe runs while the next subtile's VALU ops issue
-#pragma unroll
-        for (int i = 0; i < MS * NS; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        unpack_store(ex, g + 2u);
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-#pragma unroll
-            for (int mi = 0; mi < MS; ++mi)
-                d[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ca[1][mi], cb[1][ni], d[mi][ni], 0, 0, 0);
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-            sc_prev[ni] = sc_cur[ni];
-        __builtin_amdgcn_sched_barrier(0);  // nothing moves across steps
-    };
-
-    // prologue: groups 0..3's bits, 0..2's rows, 0..1's scales; groups 0 and 1 unpacked,
-    // group 2's bits in registers; group 4's bits issued once group 0's have been
-    // read (they share a slot); group 0's operands in registers
-#pragma unroll
-    for (uint32_t b = 0; b < 4; ++b)
-        issue_bits(b);
-    issue_scales(0);
-    issue_scales(1);
-    issue_rows(0);
-    issue_rows(1);
-    issue_rows(2);
-    wait_dma<0>();
-    barrier();  // the table and the first DMAs are in LDS
-    unpack(0);
-    unpack(1);
-    unpack_read(ubits, 2);
-    wait_dma<0>();
-    barrier();
-    issue_bits(4);
-    v4i xa[2][MS], xb[2][NS], ya[2][MS], yb[2][NS];
-    load_frags(xa, xb, 0);
-    uint32_t g = 0;
-    for (; g + 1u < groups; g += 2u) {
-        step(g, xa, xb, ya, yb);
-        step(g + 1u, ya, yb, xa, xb);
-    }
-    if (g < groups)
-        step(g, xa, xb, ya, yb);
-
-    // no DMA may still be writing LDS when it is reused or the workgroup ends
-    wait_dma<0>();
-    // epilogue of the last group
-#pragma unroll
-    for (int ni = 0; ni < NS; ++ni) {
-        const float sc = sc_prev[ni];
-        const float cneg = sc * -kMagicValue;
-#pragma unroll
-        for (int mi = 0; mi < MS; ++mi)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                acc[mi][ni][r] = acc[mi][ni][r] + __builtin_fmaf(sc, __int_as_float(d[mi][ni][r]), cneg);
-    }
-    // stage the tile in LDS, then store it row by row (16 bytes per lane where the
-    // output rows allow it); Z * s for GEMM_F32
-    barrier();
-    float* const so = reinterpret_cast<float*>(smem);
-#pragma unroll
-    for (int mi = 0; mi < MS; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                so[(wm * T::WTM + 16u * mi + 4u * (lane >> 4) + r) * T::OUT_STRIDE + wn * T::WTN + 16u * ni +
-                   (lane & 15u)] = acc[mi][ni][r];
-    wait_dma<0>();
-    barrier();
-    // stored in one of two forms, each without a branch per value
-    const auto store = [&](auto through) {
-        const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
-        const bool scaled = j.mode == MODE_SUM_SCALED;
-#pragma unroll
-        for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
-            const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
-            const uint32_t m = m0 + row, n = n0 + col;
-            if (m >= j.rows || n >= j.n)
-                continue;
-            float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
-            if (scaled) {
-                const float s = row_scale(j, m);
-                v.x = v.x * s;
-                v.y = v.y * s;
-                v.z = v.z * s;
-                v.w = v.w * s;
-            }
-            float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
-            if (vec && n + 4u <= j.n) {
-                put4(dst, v4i{__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)}, through);
-            } else {
-                put(dst, v.x, through);
-                if (n + 1u < j.n)
-                    put(dst + 1, v.y, through);
-                if (n + 2u < j.n)
-                    put(dst + 2, v.z, through);
-                if (n + 3u < j.n)
-                    put(dst + 3, v.w, through);
-            }
-        }
-    };
-    if (j.done)
-        store(std::true_type{});
-    else
-        store(std::false_type{});
-    gemm_signal(j, seq);
-}
-
-// k_gemm_co<TM, TN, WGM, WGN>: GEMM / GEMM_F32 with two workgroups per CU.  The
-// same per-group work as k_gemm_bits with a shorter pipeline, so that a 128 x 128
-// tile fits in 75 KB of LDS and 4 waves of at most 256 VGPRs: the rows' DMA runs one
-// group ahead (two slots), the unpack one, and each group's MFMA operands are read
-// right after its barrier; the other workgroup on the CU covers the latency.
-// Iteration g, after one wait and one barrier:
-//   * issue the DMAs of group g+1's rows, group g+4's bits and group g+2's scales;
-//   * look up group g+1's bits (read one iteration ago), read group g+2's bits, group
-//     g's operands and scales;
-//   * group g's first-half MFMAs interleaved with group g-1's epilogue;
-//   * store group g+1's +1/-1 tile; group g's second-half MFMAs.
-template <int TM, int TN, int WGM, int WGN>
-__global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_co(
-    GemmJob j, uint32_t mtiles, uint32_t ntiles, uint32_t band, uint64_t seq, const uint64_t* __restrict__ flag) {
-    using T = Tiling<TM, TN, WGM, WGN, 2>;
-    constexpr int MS = T::MS, NS = T::NS, THREADS = T::THREADS;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[T::SMEM];
-    if (*flag == seq) {
-        gemm_signal(j, seq);
-        return;
-    }
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave / WGN, wn = wave % WGN;
-    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
-    tile.nt = select_part(j, tile.nt);
-    const uint32_t m0 = tile.mt * TM, n0 = tile.nt * TN;
-    const uint32_t groups = j.groups;
-    unsigned char* const lds_a = smem;
-    unsigned char* const lds_b = smem + T::OFF_B;
-    unsigned char* const lds_bits = smem + T::OFF_BITS;
-    unsigned char* const lds_sc = smem + T::OFF_SC;
-    uint2* const lut = reinterpret_cast<uint2*>(smem + T::OFF_LUT);
-    if (tid < 256u)
-        lut[tid] = make_uint2(pm1_nibble(tid & 15u), pm1_nibble(tid >> 4));
-
-    const uint8_t* a_src[T::A_INS];
-#pragma unroll
-    for (uint32_t i = 0; i < T::A_INS; ++i) {
-        const uint32_t p = wave * T::A_CHUNKS + i * 64u + lane, r = min(p >> 3, TM - 1u);
-        const uint32_t c = (p & 7u) ^ ((r >> 1) & 7u);
-        a_src[i] = reinterpret_cast<const uint8_t*>(j.q) + (size_t)min(m0 + r, j.rows - 1u) * j.k + 16u * c;
-    }
-    const uint32_t f = T::BIT_LANES * wave + min(lane, T::BIT_LANES - 1u);
-    const uint8_t* bit_src = reinterpret_cast<const uint8_t*>(j.wbits) +
-                             ((size_t)min((n0 + f) >> 6, j.tiles - 1u) * groups * kTile + ((n0 + f) & 63u)) * 16u;
-    const uint32_t sc_first = (wave * T::SC_CPW) % T::SC_CHUNKS;
-    const uint32_t sc_col = n0 + 8u * (sc_first + min(lane, T::SC_CPW - 1u));
-    const uint8_t* sc_src = reinterpret_cast<const uint8_t*>(j.wscale) +
-                            ((size_t)min(sc_col >> 6, j.tiles - 1u) * groups * kTile + (sc_col & 63u)) * 2u;
-    const uint32_t la0 = lds_offset(lds_a), lbits0 = lds_offset(lds_bits), lsc0 = lds_offset(lds_sc);
-    const size_t bit_step = (size_t)kTile * 16u, sc_step = (size_t)kTile * 2u;
-    auto issue_rows = [&](uint32_t g) {
-        const uint32_t gg = min(g, groups - 1u);
-#pragma unroll
-        for (uint32_t i = 0; i < T::A_INS; ++i)
-            dma16_lanes<lane_mask<T::A_LANES>()>(a_src[i] + (size_t)gg * kGroup,
-                                                 la0 + (g & 1u) * T::A_SLOT + (wave * T::A_CHUNKS + i * 64u) * 16u);
-    };
-    auto issue_bits = [&](uint32_t g) {
-        const uint32_t gg = min(g, groups - 1u);
-        dma16_lanes<lane_mask<T::BIT_LANES>()>(bit_src + gg * bit_step,
-                                               lbits0 + (g & 3u) * T::BITS_SLOT + wave * (T::BIT_LANES * 16u));
-    };
-    auto issue_scales = [&](uint32_t g) {
-        const uint32_t gg = min(g, groups - 1u);
-        dma16_lanes<lane_mask<T::SC_CPW>()>(sc_src + gg * sc_step, lsc0 + (g & 3u) * T::SC_SLOT + 16u * sc_first);
-    };
-    constexpr uint32_t UNITS = TN * 4u, UPT = (UNITS + THREADS - 1u) / THREADS;
-    static_assert(UNITS % THREADS == 0, "whole units per thread");
-    auto unpack_read = [&](uint32_t (&w)[UPT], uint32_t g) {
-        const unsigned char* bits = lds_bits + (g & 3u) * T::BITS_SLOT;
-#pragma unroll
-        for (uint32_t i = 0; i < UPT; ++i) {
-            const uint32_t u = i * THREADS + tid;
-            w[i] = *reinterpret_cast<const uint32_t*>(bits + (u >> 2) * 16u + (u & 3u) * 4u);
-        }
-    };
-    auto unpack_lut = [&](uint2 (&e)[UPT][4], const uint32_t (&w)[UPT]) {
-#pragma unroll
-        for (uint32_t i = 0; i < UPT; ++i)
-#pragma unroll
-            for (uint32_t b = 0; b < 4; ++b)
-                e[i][b] = lut[(w[i] >> (8u * b)) & 0xffu];
-    };
-    auto unpack_store = [&](const uint2 (&e)[UPT][4], uint32_t g) {
-        unsigned char* dst = lds_b + (g & 1u) * T::B_SLOT;
-#pragma unroll
-        for (uint32_t i = 0; i < UPT; ++i) {
-            const uint32_t u = i * THREADS + tid, row = u >> 2, part = u & 3u;
-            *reinterpret_cast<uint4*>(dst + swz128(row, 2u * part)) =
-                make_uint4(e[i][0].x, e[i][0].y, e[i][1].x, e[i][1].y);
-            *reinterpret_cast<uint4*>(dst + swz128(row, 2u * part + 1u)) =
-                make_uint4(e[i][2].x, e[i][2].y, e[i][3].x, e[i][3].y);
-        }
-    };
-    const uint32_t arow0 = wm * T::WTM + (lane & 15u), brow0 = wn * T::WTN + (lane & 15u);
-    const uint32_t chunk = lane >> 4;
-    // half h of group g's MFMA operands (one register set, reused by the two halves)
-    auto load_half = [&](v4i (&a)[MS], v4i (&b)[NS], uint32_t g, uint32_t h) {
-        const unsigned char* la = lds_a + (g & 1u) * T::A_SLOT;
-        const unsigned char* lb = lds_b + (g & 1u) * T::B_SLOT;
-#pragma unroll
-        for (int mi = 0; mi < MS; ++mi)
-            a[mi] = *reinterpret_cast<const v4i*>(la + swz128(arow0 + 16u * mi, 4u * h + chunk));
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-            b[ni] = *reinterpret_cast<const v4i*>(lb + swz128(brow0 + 16u * ni, 4u * h + chunk));
-    };
-
-    float acc[MS][NS][4];
-    v4i d[MS][NS];
-    const v4i c_init = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
-#pragma unroll
-    for (int mi = 0; mi < MS; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni) {
-            d[mi][ni] = c_init;  // with scale 0 the first epilogue adds +0
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                acc[mi][ni][r] = 0.0f;
-        }
-    float sc_prev[NS];
-#pragma unroll
-    for (int ni = 0; ni < NS; ++ni)
-        sc_prev[ni] = 0.0f;
-
-    // prologue: groups 0..3's bits, 0..1's scales, group 0's rows; group 0 unpacked,
-    // group 1's bits in registers
-#pragma unroll
-    for (uint32_t b = 0; b < 4; ++b)
-        issue_bits(b);
-    issue_scales(0);
-    issue_scales(1);
-    issue_rows(0);
-    wait_dma<0>();
-    barrier();
-    uint32_t ubits[UPT];
-    {
-        uint2 e0[UPT][4];
-        unpack_read(ubits, 0);
-        unpack_lut(e0, ubits);
-        unpack_store(e0, 0);
-    }
-    unpack_read(ubits, 1);
-    wait_dma<0>();
-
-    for (uint32_t g = 0; g < groups; ++g) {
-        // this wave's DMAs but the last two have landed (group g's rows among them),
-        // its LDS accesses are done; after the barrier the same holds for every wave
-        wait_dma<2>();
-        barrier();
-        issue_rows(g + 1u);
-        issue_bits(g + 4u);
-        issue_scales(g + 2u);
-        uint2 ex[UPT][4];
-        unpack_lut(ex, ubits);
-        __builtin_amdgcn_sched_barrier(0);
-        unpack_read(ubits, g + 2u);
-        v4i ca[MS], cb[NS];
-        load_half(ca, cb, g, 0);
-        float sc_cur[NS];
-        const uint16_t* scl = reinterpret_cast<const uint16_t*>(lds_sc + (g & 3u) * T::SC_SLOT);
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-            sc_cur[ni] = __half2float(__ushort_as_half(scl[wn * T::WTN + 16u * ni + (lane & 15u)]));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni) {
-            const float sc = sc_prev[ni];
-            const float cneg = sc * -kMagicValue;  // exact
-#pragma unroll
-            for (int mi = 0; mi < MS; ++mi) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    acc[mi][ni][r] = acc[mi][ni][r] + __builtin_fmaf(sc, __int_as_float(d[mi][ni][r]), cneg);
-                d[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ca[mi], cb[ni], c_init, 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < MS * NS; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        unpack_store(ex, g + 1u);
-        load_half(ca, cb, g, 1);
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-#pragma unroll
-            for (int mi = 0; mi < MS; ++mi)
-                d[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ca[mi], cb[ni], d[mi][ni], 0, 0, 0);
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-            sc_prev[ni] = sc_cur[ni];
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    wait_dma<0>();
-#pragma unroll
-    for (int ni = 0; ni < NS; ++ni) {
-        const float sc = sc_prev[ni];
-        const float cneg = sc * -kMagicValue;
-#pragma unroll
-        for (int mi = 0; mi < MS; ++mi)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                acc[mi][ni][r] = acc[mi][ni][r] + __builtin_fmaf(sc, __int_as_float(d[mi][ni][r]), cneg);
-    }
-    barrier();
-    float* const so = reinterpret_cast<float*>(smem);
-#pragma unroll
-    for (int mi = 0; mi < MS; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NS; ++ni)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                so[(wm * T::WTM + 16u * mi + 4u * (lane >> 4) + r) * T::OUT_STRIDE + wn * T::WTN + 16u * ni +
-                   (lane & 15u)] = acc[mi][ni][r];
-    wait_dma<0>();
-    barrier();
-    // stored in one of two forms, each without a branch per value
-    const auto store = [&](auto through) {
-        const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
-        const bool scaled = j.mode == MODE_SUM_SCALED;
-#pragma unroll
-        for (uint32_t c0 = 0; c0 < TM * TN / 4u; c0 += THREADS) {
-            const uint32_t c = c0 + tid, row = c / (TN / 4u), col = 4u * (c % (TN / 4u));
-            const uint32_t m = m0 + row, n = n0 + col;
-            if (m >= j.rows || n >= j.n)
-                continue;
-            float4 v = *reinterpret_cast<const float4*>(so + row * T::OUT_STRIDE + col);
-            if (scaled) {
-                const float s = row_scale(j, m);
-                v.x = v.x * s;
-                v.y = v.y * s;
-                v.z = v.z * s;
-                v.w = v.w * s;
-            }
-            float* dst = reinterpret_cast<float*>(j.out + (size_t)m * j.out_stride) + n;
-            if (vec && n + 4u <= j.n) {
-                put4(dst, v4i{__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)}, through);
-            } else {
-                put(dst, v.x, through);
-                if (n + 1u < j.n)
-                    put(dst + 1, v.y, through);
-                if (n + 2u < j.n)
-                    put(dst + 2, v.z, through);
-                if (n + 3u < j.n)
-                    put(dst + 3, v.w, through);
-            }
-        }
-    };
-    if (j.done)
-        store(std::true_type{});
-    else
-        store(std::false_type{});
-    gemm_signal(j, seq);
-}
-
 uint32_t gemm_band(const GemmJob& job, uint32_t mtiles);
 uint32_t gemm_ntiles(GemmJob& job, uint32_t tn);
 
@@ -830,12 +223,6 @@ hipError_t launch_tiles(const GemmLaunch& at, Kernel kernel, uint32_t threads, G
     return hipGetLastError();
 }
 
-
-template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_co(const GemmLaunch& at, GemmJob job) {
-    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
-    return launch_tiles(at, k_gemm_co<TM, TN, WGM, WGN>, 64 * WGM * WGN, job, mtiles, ntiles);
-}
 
 // k_gemm_ks: F32-accumulating jobs with too few tiles to give every CU a workgroup.
 // Workgroup tile (16*TMS) x (16*TNS); the W waves split K instead of the tile: wave w
@@ -2212,12 +1599,6 @@ hipError_t launch_dots(const GemmLaunch& at, GemmJob job) {
     return launch_tiles(at, k_gemm_dots<TNS, GB, WAVES>, 64 * WAVES, job, mtiles, ntiles);
 }
 
-template <int TM, int TN, int WGM, int WGN>
-hipError_t launch_bits(const GemmLaunch& at, GemmJob job) {
-    const uint32_t mtiles = (job.rows + TM - 1u) / TM, ntiles = gemm_ntiles(job, TN);
-    return launch_tiles(at, k_gemm_bits<TM, TN, WGM, WGN>, 64 * WGM * WGN, job, mtiles, ntiles);
-}
-
 }  // namespace
 
 // The largest workgroup tile that still gives every CU a workgroup, else the tile
@@ -2232,9 +1613,6 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
             cols += (job.parts[i].n + tn - 1u) / tn;
         return (uint64_t)((job.rows + tm - 1u) / tm) * cols;
     };
-#ifndef BNN_GEMM_CO
-#define BNN_GEMM_CO 1  // F32-accumulating jobs with a 128 x 128 tile per CU: two workgroups per CU (k_gemm_co)
-#endif
     // Few rows: K split over the waves of a workgroup, every wave's operands brought into
     // LDS by DMA before anything is computed (k_gemm_kr, k_gemm_kc).  The rules follow a
     // forced-choice sweep over K = 1024..8192, N = 1024..8192 and 8..256 rows (all outputs
@@ -2243,11 +1621,12 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // 256 rows 14.5 -> 12.2 us, 6144->2048 x 128 rows 13.3 -> 9.6 us, 8192->2048 x 32 rows
     // 9.2 -> 7.0 us.  Up to 16 groups: 32 x 32 tiles while they fit one round of two per CU,
     // then 32 x 64 tiles while those fit one round (16 waves of one group each above 8 groups),
-    // then 32 x 32 tiles up to 4.5 rounds
-    // (not for 8 groups, where the tiled kernels win past one round); 17..32 groups: 16 x 32
-    // tiles in one round, then 32 x 32 up to three rounds; 33..48 groups: 16 x 32 tiles, then
-    // 16 x 64 tiles with the slices' running sums handed on (k_gemm_kc), each in one round;
-    // 49..64 groups: 16 x 16 tiles in one round.
+    // then 32 x 32 tiles up to two rounds (not up to 8 groups, where the tiled kernel wins past
+    // one round); 17..32 groups: 16 x 32 tiles, then 32 x 32; 33..48 groups: 16 x 32 tiles, then
+    // 16 x 64 tiles with the slices' running sums handed on (k_gemm_kc); 49..64 groups: 16 x 16
+    // tiles; each in one round.  Past those bounds k_gemm_mx wins (2048->2048 x 320 rows a call
+    // of 25.0 us against 23.0, x 256 20.0 against 22.6; 4096->2048 x 180 27.9 against 26.3, x
+    // 100 21.9 against 24.1).
     if (job.mode == MODE_DOT_I16) {
         // 32-column tiles up to two per CU, and past 16 groups, whose tiles of 64 columns would
         // not fit two workgroups' LDS
@@ -2267,12 +1646,12 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
                 return launch_kr<2, 4, 16, 1>(at, job);  // 2048->6144 x 64 rows 6.2 -> 5.7 us
             if (blocks(32, 64) <= cus)
                 return launch_kr<2, 4, 8, 2>(at, job);
-            if (g > 8u && blocks(32, 32) <= 9u * cus / 2u)
+            if (g > 8u && blocks(32, 32) <= 2u * cus)
                 return launch_kr<2, 2, 8, 2>(at, job);
         } else if (g <= 32u) {
             if (blocks(16, 32) <= cus)
                 return launch_kr<1, 2, 8, 4>(at, job);
-            if (blocks(32, 32) <= 3u * cus)
+            if (blocks(32, 32) <= cus)
                 return launch_kr<2, 2, 8, 4>(at, job);
         } else if (g <= 48u) {
             if (blocks(16, 32) <= cus)
@@ -2291,59 +1670,44 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     if (job.rows <= 64u && (job.rows <= 32u || job.groups <= 16u) &&
         blocks(16, 16) <= 3u * cus)
         return launch_wv<1, 1, 1, 1, 8>(at, job);
-    // K >= 6144 with between half a round and one round of 32 x 64 tiles: eight waves
-    // splitting K per tile (6144->2048 x 256 rows 17.1 us against 19.1 us for a wave per
-    // 32 x 32 block, 8192->2048 x 256 21.6 against 23.3, 8192->1024 x 320-512 21.7-22.2
-    // against 24.2-28.4; forced-choice sweep, bit-identical outputs; it loses at K = 4096,
-    // below half a round and from a second round on)
-    if (job.groups >= 48u && blocks(32, 64) > cus / 2u && blocks(32, 64) <= cus)
-        return launch_ks<2, 4, 8, 3>(at, job);
-    // K split over four waves per 32 x 64 tile: 17..47 groups with between half a round and
-    // one round of tiles (4096->2048 x 192 rows 14.0 us against 15.9 for 32 x 64
-    // workgroup tiles, 4096->6144 x 48-64 rows 13.9-14.2 against 15.7-15.9,
-    // 3072->8100 x 40-64 rows 12.0-12.2 against 13.3), and >= 48 groups with one to two
-    // rounds (6144->2048 x 384-512 rows 24.7-25.4 against 26.3-26.8, 6144->6144 x
-    // 96-128 rows 23.8-24.4 against 26.1-26.5; forced-choice sweeps, bit-identical
-    // outputs; at 16 groups and from a third round on the tiled kernels win)
-    if (job.groups > 16u && job.groups < 48u && blocks(32, 64) > cus / 2u &&
-        blocks(32, 64) <= cus)
-        return launch_ks<2, 4, 4, 3>(at, job);
-    if (job.groups >= 48u && blocks(32, 64) > cus && blocks(32, 64) <= 2u * cus)
-        return launch_ks<2, 4, 4, 3>(at, job);
-    // a long K (>= 32 groups) with two to three 32 x 32 blocks per CU: a wave per block
-    // beats the tiled kernels, whose per-group steps serialise over the long K
-    if (job.groups >= 32u && blocks(32, 32) >= 2u * cus && blocks(32, 32) <= 3u * cus)
-        return launch_wv<2, 2, 1, 1, 4>(at, job);
-    if (blocks(128, 192) >= cus)
-        return launch_mx<128, 192, 2, 4>(at, job);
-    if (blocks(64, 128) >= cus && job.groups >= 32u)
-        return launch_mx<64, 128, 2, 4>(at, job);
-    if (BNN_GEMM_CO && blocks(128, 128) >= cus)
-        return launch_co<128, 128, 2, 2>(at, job);
-    // 128 x 128 tiles also where 64 x 128 ones would need a second round of workgroups
-    // (one 8-wave 64 x 128 workgroup per CU fits the registers): 1.26-1.43x measured at
-    // 144-192 tiles of 128 x 128
-    if (blocks(128, 128) >= cus || blocks(64, 128) > cus)
-        return launch_bits<128, 128, 2, 4>(at, job);
-    if (blocks(64, 128) >= cus)
-        return launch_bits<64, 128, 2, 4>(at, job);
-    if (blocks(64, 64) >= cus)
-        return launch_bits<64, 64, 2, 2>(at, job);
-    const uint64_t enough = cus * 3u / 4u;
-    if (blocks(32, 64) < enough && blocks(32, 32) <= cus) {
-        // too few tiles for the CUs (jobs of more than 48 groups get here): K split across
-        // eight waves of a workgroup with 32 x 32 tiles while those fit one round, else four
-        // waves with 32 x 16 tiles
-        if (blocks(32, 32) >= enough)
+    // too few tiles for the CUs (jobs of more than 48 groups get here): K split across eight
+    // waves of a workgroup with 32 x 32 tiles between three quarters of a round and one round
+    // of them, or across four waves with 32 x 16 tiles in one round (8192->1000 x 180 rows a
+    // call of 31.1 us against 34.6 with k_gemm_mx, x 100 28.3 against 31.9)
+    if (blocks(32, 32) <= cus) {
+        if (blocks(32, 32) >= cus * 3u / 4u)
             return launch_ks<2, 2, 8, 3>(at, job);
-        return launch_ks<2, 1, 4, 3>(at, job);
+        if (blocks(32, 16) <= cus)
+            return launch_ks<2, 1, 4, 3>(at, job);
     }
-    // three quarters of a round of 64 x 64 tiles: those beat a round and more of 32 x 64
-    // ones (2048->2048 x 384 rows 11.7 us against 12.6, 2048->6144 x 96-128 rows 11.6-11.7
-    // against 12.0-12.4)
-    if (blocks(64, 64) >= enough)
-        return launch_bits<64, 64, 2, 2>(at, job);
-    return launch_bits<32, 64, 2, 2>(at, job);
+    // past 16 groups in one round of 32 x 64 tiles: a step of the smallest tile is the
+    // shortest (6144->2048 x 180 rows 32.1 -> 31.0 us a call against a K split over the waves
+    // of 32 x 64 tiles, 8192->1000 x 130 40.7 -> 32.9, 5120->2048 x 130 30.7 -> 27.5,
+    // 4096->8192 x 64 27.8 -> 24.7); up to 16 groups 64 x 64 tiles are as fast
+    if (job.groups > 16u && blocks(32, 64) <= cus)
+        return launch_mx<32, 64, 1, 4>(at, job);
+    // Everything else: k_gemm_mx, one workgroup per CU, in the tile whose rounds of workgroups
+    // take the least time.  A round takes ~2.5 us and, per group, the step that a sweep gave for
+    // each tile (17 shapes of K = 384..8192 and N = 1000..8192 x 14 row counts from 48 to 1024,
+    // all outputs bit-identical; the choice was within 4% of the best tile for every one).  With
+    // tiles of 128 x 192 and 64 x 128 only, other kernels had filled the gaps, a call of
+    // 6144->2048 x 389 rows 42.8 -> 34.1 us, x 640 56.4 -> 41.5, 4096->4096 x 389 43.4 -> 33.2,
+    // 2048->2048 x 640 32.5 -> 25.3, 2048->4096 x 256 27.0 -> 23.1, 8192->4096 x 768 85 -> 69.
+    const auto time = [&](uint32_t tm, uint32_t tn, double step) {
+        return (double)((blocks(tm, tn) + cus - 1u) / cus) * (2.5 + step * job.groups);
+    };
+    const double t64 = time(64, 64, 0.34), t128 = time(64, 128, 0.45), t192 = time(64, 192, 0.60);
+    const double t128x128 = time(128, 128, 0.72), t128x192 = time(128, 192, 0.88);
+    const double least = std::min({t64, t128, t192, t128x128, t128x192});
+    if (t64 == least)
+        return launch_mx<64, 64, 2, 4>(at, job);
+    if (t128 == least)
+        return launch_mx<64, 128, 2, 4>(at, job);
+    if (t192 == least)
+        return launch_mx<64, 192, 2, 4>(at, job);
+    if (t128x128 == least)
+        return launch_mx<128, 128, 2, 4>(at, job);
+    return launch_mx<128, 192, 2, 4>(at, job);
 }
 
 }  // namespace bnnhip

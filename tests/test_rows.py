@@ -299,3 +299,39 @@ def test_dot_groups_rows(pkg, hipdev, oracle_fast, k, n, rows, off, pad):
     bi.free()
     bo.free()
     m.destroy()
+
+
+# k_gemm_mx in each of its tiles, at group counts around its pipeline's depth, ragged both ways
+@pytest.mark.parametrize("op", ["GEMM_F32", "GEMM"])
+@pytest.mark.parametrize("k,n,rows,pad", [
+    (128, 1500, 500, 0),      # 64 x 64, one group
+    (2176, 701, 650, 12),     # 64 x 64, 17 groups, rows that are not 16-byte aligned
+    (256, 2100, 641, 0),      # 64 x 128
+    (384, 4000, 642, 16),     # 64 x 192
+    (640, 3999, 1000, 0),     # 128 x 128
+    (512, 5001, 770, 4),      # 128 x 192
+    (2048, 4213, 250, 0),     # 64 x 128, more workgroups than signal
+    (6144, 2048, 289, 0),     # 64 x 64, 48 groups
+    (4224, 4001, 99, 8),      # 32 x 64, 33 groups
+    (8192, 1000, 130, 0),     # 32 x 64, 64 groups
+])
+def test_gemm_tiles(pkg, hipdev, oracle_fast, op, k, n, rows, pad):
+    from bnn_cases import fast_oracle
+    host = pkg.synth.matrix(n, k, seed=k + n)
+    f32_in = op == "GEMM_F32"
+    x = pkg.synth.normal_f32(rows, k, seed=5) if f32_in else pkg.synth.int8_uniform(rows, k, seed=5)
+    m = hipdev.matrix(*host)
+    bi, bo = hipdev.buffer(x.nbytes), hipdev.buffer(rows * (4 * n + pad))
+    bi.write(x)
+    bo.write(np.full(bo.nbytes, 0x5a, np.uint8))
+    T = pkg.Type
+    job = pkg.Job(int(pkg.Op[op]), m.handle.value, bi.view(T.F32 if f32_in else T.I8), bo.view(T.F32, 0, 4 * n + pad), rows)
+    print(f"{op} {k}->{n} x {rows}", flush=True)
+    assert hipdev.execute(job) == pkg.Status.OK
+    raw = bo.read().reshape(rows, 4 * n + pad)
+    want = fast_oracle(pkg, oracle_fast, op, *host, x).reshape(rows, n)
+    assert np.array_equal(raw[:, :4 * n].copy().view(np.uint32), want.view(np.uint32))
+    assert (raw[:, 4 * n:] == 0x5a).all()
+    bi.free()
+    bo.free()
+    m.destroy()
