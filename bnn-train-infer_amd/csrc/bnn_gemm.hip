@@ -133,14 +133,6 @@ __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
-// vmcnt(N) and lgkmcnt(0): at most N of this wave's DMAs in flight, its LDS reads and
-// writes done
-template <int N>
-__device__ __forceinline__ void wait_dma() {
-    static_assert(N >= 0 && N < 16, "vmcnt field");
-    __builtin_amdgcn_s_waitcnt(0x0070 | N);
-}
-
 // A job's row scale through the global address space (a flat load would also count on the
 // LDS counter that the kernels' LDS waits use).
 __device__ __forceinline__ float row_scale(const GemmJob& j, uint32_t m) {
@@ -176,6 +168,19 @@ __device__ __forceinline__ void put2(void* p, uint16_t v, bool through) {
         *(__attribute__((address_space(1))) uint16_t*)p = v;
 }
 
+// Workgroup barrier for data handed over in LDS: this wave's LDS accesses are done before it
+// (s_barrier itself waits for none, and the compiler adds no wait on gfx950: another wave
+// could read what is still on its way into LDS), and at most VM of its DMAs are in flight
+// (63: any number).  The gfx9 encoding splits vmcnt into bits 3:0 and 15:14.
+template <uint32_t VM = 63u>
+__device__ __forceinline__ void lds_barrier() {
+    static_assert(VM < 64u, "vmcnt field");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((int)((VM & 15u) | 0x0070u | ((VM >> 4) << 14)));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");  // no LDS access moves across it
+}
+
 // The end of a workgroup in a launch whose caller waits for it (GemmJob::done): once the
 // stores of all its waves are complete (vmcnt), the workgroup stores seq into its own pinned
 // host word; the host spins on those words instead of waiting for the end of the kernel, which
@@ -184,8 +189,7 @@ __device__ __forceinline__ void put2(void* p, uint16_t v, bool through) {
 __device__ __forceinline__ void gemm_signal(const GemmJob& j, uint64_t seq) {
     if (j.done == nullptr)
         return;
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __builtin_amdgcn_s_barrier();
+    lds_barrier<0>();
     if (threadIdx.x == 0)
         __hip_atomic_store(j.done + blockIdx.x, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -1284,14 +1288,6 @@ struct MxTiling {
     static_assert(TM * TN / 4u % THREADS == 0, "output chunks per thread");
 };
 
-// s_waitcnt vmcnt(N) lgkmcnt(0) for N < 64 (the gfx9 encoding splits vmcnt into bits
-// 3:0 and 15:14)
-template <uint32_t N>
-__device__ __forceinline__ void wait_vm_lgkm0() {
-    static_assert(N < 64u, "vmcnt field");
-    __builtin_amdgcn_s_waitcnt((int)((N & 15u) | 0x0070u | ((N >> 4) << 14)));
-}
-
 template <int TM, int TN, int WGM, int WGN>
 __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t mtiles, uint32_t ntiles,
                                                             uint32_t band, uint64_t seq,
@@ -1384,8 +1380,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t 
         // this wave's DMAs of group g have landed (those of groups g+1 .. g+DEPTH-1 are
         // newer); then every wave's have, and every wave has read the slot that group
         // g+DEPTH takes
-        wait_vm_lgkm0<(DEPTH - 1u) * T::VM_PER_GROUP>();
-        barrier();
+        lds_barrier<(DEPTH - 1u) * T::VM_PER_GROUP>();
         const unsigned char* slot = smem + (g % T::SLOTS) * T::SLOT_BYTES;
         uint32_t bits[NS];
         uint16_t sraw[NS];
@@ -1472,8 +1467,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t 
                                                                                            : dd[0][mi][ni][r]),
                                                                  cneg_prev[ni]);
     // no DMA may still be writing LDS when it is reused for the staged tile
-    wait_dma<0>();
-    barrier();
+    lds_barrier<0>();
     float* const so = reinterpret_cast<float*>(smem);
 #pragma unroll
     for (uint32_t mi = 0; mi < MS; ++mi)
@@ -1483,7 +1477,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_mx(GemmJob j, uint32_t 
             for (uint32_t r = 0; r < 4; ++r)
                 so[(wm * T::WTM + 16u * mi + 4u * chunk + r) * T::OUT_STRIDE + wn * T::WTN + 16u * ni + (lane & 15u)] =
                     acc[mi][ni][r];
-    barrier();
+    lds_barrier();
     // stored in one of two forms, each without a branch per value
     const auto store = [&](auto through) {
         const bool vec = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 15u) == 0;
