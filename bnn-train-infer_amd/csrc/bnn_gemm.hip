@@ -194,11 +194,6 @@ __device__ __forceinline__ void gemm_signal(const GemmJob& j, uint64_t seq) {
         __hip_atomic_store(j.done + blockIdx.x, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-__device__ __forceinline__ void barrier() {
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");  // no LDS access moves across it
-}
-
 uint32_t gemm_band(const GemmJob& job, uint32_t mtiles);
 uint32_t gemm_ntiles(GemmJob& job, uint32_t tn);
 
@@ -361,9 +356,8 @@ __global__ __launch_bounds__(64 * W) void k_gemm_ks(GemmJob j, uint32_t mtiles, 
                 }
             }
         }
+        lds_barrier();               // the previous round's reads of prod are done
         expand(o[(d + 1) % DEPTH]);  // round r+1's operands, loaded one round ago
-        // the previous round's reads of prod are done (their sums consumed them)
-        barrier();
         if (g < groups) {
 #pragma unroll
             for (int mi = 0; mi < TMS; ++mi)
@@ -371,8 +365,7 @@ __global__ __launch_bounds__(64 * W) void k_gemm_ks(GemmJob j, uint32_t mtiles, 
                 for (int ni = 0; ni < TNS; ++ni)
                     *reinterpret_cast<float4*>(&prod[wave][((mi * TNS + ni) * 64u + lane) * 4u]) = p[mi][ni];
         }
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's LDS writes are done
-        barrier();
+        lds_barrier();  // every wave's products are in LDS
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             if (W * r + w < groups) {
@@ -394,7 +387,7 @@ __global__ __launch_bounds__(64 * W) void k_gemm_ks(GemmJob j, uint32_t mtiles, 
 #pragma unroll
     for (int d = 0; d + 1 < DEPTH; ++d)
         load(o[d], d);
-    barrier();  // the table is in LDS
+    lds_barrier();  // the table is in LDS
     expand(o[0]);
     const uint32_t rounds = (groups + W - 1u) / W;
     // the round count is padded to a multiple of DEPTH with rounds of no groups
@@ -538,7 +531,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wv(GemmJob j, uint32_t mt
 #pragma unroll
     for (int d = 0; d + 1 < DEPTH; ++d)
         load(o[d], d);
-    barrier();  // the table is in LDS
+    lds_barrier();  // the table is in LDS
 
     // group g = g0 + d from ring slot d: refill the slot emptied one group ago, expand
     // the bits, group g's MFMAs into D set d % 2, group g-1's epilogue from the other
@@ -883,8 +876,7 @@ __global__ __launch_bounds__(64 * W) void k_gemm_kr(GemmJob j, uint32_t mtiles, 
     uint2* const lut = reinterpret_cast<uint2*>(smem + T::OFF_LUT);
     for (uint32_t i = tid; i < 256u; i += T::NT)
         lut[i] = make_uint2(pm1_nibble(i & 15u), pm1_nibble(i >> 4));
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's table entries are written
-    barrier();                           // ... and every wave's
+    lds_barrier();  // the table is in LDS
 
     // 2. the rounds, software-pipelined: iteration i reads round i's operands from LDS
     // (after waiting for this wave's DMAs of round i: at most (R - 1 - i) rounds of them
@@ -1099,9 +1091,7 @@ __global__ __launch_bounds__(64 * WN * KS) void k_gemm_kc(GemmJob j, uint32_t mt
     uint2* const lut = reinterpret_cast<uint2*>(smem + T::OFF_LUT);
     for (uint32_t i = tid; i < 256u; i += T::NT)
         lut[i] = make_uint2(pm1_nibble(i & 15u), pm1_nibble(i >> 4));
-    wait_vm<0>();
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's DMAs and table entries are done
-    barrier();                           // ... and every wave's
+    lds_barrier<0>();  // every wave's DMAs and the table are in LDS
 
     // 2. this wave's products over its K slice, software-pipelined as in k_gemm_kr
     const uint32_t nn = wave % WN, s = wave / WN, g0 = s * T::GS;
@@ -1202,8 +1192,7 @@ __global__ __launch_bounds__(64 * WN * KS) void k_gemm_kc(GemmJob j, uint32_t mt
                 for (uint32_t ni = 0; ni < (uint32_t)TNW; ++ni)
                     xchg[(mi * TNW + ni) * 64u] = acc[mi][ni];
         }
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-        barrier();
+        lds_barrier();
         if (s == t) {
 #pragma unroll
             for (uint32_t mi = 0; mi < (uint32_t)TMS; ++mi)

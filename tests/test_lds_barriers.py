@@ -106,12 +106,23 @@ def test_counting():
     assert at_barriers(["ds_write_b32 v0, v1", "s_waitcnt lgkmcnt(0)", "ds_bpermute_b32 v0, v0, v1", "s_barrier"]) == [0]
 
 
-def test_gemm_mx(tmp_path):
-    kernels = functions(device_assembly(tmp_path, PKG_DIR / "csrc" / "bnn_gemm.hip"))
+# the sources that use the builtin, themselves or through a header (__syncthreads brings its waits)
+SOURCES = ["csrc/bnn_gemm.hip", "csrc/bnn_fused.hip", "csrc/bnn_rows.hip", "csrc/bnn_chain.hip", "engine/resident.hip"]
+
+
+@pytest.mark.parametrize("source", SOURCES)
+def test_barriers(tmp_path, source):
     checked = 0
-    for name, body in kernels.items():
-        if "k_gemm_mx" in name:
-            counts = at_barriers(body)
-            assert len(counts) >= 4 and not any(counts), (name, counts)
-            checked += 1
-    assert checked == 6
+    for name, body in functions(device_assembly(tmp_path, PKG_DIR / source)).items():
+        counts = at_barriers(body)
+        assert not any(counts), (name, counts)
+        checked += len(counts)
+    assert checked
+
+
+def test_every_source_is_checked():
+    texts = {p.relative_to(PKG_DIR): p.read_text() for p in PKG_DIR.rglob("*.h*") if p.suffix in (".hip", ".h")}
+    headers = {p.name for p, text in texts.items() if p.suffix == ".h" and "__builtin_amdgcn_s_barrier" in text}
+    users = {str(p) for p, text in texts.items() if p.suffix == ".hip" and (
+        "__builtin_amdgcn_s_barrier" in text or any(h in text and "lds_barrier" in text for h in headers))}
+    assert users == set(SOURCES)
