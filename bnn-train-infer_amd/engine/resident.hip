@@ -1170,10 +1170,11 @@ struct Resident {
     bool allow_fused, fused;
     BNNX_Batch *qkv, *attn_out, *gate_up, *down;
     BNNX_Batch lm_head;
-    // prefill: the activations of a block of block_rows prompt tokens (made by the first call
-    // with more than one token), block_out written by the linear layers and block_in read by
-    // them as buffers of the accelerator, the residual stream and the scores of one layer
-    uint32_t block_rows;
+    // prefill: the activations of a block of prompt tokens (made by the first call that runs
+    // one), block_out written by the linear layers and block_in read by them as buffers of the
+    // accelerator, the residual stream (x twice), each with the tokens that it holds, and the
+    // scores of one layer
+    uint32_t out_rows, in_rows, x_rows;
     BNN_Buffer b_block_out, b_block_in;
     float *block_out, *block_in, *block_x;
     float* block_scores;
@@ -1700,37 +1701,46 @@ uint32_t block_rows_for(const Resident* r, uint32_t n, uint32_t pos0) {
     return n <= rows ? n : (uint32_t)(rows >= 64u ? rows & ~(size_t)63u : rows);
 }
 
-// Memory for blocks of `rows` tokens and `scores` scores.  Rows grow by doubling from
-// kBlockFirstRows, and outgrown buffers stay with the context: giving a buffer back makes every
+// Memory for blocks of `rows` tokens and `scores` scores.  Every part grows by itself, at least
+// doubling from kBlockFirstRows.  Outgrown accelerator buffers stay with the context, and so
+// does a buffer that has grown when another part finds no memory: giving one back makes every
 // prepared batch of the device stale, a caller's own ones too.
 BNNE_Status ready_block(Resident* r, uint32_t rows, size_t scores) {
-    BNNE_Status st = BNNE_OK;
-    if (rows > r->block_rows) {
-        rows = std::min(std::max({rows, 2u * r->block_rows, kBlockFirstRows}), kBlockRows);
-        const BlockLayout at(r, rows);
-        BNN_Buffer b_out = nullptr, b_in = nullptr;
-        float *out = nullptr, *in = nullptr, *x = nullptr;
-        st = alloc_buffer(r, at.out_floats, &b_out, &out);
-        if (st == BNNE_OK)
-            st = alloc_buffer(r, at.in_floats, &b_in, &in);
-        if (st == BNNE_OK)
-            st = upload(&x, nullptr, 2u * (size_t)rows * r->C * sizeof(float));
-        if (st != BNNE_OK) {
-            BNN_BufferFree(b_out);
-            BNN_BufferFree(b_in);
+    const auto grown = [&](uint32_t held) { return std::min(std::max({rows, 2u * held, kBlockFirstRows}), kBlockRows); };
+    const auto grow = [&](uint32_t* held, BNN_Buffer* buffer, float** at, size_t BlockLayout::*floats) {
+        if (rows <= *held)
+            return BNNE_OK;
+        const uint32_t to = grown(*held);
+        BNN_Buffer b = nullptr;
+        float* p = nullptr;
+        const BNNE_Status st = alloc_buffer(r, BlockLayout(r, to).*floats, &b, &p);
+        if (st != BNNE_OK)
             return st;
+        if (*buffer)
+            r->outgrown[r->outgrown_count++] = *buffer;
+        *buffer = b;
+        *at = p;
+        *held = to;
+        return BNNE_OK;
+    };
+    BNNE_Status st = grow(&r->out_rows, &r->b_block_out, &r->block_out, &BlockLayout::out_floats);
+    if (st == BNNE_OK)
+        st = grow(&r->in_rows, &r->b_block_in, &r->block_in, &BlockLayout::in_floats);
+    if (st == BNNE_OK && rows > r->x_rows) {
+        const uint32_t to = grown(r->x_rows);
+        float* x = nullptr;
+        st = upload(&x, nullptr, 2u * (size_t)to * r->C * sizeof(float));
+        if (st == BNNE_OK) {
+            if (r->block_x) {
+                (void)hipStreamSynchronize(r->stream);
+                (void)hipFree(r->block_x);
+            }
+            r->block_x = x;
+            r->x_rows = to;
         }
-        if (r->block_rows) {
-            (void)hipStreamSynchronize(r->stream);
-            (void)hipFree(r->block_x);
-            r->outgrown[r->outgrown_count++] = r->b_block_out;
-            r->outgrown[r->outgrown_count++] = r->b_block_in;
-        }
-        r->b_block_out = b_out, r->block_out = out;
-        r->b_block_in = b_in, r->block_in = in;
-        r->block_x = x;
-        r->block_rows = rows;
     }
+    if (st != BNNE_OK)
+        return st;
     if (scores > r->block_score_floats) {
         if (r->block_scores) {
             (void)hipStreamSynchronize(r->stream);
@@ -1779,9 +1789,9 @@ bool block_path(const Resident* r) {
 // last token's residual stream in x and o, where the lm_head batch reads them.
 BNNE_Status enqueue_block(Resident* r, const int32_t* tokens_dev, uint32_t rows, uint32_t pos0, bool first) {
     const uint32_t C = r->C, HD = r->HD;
-    const BlockLayout at(r, r->block_rows);
+    const BlockLayout at(r, r->out_rows);
     float* const x = r->block_x;
-    float* const x2 = x + (size_t)r->block_rows * C;
+    float* const x2 = x + (size_t)r->x_rows * C;
     float* const o = r->block_out + at.o;
     const float* attn_norm = r->gains;
     const float* ffn_norm = r->gains + (size_t)r->L * C;
@@ -1853,8 +1863,6 @@ BNNE_Status enqueue_blocks(Resident* r, const int32_t* tokens, uint32_t n, uint3
     const uint32_t rows = block_rows_for(r, n, pos0);
     const size_t pitch = ((size_t)pos0 + n + 63u) & ~(size_t)63u;
     BNNE_Status st = ready_block(r, rows, pitch * r->H * rows);
-    if (st == BNNE_OK)
-        st = ready_batches(r);  // a failed growth frees buffers, which makes batches stale
     if (st != BNNE_OK)
         return st;
     std::memcpy(r->pinned_tokens, tokens, (size_t)n * sizeof(int32_t));
@@ -1909,9 +1917,8 @@ BNNE_Status resident_step(bnne_context* c, Resident* r, const int32_t* tokens, u
         (st == BNNE_ENOMEM || st == BNNE_ENOTSUP ||
          (st == BNNE_OK && (sync != BNN_OK || *static_cast<volatile int*>(err_host) != kErrNone)))) {
         forget_message();
-        st = ready_batches(r);
-        if (st == BNNE_OK)
-            pass(false);
+        st = BNNE_OK;
+        pass(false);
     }
     if (st != BNNE_OK)
         return st;

@@ -4,12 +4,14 @@ fixtures of test_engine.py pin to the reference).  All comparisons bit for bit."
 from __future__ import annotations
 
 import ctypes
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
 from bnn_cases import first_mismatch
-from conftest import load_pkg
+from conftest import ROOT, load_pkg
 from test_engine import ERR, _engine_lib, write_error_model
 from test_fused import f32, host_rmsnorm, host_silu_mul
 
@@ -217,6 +219,16 @@ def test_growing_block_keeps_batches(pkg, hip, tmp_path):
         mat.destroy()
         bi.free()
         bo.free()
+
+
+def test_block_growth_without_memory(pkg, tmp_path):
+    """A block buffer that finds no memory: the prompt runs token by token, same logits, and the
+    program's own prepared batch on the device stays valid."""
+    path = tmp_path / "m.gguf"
+    pkg.gguf.qwen3_random(path, **TINY)
+    r = subprocess.run([sys.executable, str(ROOT / "tests" / "block_growth_run.py"), str(path)], capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.endswith("OK\n"), r.stdout[-500:] + r.stderr[-1500:]
 
 
 # Batches whose multi-row jobs run on the matrix cores: groups of up to four alike jobs (one k,
