@@ -1058,58 +1058,102 @@ struct BatchPlan {
     }
 };
 
-// Which jobs run on the matrix cores: groups of up to kGemmParts jobs of one k, one number of
-// rows and one mode, each group one launch of ~4 us and more, against
-// ~4 us for the one dot launch of every other job plus ~36 us per 10^9 weights times rows in
-// it (q/k/v of 8 / 64 / 256 rows 9.0 / 19.4 / 52 us a pass with dots, 7.9 / 8.4 / 15 us on
-// the matrix cores; 6144->6144 x 64 rows 60 against 22 us).  A group is worth its launch from
-// 0.11 * 10^9 on, or when it leaves the dot launch without work.  Fewest rows: 8, or 4 for
-// K > 2048, where the dots run in longer chains (6144->2048 x 4 rows 15.1 against 11.8 us; at
-// K = 2048 both take the same time, and the dots share the chip better with other streams).
-constexpr double kGemmGroupWork = 0.11e9;
-
+// Which jobs run on the matrix cores.  Jobs of one k, one number of rows and one mode form
+// groups of up to kGemmParts, each a launch of its own; every other job shares the one dot
+// launch.  Fewest rows of a group's jobs: 8, or 4 for K > 2048, where the dots run in longer
+// chains (at K = 2048 both take the same time, and the dots share the chip better with other
+// streams).  A launch on the matrix cores takes 4.4 us and more however little it does, the
+// dots ~19 us per 10^9 weights times rows behind a start of a few us, so many jobs of few rows
+// are faster as dots and few jobs of many rows in groups: of all dots, all groups, and the
+// groups that alone take less than the dots need for their jobs, the plan is the one with the
+// least time by the launchers' models.  Us a pass (GEMM_F32, dots / groups): 3 of 2048->1024 x
+// 64 rows 16.4 / 10.5; 32 of them x 16 32.4 / 41.9, x 32 53 / 47; 32 of 2048->6144 x 8 68.7 /
+// 93, x 16 127 / 96; 32 of 4096->4096 x 4 52 / 103, x 16 163 / 110; 128 x 4 179 / 420.
 constexpr uint32_t kGemmLookAhead = 64;  // jobs behind its first that a group is filled from
 
-BNN_Status place_jobs(const BNN_Job* jobs, BatchPlan* bp) {
+struct BatchGroup {
+    double us, work;  // of its launch; weights times rows
+    bool kept;
+};
+
+BNN_Status place_jobs(const BNN_Job* jobs, uint32_t cu_count, BatchPlan* bp) {
     const uint32_t count = bp->count;
-    double* work = static_cast<double*>(malloc(sizeof(double) * count));  // of group g
-    if (work == nullptr)
+    BatchGroup* group = static_cast<BatchGroup*>(malloc(sizeof(BatchGroup) * count));
+    if (group == nullptr)
         return BNN_ENOMEM;
-    uint32_t groups = 0, small = 0, dots = 0;
+    const auto work_of = [&](uint32_t i) { return (double)jobs[i].rows * bp->plans[i].m->n * bp->plans[i].m->k; };
+    uint32_t groups = 0;
     for (uint32_t i = 0; i < count; ++i)
         bp->places[i] = BatchPlace{kNoGemm, i, 0};
     for (uint32_t i = 0; i < count; ++i) {
-        if (bp->places[i].gemm != kNoGemm)
-            continue;
         const JobPlan& p = bp->plans[i];
-        if (jobs[i].rows < (p.m->k > 2048u ? 4u : 8u)) {
-            ++dots;
+        if (bp->places[i].gemm != kNoGemm || jobs[i].rows < (p.m->k > 2048u ? 4u : 8u))
             continue;
-        }
-        work[groups] = 0.0;
+        GemmJob shape = {};
+        shape.n = p.m->n, shape.k = p.m->k, shape.groups = p.m->groups, shape.tiles = p.m->tiles;
+        shape.rows = jobs[i].rows, shape.mode = p.mode;
+        BatchGroup& g = group[groups];
+        g = BatchGroup{0.0, 0.0, false};
         for (uint32_t j = i, members = 0; j < count && j - i < kGemmLookAhead && members < kGemmParts; ++j) {
             const JobPlan& o = bp->plans[j];
             if (bp->places[j].gemm != kNoGemm || jobs[j].rows != jobs[i].rows || o.m->k != p.m->k || o.mode != p.mode)
                 continue;
             bp->places[j].gemm = groups;
-            work[groups] += (double)jobs[j].rows * o.m->n * o.m->k;
-            ++members;
+            g.work += work_of(j);
+            if (members++ != 0)
+                shape.parts[shape.extra++].n = o.m->n;
         }
-        small += work[groups] < kGemmGroupWork;
+        g.us = gemm_launch_us(shape, cu_count);
         ++groups;
     }
-    // small groups go with the dots, unless the only one is all that the dots would have
-    const bool keep_small = small == 0 || (small == 1 && dots == 0);
+    // the dots of every job that is in no kept group; the launches of the kept ones
+    const auto dots_us = [&](double* per_work) {
+        double work = 0.0;
+        uint64_t items = 0;
+        uint32_t most = 0;
+        for (uint32_t pass = 0; pass < 2u; ++pass)  // the items follow from the most groups
+            for (uint32_t i = 0; i < count; ++i) {
+                const BNN_Matrix m = bp->plans[i].m;
+                if (bp->places[i].gemm != kNoGemm && group[bp->places[i].gemm].kept)
+                    continue;
+                if (pass == 0) {
+                    most = m->groups > most ? m->groups : most;
+                } else {
+                    items += dot_items(m->tiles, jobs[i].rows, most);
+                    work += work_of(i);
+                }
+            }
+        return dot_launch_us(items, most, work, cu_count, per_work);
+    };
+    const auto keep = [&](auto&& rule) {
+        double us = 0.0;
+        for (uint32_t g = 0; g < groups; ++g) {
+            group[g].kept = rule(group[g]);
+            us += group[g].kept ? group[g].us : 0.0;
+        }
+        return us;
+    };
+    double per_work = 0.0, unused;
+    const auto none = [](const BatchGroup&) { return false; };
+    const auto worth = [&](const BatchGroup& g) { return g.us < g.work * per_work; };
+    const auto all = [](const BatchGroup&) { return true; };
+    const double t_none = keep(none) + dots_us(&per_work);
+    const double t_worth = keep(worth) + dots_us(&unused);
+    const double t_all = keep(all) + dots_us(&unused);
+    if (t_none <= t_worth && t_none <= t_all)
+        keep(none);
+    else if (t_worth <= t_all)
+        keep(worth);
     uint32_t kept = 0;
     for (uint32_t g = 0; g < groups; ++g)
-        work[g] = keep_small || work[g] >= kGemmGroupWork ? (double)kept++ : -1.0;  // the group's new number
+        group[g].work = group[g].kept ? (double)kept++ : -1.0;  // its new number
     for (uint32_t i = 0; i < count; ++i)
         if (bp->places[i].gemm != kNoGemm) {
-            const double to = work[bp->places[i].gemm];
+            const double to = group[bp->places[i].gemm].work;
             bp->places[i].gemm = to < 0.0 ? kNoGemm : (uint32_t)to;
         }
     bp->gemm_count = kept;
-    free(work);
+    free(group);
     return BNN_OK;
 }
 
@@ -1146,7 +1190,7 @@ BNN_Status plan_batch(BNN_Device device, const BNN_Job* jobs, uint32_t count, Ba
         ins[i] = jobs[i].input.buffer;
     }
     if (st == BNN_OK)
-        st = place_jobs(jobs, bp);
+        st = place_jobs(jobs, device->cu_count, bp);
     for (uint32_t i = 0; st == BNN_OK && i < count; ++i) {
         const JobPlan& p = bp->plans[i];
         if (bp->places[i].gemm == kNoGemm) {

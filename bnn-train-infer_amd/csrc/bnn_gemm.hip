@@ -1584,18 +1584,61 @@ hipError_t launch_dots(const GemmLaunch& at, GemmJob job) {
 
 }  // namespace
 
-// The largest workgroup tile that still gives every CU a workgroup, else the tile
-// with the most workgroups.
+// Workgroups of tm x tn tiles over every part of the job.
+static uint64_t gemm_blocks(const GemmJob& job, uint32_t tm, uint32_t tn) {
+    uint64_t cols = (job.n + tn - 1u) / tn;
+    for (uint32_t i = 0; i < job.extra; ++i)
+        cols += (job.parts[i].n + tn - 1u) / tn;
+    return (uint64_t)((job.rows + tm - 1u) / tm) * cols;
+}
+
+// The tiles of k_gemm_mx and the time of the job in the one whose rounds of workgroups take
+// the least.  A round takes ~2.5 us and, per group, the step that a sweep gave for each tile
+// (17 shapes of K = 384..8192 and N = 1000..8192 x 14 row counts from 48 to 1024, all outputs
+// bit-identical; the choice was within 4% of the best tile for every one).
+enum MxTile { MX_64x64, MX_64x128, MX_64x192, MX_128x128, MX_128x192, MX_TILES };
+static MxTile mx_tile(const GemmJob& job, uint64_t cus, double* us) {
+    static const struct {
+        uint32_t tm, tn;
+        double step;
+    } tiles[MX_TILES] = {{64, 64, 0.34}, {64, 128, 0.45}, {64, 192, 0.60}, {128, 128, 0.72}, {128, 192, 0.88}};
+    MxTile best = MX_64x64;
+    for (int t = 0; t < MX_TILES; ++t) {
+        const uint64_t rounds = (gemm_blocks(job, tiles[t].tm, tiles[t].tn) + cus - 1u) / cus;
+        const double time = (double)rounds * (2.5 + tiles[t].step * job.groups);
+        if (t == 0 || time < *us)
+            best = (MxTile)t, *us = time;
+    }
+    return best;
+}
+
+double gemm_launch_us(const GemmJob& job, uint32_t cu_count) {
+    const uint64_t cus = cu_count ? cu_count : 256u;
+    const uint32_t g = job.groups;
+    double us = 0.0;
+    if (job.mode == MODE_DOT_I16) {
+        double columns = job.n;
+        for (uint32_t i = 0; i < job.extra; ++i)
+            columns += job.parts[i].n;
+        us = 2.9 + 0.07 * g + 0.45e-6 * (columns * g * 2.0 * job.rows);
+    } else if (gemm_blocks(job, 16, 32) <= cus || (g <= 16u && gemm_blocks(job, 32, 64) <= cus)) {
+        us = 1.3 + 0.12 * g;
+    } else if (g > 16u && gemm_blocks(job, 32, 64) <= cus) {
+        us = 3.0 + 0.30 * g;
+    } else {
+        (void)mx_tile(job, cus, &us);
+        us += 1.0;
+    }
+    return std::max(us, 4.4);
+}
+
+// launch_gemm's rules: the K-split kernels for few rows, then a wave per block, then the tile
+// of k_gemm_mx whose rounds of workgroups take the least time.
 hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count, uint64_t seq,
                        const uint64_t* flag, uint32_t* signals) {
     const GemmLaunch at{stream, seq, flag, signals};
     const uint64_t cus = cu_count ? cu_count : 256u;
-    auto blocks = [&](uint32_t tm, uint32_t tn) {
-        uint64_t cols = (job.n + tn - 1u) / tn;
-        for (uint32_t i = 0; i < job.extra; ++i)
-            cols += (job.parts[i].n + tn - 1u) / tn;
-        return (uint64_t)((job.rows + tm - 1u) / tm) * cols;
-    };
+    const auto blocks = [&](uint32_t tm, uint32_t tn) { return gemm_blocks(job, tm, tn); };
     // Few rows: K split over the waves of a workgroup, every wave's operands brought into
     // LDS by DMA before anything is computed (k_gemm_kr, k_gemm_kc).  The rules follow a
     // forced-choice sweep over K = 1024..8192, N = 1024..8192 and 8..256 rows (all outputs
@@ -1669,28 +1712,23 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // 4096->8192 x 64 27.8 -> 24.7); up to 16 groups 64 x 64 tiles are as fast
     if (job.groups > 16u && blocks(32, 64) <= cus)
         return launch_mx<32, 64, 1, 4>(at, job);
-    // Everything else: k_gemm_mx, one workgroup per CU, in the tile whose rounds of workgroups
-    // take the least time.  A round takes ~2.5 us and, per group, the step that a sweep gave for
-    // each tile (17 shapes of K = 384..8192 and N = 1000..8192 x 14 row counts from 48 to 1024,
-    // all outputs bit-identical; the choice was within 4% of the best tile for every one).  With
-    // tiles of 128 x 192 and 64 x 128 only, other kernels had filled the gaps, a call of
-    // 6144->2048 x 389 rows 42.8 -> 34.1 us, x 640 56.4 -> 41.5, 4096->4096 x 389 43.4 -> 33.2,
-    // 2048->2048 x 640 32.5 -> 25.3, 2048->4096 x 256 27.0 -> 23.1, 8192->4096 x 768 85 -> 69.
-    const auto time = [&](uint32_t tm, uint32_t tn, double step) {
-        return (double)((blocks(tm, tn) + cus - 1u) / cus) * (2.5 + step * job.groups);
-    };
-    const double t64 = time(64, 64, 0.34), t128 = time(64, 128, 0.45), t192 = time(64, 192, 0.60);
-    const double t128x128 = time(128, 128, 0.72), t128x192 = time(128, 192, 0.88);
-    const double least = std::min({t64, t128, t192, t128x128, t128x192});
-    if (t64 == least)
+    // Everything else: k_gemm_mx, one workgroup per CU (mx_tile).  With tiles of 128 x 192 and 64
+    // x 128 only, other kernels had filled the gaps, a call of 6144->2048 x 389 rows 42.8 -> 34.1
+    // us, x 640 56.4 -> 41.5, 4096->4096 x 389 43.4 -> 33.2, 2048->2048 x 640 32.5 -> 25.3,
+    // 2048->4096 x 256 27.0 -> 23.1, 8192->4096 x 768 85 -> 69.
+    double us = 0.0;
+    switch (mx_tile(job, cus, &us)) {
+    case MX_64x64:
         return launch_mx<64, 64, 2, 4>(at, job);
-    if (t128 == least)
+    case MX_64x128:
         return launch_mx<64, 128, 2, 4>(at, job);
-    if (t192 == least)
+    case MX_64x192:
         return launch_mx<64, 192, 2, 4>(at, job);
-    if (t128x128 == least)
+    case MX_128x128:
         return launch_mx<128, 128, 2, 4>(at, job);
-    return launch_mx<128, 192, 2, 4>(at, job);
+    default:
+        return launch_mx<128, 192, 2, 4>(at, job);
+    }
 }
 
 }  // namespace bnnhip

@@ -217,6 +217,9 @@ hipError_t launch_dot(hipStream_t stream, const DotJob& job, uint32_t cu_count, 
 // Work items of the dot kernel for a job (rows x groups of tiles); in a batch the
 // tiles per item follow the batch's largest group count.
 uint32_t dot_items(uint32_t tiles, uint32_t rows, uint32_t max_groups);
+// About what launch_dot_batch takes for that many items, in us, and the part of it that a
+// weight and row costs: a batch weighs its launches with it (place_jobs).
+double dot_launch_us(uint64_t items, uint32_t max_groups, double work, uint32_t cu_count, double* per_work);
 // Batch: device-resident job tables.  Prep: one block per row, block -> job map.
 // Dot: items = sum of rows*tiles; job of an item = item / uniform_items when every
 // job has that many items, else item_job[item].
@@ -232,6 +235,9 @@ hipError_t launch_dot_batch(hipStream_t stream, const DotJob* jobs, const uint32
 // launch has too many for that.
 hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count, uint64_t seq,
                        const uint64_t* flag, uint32_t* signals = nullptr);
+// About what launch_gemm's launch of the job takes, in us (the pointers may be null): a
+// batch weighs its launches with it (place_jobs).
+double gemm_launch_us(const GemmJob& job, uint32_t cu_count);
 // One launch of a fused batch of `tiles` 64-feature tiles on `grid` workgroups
 // (bnn_fused.hip).
 hipError_t launch_fused(hipStream_t stream, const FusedArgs& args, uint32_t tiles, uint32_t grid, uint64_t seq,

@@ -733,14 +733,25 @@ hipError_t launch_dot(hipStream_t stream, const DotJob& job, uint32_t cu_count, 
     return launch_dot_t<64, MAP_SINGLE, 1>(stream, job, nullptr, nullptr, items, 0, grid, seq, flag);
 }
 
+// One wave per item streams best when the items fill the chip several times; a small batch is
+// latency-bound, and the group-split kernel (4 waves per item) finishes each item sooner.
+static bool many_items(uint64_t items, uint32_t cu_count) {
+    return items >= (uint64_t)(cu_count ? cu_count : 256u) * BNN_DOT_WAVE_MIN_ITEMS_PER_CU;
+}
+
+// From batches of 1..128 jobs of K = 512..8192 x 2..64 rows: a start that grows with the chain of
+// groups, then ~18.5 us per 10^9 weights times rows, twice that in the group-split kernel's long
+// chains (6144->2048: 32 jobs x 3 rows 64 us a pass, x 4 rows 46).
+double dot_launch_us(uint64_t items, uint32_t max_groups, double work, uint32_t cu_count, double* per_work) {
+    *per_work = max_groups <= 16u || many_items(items, cu_count) ? 18.5e-9 : 38e-9;
+    return items == 0 ? 0.0 : 1.5 + 0.19 * max_groups + *per_work * work;
+}
+
 hipError_t launch_dot_batch(hipStream_t stream, const DotJob* jobs, const uint32_t* item_job, uint32_t items,
                             uint32_t uniform_items, uint32_t max_groups, bool scales, uint32_t cu_count, uint64_t seq,
                             const uint64_t* flag) {
     DotJob none = {};
-    // One wave per item streams best when the items fill the chip several times;
-    // a small batch is latency-bound, and the group-split kernel (4 waves per item)
-    // finishes each item sooner.
-    const bool many = (uint64_t)items >= (uint64_t)(cu_count ? cu_count : 256u) * BNN_DOT_WAVE_MIN_ITEMS_PER_CU;
+    const bool many = many_items(items, cu_count);
     if (BNN_DOT_WAVE_ITEMS && max_groups <= (uint32_t)kWaveMaxGroups && many) {
         if (uniform_items && scales)
             launch_dot_wave<MAP_UNIFORM, true>(stream, jobs, item_job, items, uniform_items, seq, flag);

@@ -277,6 +277,45 @@ def test_batch_jobs_on_the_matrix_cores(pkg, hipdev, oracle_fast, specs, shared)
     _free(mats, bi, bo)
 
 
+@pytest.mark.parametrize("specs,gemms,dots", [
+    ([("GEMM_F32", 2048, 1024, 64)] * 3, 1, 0),
+    ([("GEMM_F32", 2048, 1024, 64)] * 32, 8, 0),
+    ([("GEMM_F32", 2048, 1024, 16)] * 32, 0, 1),   # eight launches against one: 41.9 us a pass, 32.4 as dots
+    ([("GEMM_F32", 512, 512, 8)], 0, 1),
+    ([("GEMM_F32", 4096, 512, 4)], 1, 0),
+    ([("DOT_GROUPS", 1024, 1000, 40)] * 4, 1, 0),
+    ([("DOT_GROUPS", 1024, 1000, 40)] * 16, 0, 1),
+    ([("GEMM_F32", 2048, 2048, 64)] * 4 + [("GEMV_F32", 2048, 64, 1)] * 3, 1, 1),
+], ids=["qkv", "many-rows", "many-jobs", "one-small", "one-long", "dots-four", "dots-many", "beside"])
+def test_batch_routes(pkg, hipdev, specs, gemms, dots):
+    """Few jobs of many rows take launches on the matrix cores, many jobs of few rows the one dot
+    launch (what each gives is compared above and in test_hip_batch.py)."""
+    host = {(k, n): pkg.synth.matrix(n, k, seed=4) for _, k, n, _ in specs}
+    mats = [hipdev.matrix(*host[k, n]) for _, k, n, _ in specs]
+    jobs, bufs = (pkg.Job * len(specs))(), []
+    for i, (op, k, n, rows) in enumerate(specs):
+        in_t, out_t = pkg.api.OP_TYPES[pkg.Op[op]]
+        bi = hipdev.buffer(rows * k * (4 if in_t == pkg.Type.F32 else 1))
+        bo = hipdev.buffer(rows * n * (2 * (k // 128) if op == "DOT_GROUPS" else 4))
+        bi.write(np.zeros(bi.nbytes, np.uint8))
+        bufs += [bi, bo]
+        jobs[i] = pkg.Job(int(pkg.Op[op]), mats[i].handle.value, bi.view(in_t), bo.view(out_t), rows)
+    batch = ctypes.c_void_p()
+    assert hipdev.api.BNNX_BatchCreate(hipdev.handle, jobs, len(specs), ctypes.byref(batch)) == pkg.Status.OK
+    hipdev.kernel_timing(True)
+    before = [hipdev.kernel_timing_read(kind)[1] for kind in (3, 1)]
+    assert hipdev.api.BNNX_BatchLaunch(batch) == pkg.Status.OK
+    assert hipdev.api.BNNX_DeviceSynchronize(hipdev.handle) == pkg.Status.OK
+    ran = [hipdev.kernel_timing_read(kind)[1] - b for kind, b in zip((3, 1), before)]
+    hipdev.kernel_timing(False)
+    hipdev.api.BNNX_BatchDestroy(batch)
+    for m in mats:
+        m.destroy()
+    for b in bufs:
+        b.free()
+    assert ran == [gemms, dots]
+
+
 @pytest.mark.parametrize("k,n,rows,off,pad", [
     (896, 1000, 37, 0, 0),      # 7 groups, 16-byte rows
     (896, 1001, 20, 0, 0),      # rows that start at odd multiples of 2 bytes
