@@ -315,6 +315,8 @@ struct bnn_accel_device {
     unsigned char* scratch;    // grow-only device scratch
     size_t scratch_bytes;
     unsigned char* static_scratch;  // this GPU's fixed scratch array (BNNX_ExecuteNoAlloc)
+    hipEvent_t call_end;       // recorded behind a multi-row call's last launch (run_rows) ...
+    bool copied_out;           // ... if the copy engine has read a buffer since the call before
     unsigned char* pinned;     // grow-only pinned host staging for transfers
     size_t pinned_bytes;
     unsigned char* wring;      // pinned ring for small writes, copied asynchronously on `stream`

@@ -277,6 +277,28 @@ def test_batch_jobs_on_the_matrix_cores(pkg, hipdev, oracle_fast, specs, shared)
     _free(mats, bi, bo)
 
 
+@pytest.mark.parametrize("n,rows", [(1024, 4), (1024, 5), (1000, 16), (6144, 64)])
+def test_call_and_read_in_turn(pkg, hipdev, oracle_fast, n, rows):
+    """Write, call and read in turn, reads by the copy kernel (16 KB) and the copy engine, calls
+    with and without a read before: every read holds the results of the call before it."""
+    from bnn_cases import fast_oracle
+    k, T = 2048, pkg.Type.F32
+    host = pkg.synth.matrix(n, k, seed=9)
+    xs = [pkg.synth.normal_f32(rows, k, seed=40 + i) for i in range(3)]
+    wants = [fast_oracle(pkg, oracle_fast, "GEMM_F32", *host, x).reshape(-1) for x in xs]
+    m, bi, bo = hipdev.matrix(*host), hipdev.buffer(xs[0].nbytes), hipdev.buffer(4 * n * rows)
+    job = pkg.Job(int(pkg.Op.GEMM_F32), m.handle.value, bi.view(T), bo.view(T), rows)
+    for turn in range(12):
+        bi.write(xs[turn % 3])
+        assert hipdev.execute(job) == pkg.Status.OK
+        if turn % 4 != 3:
+            got = bo.read().view(np.float32)
+            assert np.array_equal(got.view(np.uint32), wants[turn % 3].view(np.uint32)), (turn, first_mismatch(got, wants[turn % 3]))
+    m.destroy()
+    bi.free()
+    bo.free()
+
+
 @pytest.mark.parametrize("specs,gemms,dots", [
     ([("GEMM_F32", 2048, 1024, 64)] * 3, 1, 0),
     ([("GEMM_F32", 2048, 1024, 64)] * 32, 8, 0),
