@@ -16,7 +16,7 @@
 //     increasing order, one rounding per add.  A zero product comes out as +0
 //     where the reference may form -0; the accumulator starts at +0 and never
 //     becomes -0 (x + -x == +0 in round-to-nearest), so the sums agree bit for bit.
-// DOT_GROUPS stores D itself as int16 (k_gemm_dots).
+// DOT_GROUPS stores D itself as int16 (k_gemm_dots, k_gemm_dotf).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -166,6 +166,14 @@ __device__ __forceinline__ void put2(void* p, uint16_t v, bool through) {
         asm volatile("global_store_short %0, %1, off sc0 sc1" ::"v"(p), "v"((uint32_t)v) : "memory");
     else
         *(__attribute__((address_space(1))) uint16_t*)p = v;
+}
+// two int16 at any even address
+typedef uint32_t u32_at2 __attribute__((aligned(2)));
+__device__ __forceinline__ void put2x2(void* p, uint32_t v, bool through) {
+    if (through)
+        asm volatile("global_store_dword %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+    else
+        *(__attribute__((address_space(1))) u32_at2*)p = v;
 }
 
 // Workgroup barrier for data handed over in LDS: this wave's LDS accesses are done before it
@@ -598,8 +606,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wv(GemmJob j, uint32_t mt
 // groups w, w + WAVES, ... (at most GB blocks in all): a block's rows and sign bits are requested at
 // once, straight into registers, expanded through the byte table, and each output's four dots
 // go to LDS as 8 bytes.  A row's part of the tile, [column][group] int16, is one contiguous run
-// of the output, so the tile leaves in 16- or 8-byte pieces of that run (2-byte ones for
-// odd-aligned views).  Bound by the launch for small jobs, by the stores for large ones; against
+// of the output, so the tile leaves in 16- or 8-byte pieces of that run (4-byte ones at
+// other alignments).  Bound by the launch for small jobs, by the stores for large ones; against
 // the accumulating kernels' tiles storing 2 bytes per output and group from the loop: 896->1000
 // x 37 rows 7.3 -> 5.3 us, 2048->2048 x 256 rows 27.7 -> 10.2, 8192->1000 x 64 rows 89.7 -> 11.3.
 template <int TNS, int GB, int WAVES>
@@ -727,16 +735,136 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_dots(GemmJob j, uint32_t mt
                     put2(run + i, *reinterpret_cast<const uint16_t*>(dots + row * ROW + i), through);
             }
         });
-    } else {  // any other alignment: value by value
-        each(cols * groups, [&](uint32_t row, uint32_t p, unsigned char* run) {
-            uint32_t at = 2u * p;
+    } else {  // any other alignment: two values at a time, the last of an odd number alone
+        const uint32_t bytes = cols * groups * 2u, per = groups / 2u;
+        each((bytes + 3u) / 4u, [&](uint32_t row, uint32_t p, unsigned char* run) {
+            uint32_t at = 4u * p;
             if (gaps) {
-                const uint32_t col = p / groups;
-                at = col * PITCH + 2u * (p - col * groups);
+                const uint32_t col = p / per;
+                at = col * PITCH + 4u * (p - col * per);
             }
-            put2(run + 2u * p, *reinterpret_cast<const uint16_t*>(dots + row * ROW + at), through);
+            const unsigned char* src = dots + row * ROW + at;
+            if (4u * p + 4u <= bytes)
+                put2x2(run + 4u * p, *reinterpret_cast<const uint32_t*>(src), through);
+            else
+                put2(run + 4u * p, *reinterpret_cast<const uint16_t*>(src), through);
         });
     }
+    gemm_signal(j, seq);
+}
+
+// k_gemm_dotf<MS, NS, GC>: DOT_GROUPS of up to 8 groups.  With so few groups a tile over the
+// whole K (k_gemm_dots) has next to nothing to compute, and its table, barriers and staging are
+// most of a workgroup's time; here each of a workgroup's four waves takes a (16 MS) x (16 NS)
+// block by itself, GC groups at a time: their rows and sign bits straight into registers, then
+// each output's GC dots straight from the registers to memory, 2 GC contiguous bytes (two dots
+// at a time and the last one alone where the group count is no multiple of GC).  Bound by the
+// stores for large jobs; calls of 128->8000 x 700 rows 58.6 -> 22.1 us against k_gemm_dots,
+// 256->2417 x 383 29.1 -> 17.5, 512->1001 x 200 22.4 -> 16.8, 896->6046 x 106 29.5 -> 24.8.
+template <int MS, int NS, int GC>
+__global__ __launch_bounds__(256) void k_gemm_dotf(GemmJob j, uint32_t mtiles, uint32_t ntiles, uint32_t band,
+                                                   uint64_t seq, const uint64_t* __restrict__ flag) {
+    static_assert(GC == 1 || GC == 2 || GC == 4, "dots per store");
+    constexpr uint32_t TM = 32u * MS, TN = 32u * NS;
+    __shared__ uint2 lut[256];
+    const uint64_t failed_seq = *flag;  // checked before anything is stored
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, chunk = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    TileRC tile = gemm_tile_of_block(blockIdx.x, gridDim.x, mtiles, ntiles, band);
+    tile.nt = select_part(j, tile.nt);
+    const uint32_t m0 = tile.mt * TM + 16u * MS * (wave >> 1), n0 = tile.nt * TN + 16u * NS * (wave & 1u);
+    const uint32_t groups = j.groups;
+    // rows past the end are clamped (never stored); so is the matrix tile of columns past the
+    // last one.  The K order inside a group is that of k_gemm_ks / k_gemm_wv.
+    const uint8_t* a_ptr[MS];
+    const uint8_t* b_ptr[NS];
+#pragma unroll
+    for (int mi = 0; mi < MS; ++mi)
+        a_ptr[mi] = reinterpret_cast<const uint8_t*>(j.q) +
+                    (size_t)min(m0 + 16u * mi + (lane & 15u), j.rows - 1u) * j.k + 32u * chunk;
+#pragma unroll
+    for (int ni = 0; ni < NS; ++ni) {
+        const uint32_t n = n0 + 16u * ni + (lane & 15u), st = min(n >> 6, j.tiles - 1u);
+        b_ptr[ni] = reinterpret_cast<const uint8_t*>(j.wbits) + ((size_t)st * groups * kTile + (n & 63u)) * 16u +
+                    4u * chunk;
+    }
+    v4i a[GC][MS][2];
+    uint32_t bits[GC][NS];
+    const auto load = [&](uint32_t g0) {
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)GC; ++i) {
+            const uint32_t g = min(g0 + i, groups - 1u);
+#pragma unroll
+            for (int mi = 0; mi < MS; ++mi)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    a[i][mi][h] = gload_v4i(a_ptr[mi] + (size_t)g * kGroup + 16u * h);
+#pragma unroll
+            for (int ni = 0; ni < NS; ++ni)
+                bits[i][ni] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(
+                    (uintptr_t)(b_ptr[ni] + (size_t)g * kTile * 16u));
+        }
+    };
+    load(0);
+    lut[tid] = make_uint2(pm1_nibble(tid & 15u), pm1_nibble(tid >> 4));
+    lds_barrier();  // the table is in LDS
+    if (failed_seq == seq) {
+        gemm_signal(j, seq);
+        return;
+    }
+    const v4i zero = {0, 0, 0, 0};
+    const bool at8 = ((j.out_stride | (uint64_t)(uintptr_t)j.out) & 7u) == 0;  // and 8 bytes per 4 groups
+    // in one of two forms, each without a branch per store
+    const auto run = [&](auto through) {
+        for (uint32_t g0 = 0; g0 < groups; g0 += GC) {
+            v4i d[GC][MS][NS];
+#pragma unroll
+            for (int i = 0; i < GC; ++i)
+#pragma unroll
+                for (int ni = 0; ni < NS; ++ni) {
+                    const uint32_t w = bits[i][ni];
+                    const uint2 e0 = lut[w & 0xffu], e1 = lut[(w >> 8) & 0xffu], e2 = lut[(w >> 16) & 0xffu], e3 = lut[w >> 24];
+                    const v4i b0 = {(int)e0.x, (int)e0.y, (int)e1.x, (int)e1.y}, b1 = {(int)e2.x, (int)e2.y, (int)e3.x, (int)e3.y};
+#pragma unroll
+                    for (int mi = 0; mi < MS; ++mi) {
+                        const v4i x = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][mi][0], b0, zero, 0, 0, 0);
+                        d[i][mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][mi][1], b1, x, 0, 0, 0);
+                    }
+                }
+            if (g0 + GC < groups)
+                load(g0 + GC);  // the next groups' operands, in flight during the stores
+            const auto pair = [&](int i, int mi, int ni, int r) {
+                return ((uint32_t)d[i][mi][ni][r] & 0xffffu) | ((uint32_t)d[(i + 1) % GC][mi][ni][r] << 16);
+            };
+#pragma unroll
+            for (int mi = 0; mi < MS; ++mi)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t m = m0 + 16u * mi + 4u * chunk + r;
+                    unsigned char* const row = j.out + (size_t)m * j.out_stride + 2u * g0;
+#pragma unroll
+                    for (int ni = 0; ni < NS; ++ni) {
+                        const uint32_t n = n0 + 16u * ni + (lane & 15u);
+                        if (m >= j.rows || n >= j.n)
+                            continue;
+                        unsigned char* const to = row + (size_t)n * groups * 2u;
+                        if (GC == 1 || g0 + GC > groups) {  // one group, or the last of an odd number
+                            put2(to, (uint16_t)d[0][mi][ni][r], through);
+                        } else if (GC == 4 && at8) {
+                            put8(to, pair(0, mi, ni, r) | ((uint64_t)pair(2 % GC, mi, ni, r) << 32), through);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i + 1 < GC; i += 2)
+                                put2x2(to + 2u * i, pair(i, mi, ni, r), through);
+                        }
+                    }
+                }
+        }
+    };
+    if (j.done)
+        run(std::true_type{});
+    else
+        run(std::false_type{});
     gemm_signal(j, seq);
 }
 
@@ -1582,6 +1710,14 @@ hipError_t launch_dots(const GemmLaunch& at, GemmJob job) {
     return launch_tiles(at, k_gemm_dots<TNS, GB, WAVES>, 64 * WAVES, job, mtiles, ntiles);
 }
 
+template <int MS, int NS, int GC>
+hipError_t launch_dotf(const GemmLaunch& at, GemmJob job) {
+    if (job.groups > 8u || job.groups % (GC == 4 ? 4u : 1u) != 0 || job.mode != MODE_DOT_I16)
+        return hipErrorInvalidValue;  // the selection below never asks for this
+    const uint32_t mtiles = (job.rows + 32u * MS - 1u) / (32u * MS), ntiles = gemm_ntiles(job, 32u * NS);
+    return launch_tiles(at, k_gemm_dotf<MS, NS, GC>, 256, job, mtiles, ntiles);
+}
+
 }  // namespace
 
 // Workgroups of tm x tn tiles over every part of the job.
@@ -1639,6 +1775,28 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     const GemmLaunch at{stream, seq, flag, signals};
     const uint64_t cus = cu_count ? cu_count : 256u;
     const auto blocks = [&](uint32_t tm, uint32_t tn) { return gemm_blocks(job, tm, tn); };
+    if (job.mode == MODE_DOT_I16) {
+        const uint32_t g = job.groups;
+        // Up to 4 groups, and up to 8 past a round of k_gemm_dots' smallest tiles, the blocks of
+        // k_gemm_dotf, 64 x 64 per workgroup up to one per CU (those signal), then 64 x 128: a
+        // sweep of 100 shapes of up to 8 groups, N = 64..8192 and 17..1024 rows, both kernels, e.g.
+        // 640->5065 x 27 rows 23.9 -> 19.2 us, 640->1226 x 72, less than a round, 18.8 and 19.2.
+        if (g <= 4u || (g <= 8u && blocks(16, 32) > cus)) {
+            if (blocks(64, 64) <= cus)
+                return g == 1u       ? launch_dotf<2, 2, 1>(at, job)
+                       : g % 4u == 0 ? launch_dotf<2, 2, 4>(at, job)
+                                     : launch_dotf<2, 2, 2>(at, job);
+            return g == 1u       ? launch_dotf<2, 4, 1>(at, job)
+                   : g % 4u == 0 ? launch_dotf<2, 4, 4>(at, job)
+                                 : launch_dotf<2, 4, 2>(at, job);
+        }
+        // 32-column tiles up to two per CU, and past 16 groups, whose tiles of 64 columns would
+        // not fit two workgroups' LDS
+        if (g > 16u)
+            return launch_dots<2, 16, 8>(at, job);
+        return blocks(16, 32) <= 2u * cus ? launch_dots<2, 4, 4>(at, job)
+                                          : launch_dots<4, 4, 4>(at, job);
+    }
     // Few rows: K split over the waves of a workgroup, every wave's operands brought into
     // LDS by DMA before anything is computed (k_gemm_kr, k_gemm_kc).  The rules follow a
     // forced-choice sweep over K = 1024..8192, N = 1024..8192 and 8..256 rows (all outputs
@@ -1653,14 +1811,6 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // tiles; each in one round.  Past those bounds k_gemm_mx wins (2048->2048 x 320 rows a call
     // of 25.0 us against 23.0, x 256 20.0 against 22.6; 4096->2048 x 180 27.9 against 26.3, x
     // 100 21.9 against 24.1).
-    if (job.mode == MODE_DOT_I16) {
-        // 32-column tiles up to two per CU, and past 16 groups, whose tiles of 64 columns would
-        // not fit two workgroups' LDS
-        if (job.groups > 16u)
-            return launch_dots<2, 16, 8>(at, job);
-        return blocks(16, 32) <= 2u * cus ? launch_dots<2, 4, 4>(at, job)
-                                          : launch_dots<4, 4, 4>(at, job);
-    }
     {
         const uint32_t g = job.groups;
         if (g <= 16u) {

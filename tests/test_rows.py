@@ -344,10 +344,20 @@ def test_batch_routes(pkg, hipdev, specs, gemms, dots):
     (128, 33, 17, 2, 0),        # one group, a view at offset 2
     (2048, 100, 16, 0, 0),      # 16 groups: 16-byte pieces, a partial column tile
     (512, 70, 49, 8, 8),        # 4 groups, 8-byte aligned rows
-    (2048, 70, 9, 2, 6),        # 16 groups from an odd address: value by value
-    (2176, 65, 18, 0, 0),       # 17 groups
+    (2048, 70, 9, 2, 6),        # 16 groups from an odd address: two values at a time
+    (2176, 65, 18, 0, 0),       # 17 groups, an odd number of values in a tile's row
     (8192, 40, 33, 0, 16),      # 64 groups
-    (1024, 5000, 130, 0, 0),    # more than two tiles per CU: 64-column tiles
+    (1280, 5000, 130, 0, 0),    # more than two tiles per CU: 64-column tiles
+    # the blocks for few groups: one group, pairs, fours; a last group alone; odd addresses
+    (128, 8000, 300, 0, 0),     # 64 x 128 blocks, more workgroups than signal
+    (256, 2417, 70, 2, 0),
+    (384, 1001, 65, 0, 2),
+    (512, 301, 130, 4, 4),      # fours at addresses that are no multiples of 8
+    (640, 5065, 27, 0, 0),
+    (768, 1223, 119, 0, 0),
+    (896, 6046, 106, 2, 2),
+    (1024, 6421, 170, 0, 0),    # fours in 64 x 128 blocks
+    (1024, 3001, 63, 0, 8),
 ])
 def test_dot_groups_rows(pkg, hipdev, oracle_fast, k, n, rows, off, pad):
     """DOT_GROUPS of many rows: every store width; padding and neighbours untouched."""
