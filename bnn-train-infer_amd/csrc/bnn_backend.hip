@@ -887,6 +887,16 @@ BNN_Status run_single_row(BNN_Device device, const BNN_Job* job, const JobPlan& 
     return result;
 }
 
+// Whether the rows of BNN_Execute's jobs that are not one fused launch run on the matrix
+// cores: all but few short ones whose output goes through staging rows.  A launch that writes
+// the output itself also signals its end, which the bit-plane kernels do not (2048->6144 x 2
+// rows 19.3 us with dots, 15.7; 6144->2048 x 2 rows 25.4, 18.3); behind a staging copy the call
+// waits for the stream either way (384->1000 x 2 rows 19.3 with dots, 20.3; 1024->6144 x 4 19.6,
+// 20.8; 2048->2048 x 2 20.5, 20.8; 6144->2048 x 2 27.1, 24.3).
+bool on_matrix_cores(const BNN_Job* job, const JobPlan& p) {
+    return p.out_aligned || job->rows >= 8u || p.m->groups > 8u;
+}
+
 // A multi-row job (or a single row the fused kernel does not take) in chunks of
 // `chunk` rows whose quantised forms occupy the first `rows_bytes` of `scratch`,
 // followed by the chunk's staging rows when the output view is not aligned.
@@ -965,7 +975,7 @@ EXPORT BNN_Status BNN_Execute(BNN_Device device, const BNN_Job* job) {
         return run_single_row(device, job, p, true);
 
     // rows in chunks that fit the device's scratch (allocated with the device)
-    const bool mfma = job->rows >= kMfmaMinRows;
+    const bool mfma = on_matrix_cores(job, p);
     size_t chunk = 0, rows_bytes = 0;
     chunk_rows(p, job->rows, mfma, device->scratch_bytes, &chunk, &rows_bytes);
     if (chunk == 0)

@@ -1,7 +1,6 @@
-// Multi-row jobs (GEMM, GEMM_F32, DOT_GROUPS with rows >= kMfmaMinRows) on the
-// gfx950 matrix cores (v_mfma_i32_16x16x64_i8), fed from the matrix's resident
-// 1.125-bit layout: a byte table in LDS turns the sign bits of each 128-weight group into
-// the MFMAs' +1/-1 operands.
+// Multi-row jobs (GEMM, GEMM_F32, DOT_GROUPS) on the gfx950 matrix cores
+// (v_mfma_i32_16x16x64_i8), fed from the matrix's resident 1.125-bit layout: a byte table in
+// LDS turns the sign bits of each 128-weight group into the MFMAs' +1/-1 operands.
 //
 // Numeric contract (reference bnn-accelerator.h:133-149, soft-bnn-accelerator.c:219-276),
 // per 128-weight group g:

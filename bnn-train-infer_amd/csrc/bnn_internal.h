@@ -86,8 +86,7 @@ struct DotJob {
     uint32_t first_block;
 };
 
-// One multi-row job on the matrix cores (rows >= kMfmaMinRows), read from the
-// matrix's resident layout (sign bits unpacked in LDS by the kernel).  Up to kGemmParts jobs
+// One multi-row job on the matrix cores, read from the matrix's resident layout (sign bits unpacked in LDS by the kernel).  Up to kGemmParts jobs
 // of one k, one number of rows and one mode (the q, k and v projections of a block of tokens,
 // jobs of a batch) may share a launch: the job's own fields describe the first, parts[] the
 // others, whose column tiles follow the first's; column tile t of the launch belongs to the
@@ -119,15 +118,6 @@ struct GemmJob {
     uint64_t* done;  // a launch whose caller waits for it: pinned host words, one per workgroup, that receive seq
     GemmPart parts[kGemmParts - 1];
 };
-
-// Rows from which a job of BNN_Execute that is not one fused launch runs on the matrix cores
-// instead of the bit-plane kernels: all of them (a call of 2048->6144 x 2 rows 19.3 us with
-// dots, 15.7 on the matrix cores with their own completion words; 6144->2048 x 2 rows 25.4 and
-// 18.3).
-#ifndef BNN_MFMA_MIN_ROWS
-#define BNN_MFMA_MIN_ROWS 1
-#endif
-constexpr uint32_t kMfmaMinRows = BNN_MFMA_MIN_ROWS;
 
 // Fused batches (bnn_fused.hip): GEMV_F32 jobs sharing one input row produced on
 // the device by a pre-operation.  One entry per job; the job's tiles are the

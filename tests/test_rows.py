@@ -277,6 +277,30 @@ def test_batch_jobs_on_the_matrix_cores(pkg, hipdev, oracle_fast, specs, shared)
     _free(mats, bi, bo)
 
 
+@pytest.mark.parametrize("op,k,n,rows", [
+    ("GEMM_F32", 384, 70, 1), ("GEMM_F32", 384, 70, 7), ("GEMM_F32", 384, 70, 8), ("GEMM", 1152, 65, 5),
+    ("DOT_GROUPS", 256, 70, 7), ("DOT_GROUPS", 1024, 33, 2), ("DOT_GROUPS", 1024, 33, 9),
+])
+def test_outputs_at_any_address(pkg, hipdev, oracle_fast, op, k, n, rows):
+    """Outputs that are not naturally aligned, by the dots and on the matrix cores."""
+    from bnn_cases import fast_oracle
+    host = pkg.synth.matrix(n, k, seed=k + n)
+    in_t, out_t = pkg.api.OP_TYPES[pkg.Op[op]]
+    x = pkg.synth.normal_f32(rows, k, seed=6) if op == "GEMM_F32" else pkg.synth.int8_uniform(rows, k, seed=6)
+    row = n * (2 * (k // 128) if op == "DOT_GROUPS" else 4)
+    m, bi, bo = hipdev.matrix(*host), hipdev.buffer(x.nbytes), hipdev.buffer(1 + rows * (row + 3))
+    bi.write(x)
+    bo.write(np.full(bo.nbytes, 0x5a, np.uint8))
+    job = pkg.Job(int(pkg.Op[op]), m.handle.value, bi.view(in_t), bo.view(out_t, 1, row + 3), rows)
+    assert hipdev.execute(job) == pkg.Status.OK
+    want = np.full((rows, row + 3), 0x5a, np.uint8)
+    want[:, :row] = fast_oracle(pkg, oracle_fast, op, *host, x).reshape(rows, -1).view(np.uint8)
+    assert np.array_equal(bo.read()[1:], want.reshape(-1))
+    m.destroy()
+    bi.free()
+    bo.free()
+
+
 @pytest.mark.parametrize("n,rows", [(1024, 4), (1024, 5), (1000, 16), (6144, 64)])
 def test_call_and_read_in_turn(pkg, hipdev, oracle_fast, n, rows):
     """Write, call and read in turn, reads by the copy kernel (16 KB) and the copy engine, calls
