@@ -75,6 +75,10 @@ class Rows:
     (6144, [200], 9, PreOp.SILU_MUL, True),
     (384, [1000], 66, PreOp.SILU_MUL, True),
     (2048, [96, 33], 40, PreOp.ROW, False),
+    # more jobs than one launch's parts
+    (512, [64, 33, 70, 128, 100], 20, PreOp.RMSNORM, True),
+    (256, [64, 5, 70, 64, 130, 64, 1, 33], 9, PreOp.SILU_MUL, True),
+    (384, [65, 64, 63, 62, 61, 60], 35, PreOp.ROW, False),
 ])
 def test_launch_rows(pkg, hipdev, oracle, k, ns, rows, kind, with_b):
     f = Rows(pkg, hipdev, k, ns, rows, kind, with_b)
@@ -111,6 +115,84 @@ def test_launch_rows_illegal_row(pkg, hipdev, kind):
         assert f.launch() == (0, 0)
     finally:
         f.free()
+
+
+def test_launch_rows_argument_checks(pkg, hipdev):
+    """What a call refuses, with its status; nothing is launched."""
+    S, T, api = pkg.Status, pkg.Type, hipdev.api
+    f = Rows(pkg, hipdev, 256, [70, 64], 6, PreOp.RMSNORM, True)
+    ptr = {name: b.device_pointer() for name, b in f.bufs.items()}
+    out = [o.device_pointer() for o in f.outs]
+    other = hipdev.matrix(*pkg.synth.matrix(64, 128, seed=1))
+
+    def call(kind=PreOp.RMSNORM, count=2, width=256, pre=True, job=None, **fields):
+        jobs = (pkg.Job * 9)(*[pkg.Job(int(pkg.Op.GEMM_F32), m.handle.value, f.bufs["a"].view(T.F32), o.view(T.F32), 6)
+                               for m, o in zip(f.mats, f.outs)])
+        for name, value in (job or {}).items():
+            setattr(jobs[1], name, value)
+        p = PreOp(kind, width)
+        if kind != PreOp.ROW:
+            p.a, p.b = ptr["a"], ptr["b"]
+        if kind == PreOp.RMSNORM:
+            p.gain, p.a_out, p.eps = ptr["gain"], ptr["x"], 1e-6
+        for name, value in fields.items():
+            setattr(p, name, value)
+        return api.BNNX_LaunchRows(hipdev.handle, jobs, count, ctypes.byref(p) if pre else None)
+
+    try:
+        assert call(count=0) == S.EINVAL and call(pre=False) == S.EINVAL
+        assert call(count=9) == S.ENOTSUP  # more than 8 jobs
+        assert call(kind=3) == S.EINVAL
+        assert call(width=0) == S.EINVAL and call(width=200) == S.EINVAL and call(width=128) == S.EINVAL
+        for missing in ("a", "gain"):
+            assert call(**{missing: None}) == S.EINVAL
+        for missing in ("a", "b"):
+            assert call(PreOp.SILU_MUL, **{missing: None}) == S.EINVAL
+        # jobs that differ in rows, K or (plain rows) the input view
+        assert call(job={"rows": 5}) == S.EINVAL
+        assert call(job={"matrix": other.handle.value, "output": f.outs[1].view(T.F32)}) == S.EINVAL
+        assert call(PreOp.ROW, job={"input": f.bufs["b"].view(T.F32)}) == S.EINVAL
+        # int8 rows, an output at an odd address; then a call that runs
+        assert call(job={"operation": int(pkg.Op.GEMM), "input": f.bufs["a"].view(T.I8)}) == S.ENOTSUP
+        assert call(job={"output": f.bufs["x"].view(T.F32, 2)}, a_out=None) == S.ENOTSUP
+        assert call(PreOp.ROW, count=1, job={}) == S.OK
+        # an output over another output, over an operand, over the stored sum; the sum over an operand
+        assert call(job={"output": f.outs[0].view(T.F32)}) == S.EINVAL
+        assert call(job={"output": f.bufs["b"].view(T.F32)}) == S.EINVAL
+        assert call(job={"output": f.bufs["gain"].view(T.F32)}) == S.EINVAL
+        assert call(job={"output": f.bufs["x"].view(T.F32)}) == S.EINVAL
+        assert call(a_out=ptr["a"]) == S.EINVAL and call(a_out=out[0] + 4) == S.EINVAL
+        assert call(PreOp.ROW, job={"output": f.bufs["a"].view(T.F32)}) == S.EINVAL
+        f.outs[0].write(np.full(6 * 70, 5.0, np.float32))  # after the one call that ran
+        assert call(job={"rows": 5}) == S.EINVAL
+        assert api.BNNX_DeviceSynchronize(hipdev.handle) == S.OK
+        assert all((o.read().view(np.float32) == 5.0).all() for o in f.outs)
+    finally:
+        other.destroy()
+        f.free()
+
+
+def test_launch_rows_limits(pkg, hipdev):
+    """4096 rows a call, and no more than the 32 MiB scratch holds."""
+    S, T = pkg.Status, pkg.Type.F32
+    a, out = hipdev.buffer(4 * 4096 * 8192), hipdev.buffer(4 * 4097 * 8)
+    wide, narrow = (hipdev.matrix(*pkg.synth.matrix(8, k, seed=k)) for k in (8192, 128))
+
+    def call(m, k, rows):
+        job = (pkg.Job * 1)(pkg.Job(int(pkg.Op.GEMM_F32), m.handle.value, a.view(T), out.view(T), rows))
+        return hipdev.api.BNNX_LaunchRows(hipdev.handle, job, 1, ctypes.byref(PreOp(PreOp.ROW, k)))
+
+    assert call(narrow, 128, 4097) == S.ENOTSUP
+    assert call(wide, 8192, 4096) == S.ENOTSUP
+    a.write(np.ones(4096 * 128, np.float32))
+    assert call(narrow, 128, 4096) == S.OK
+    assert hipdev.api.BNNX_DeviceSynchronize(hipdev.handle) == S.OK
+    got = out.read().view(np.float32)[:4096 * 8].reshape(4096, 8)
+    assert (got == got[0]).all() and np.isfinite(got).all()
+    wide.destroy()
+    narrow.destroy()
+    a.free()
+    out.free()
 
 
 @pytest.mark.parametrize("k", [128, 384, 640, 2048, 2176, 4096, 8192])
@@ -171,6 +253,86 @@ def test_prompt_blocks_match_single_tokens(pkg, hip, tmp_path, count, split):
         for c in (one, block):
             c.free()
         m.free()
+
+
+def last_step_and_block(pkg, hip, path, ids, context, singles):
+    """The last logits with the last `singles` tokens decoded one by one behind a prompt block,
+    and with every token in blocks."""
+    with pkg.Device(hip, 0) as dev:
+        m = pkg.engine.Model(_engine_lib(pkg), dev, path)
+        step, block = (pkg.engine.Context(m, n_ctx=context) for _ in range(2))
+        step.decode(ids[:-singles], want_logits=False)
+        for t in ids[-singles:-1]:
+            step.decode([t], want_logits=False)
+        got = step.decode(ids[-1:])
+        want = block.decode(ids)
+        for c in (step, block):
+            c.free()
+        m.free()
+    return got, want
+
+
+def test_step_past_the_kept_exponentials(pkg, hip, tmp_path):
+    """Steps around 16384 positions: past them k_attn_pv forms its exponentials again."""
+    path, context = tmp_path / "m.gguf", 16400
+    pkg.gguf.qwen3_random(path, **{**TINY, "context": context})
+    ids = np.random.default_rng(2).integers(0, TINY["vocab"], 16388, dtype=np.int32)
+    print("16388 positions", flush=True)
+    got, want = last_step_and_block(pkg, hip, path, ids, context, 6)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("count", [400, 4300])
+def test_softmax_sum_off_the_windows(pkg, hip, tmp_path, count):
+    """A softmax whose first term is 1 and whose others lie below half an ulp of 1: the in-order
+    sum stays at 1 while the prefix sums in 64 bits leave it by more than the candidates reach,
+    so k_attn_pv adds every segment term by term."""
+    hidden, hd, vocab = TINY["hidden"], 128, TINY["vocab"]
+    kept = {}
+
+    def signs(bits):
+        return np.unpackbits(bits, axis=1, bitorder="little").astype(np.float64) * 2 - 1
+
+    def note(name, data):  # the first layer's weights, its input norm without gains
+        if name == "blk.0.attn_norm.weight":
+            return np.ones_like(data)
+        if name in ("token_embd.weight", "blk.0.attn_q.weight", "blk.0.attn_k.weight"):
+            kept[name] = signs(data[0])
+        return data
+
+    pkg.gguf.qwen3_random(tmp_path / "weights.gguf", **{**TINY, "context": 4608}, tweak=note)
+    # head 0's queries and keys of every token: signs times signs; norm to RMS 1; of them only the
+    # pair of dims that turns least with the position
+    pair = [hd // 2 - 1, hd - 1]
+
+    def heads(w):
+        y = kept["token_embd.weight"] @ w[:hd].T
+        return (y / np.sqrt((y * y).mean(axis=1, keepdims=True)))[:, pair]
+
+    q, key = heads(kept["blk.0.attn_q.weight"]), heads(kept["blk.0.attn_k.weight"])
+    # a token x ahead of many y: score(y, x) - score(y, y) = 16.9, so a term of y is 4.6e-8
+    lead = q @ key.T - (q * key).sum(axis=1)[:, None]
+    y, x = np.unravel_index(lead.argmax(), lead.shape)
+    assert lead[y, x] > 1.0 and x != y
+    gain = np.float32(np.sqrt(16.9 / (lead[y, x] / np.sqrt(hd))))
+
+    def tweak(name, data):
+        if name in ("blk.0.attn_q_norm.weight", "blk.0.attn_k_norm.weight"):
+            data = np.zeros_like(data)
+            data[pair] = gain
+            return data
+        return note(name, data)
+
+    path = tmp_path / "m.gguf"
+    pkg.gguf.qwen3_random(path, **{**TINY, "context": 4608}, tweak=tweak)
+    ids = np.full(count, y, np.int32)
+    ids[0] = x
+    term = np.exp(-float(gain) ** 2 * lead[y, x] / np.sqrt(hd))
+    # (with the position's turn: below 6e-3, a few percent of a term)
+    assert 0.8 * 128 * term > 33 * 2.0 ** -23 and term * 1.25 < 2.0 ** -24
+    print(f"{count} positions, tokens {x} and {y}, a term {term:.3g}", flush=True)
+    got, want = last_step_and_block(pkg, hip, path, ids, 4608, 3)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
 def test_prompt_block_error_then_prompt(pkg, hip, tmp_path):
@@ -417,7 +579,9 @@ def test_dot_groups_rows(pkg, hipdev, oracle_fast, k, n, rows, off, pad):
     (384, 4000, 642, 16),     # 64 x 192
     (640, 3999, 1000, 0),     # 128 x 128
     (512, 5001, 770, 4),      # 128 x 192
-    (2048, 4213, 250, 0),     # 64 x 128, more workgroups than signal
+    (2048, 4213, 250, 0),     # 64 x 128, half a round
+    (2048, 5900, 400, 0),     # 64 x 192
+    (896, 8000, 1000, 0),     # 128 x 128, more workgroups than signal
     (6144, 2048, 289, 0),     # 64 x 64, 48 groups
     (4224, 4001, 99, 8),      # 32 x 64, 33 groups
     (8192, 1000, 130, 0),     # 32 x 64, 64 groups
