@@ -212,10 +212,12 @@ struct GemmLaunch {
     uint32_t* signals;  // with job.done: receives the workgroups that signal
 };
 
-// One workgroup per tile.  Launches of more than kDoneWords workgroups do not signal: from a
-// second round of workgroups on, stores written through cost what the earlier word to the
-// host saves (2048->6144 x 128 rows, 768 workgroups, 23.6 us either way; 2048->4213 x 250
-// rows, 1056 of them counted on a device word, 28.0 -> 30.0).
+// One workgroup per tile.  Launches of more than kDoneWords workgroups, one per CU, do not
+// signal.  Up to there it always paid (70 launches of 141..256 workgroups, 0.8 to 5.7 us a call:
+// 1536->3000 x 160 rows, 235 workgroups, 21.7 -> 19.5 us); past it stores written through cost
+// some launches more than the earlier word to the host saves (2048->8192 x 1500 rows, 768
+// workgroups, 69.8 -> 70.2; 128->8000 x 700 dots, 693 of them, 23.1 -> 28.0), though not all
+// (2048->8192 x 800 rows, 448 workgroups, 51.4 -> 49.6).
 template <class Kernel>
 hipError_t launch_tiles(const GemmLaunch& at, Kernel kernel, uint32_t threads, GemmJob& job, uint32_t mtiles,
                         uint32_t ntiles) {
@@ -1802,14 +1804,13 @@ hipError_t launch_gemm(hipStream_t stream, const GemmJob& job, uint32_t cu_count
     // bit-identical); against the kernels below, e.g. 2048->6144 x 64 rows 9.6 -> 5.8 us,
     // 6144->2048 x 64 rows 9.6 -> 6.4 us, 2048->2048 x 128 rows 7.7 -> 4.6 us, 4096->2048 x
     // 256 rows 14.5 -> 12.2 us, 6144->2048 x 128 rows 13.3 -> 9.6 us, 8192->2048 x 32 rows
-    // 9.2 -> 7.0 us.  Up to 16 groups: 32 x 32 tiles while they fit one round of two per CU,
-    // then 32 x 64 tiles while those fit one round (16 waves of one group each above 8 groups),
-    // then 32 x 32 tiles up to two rounds (not up to 8 groups, where the tiled kernel wins past
-    // one round); 17..32 groups: 16 x 32 tiles, then 32 x 32; 33..48 groups: 16 x 32 tiles, then
-    // 16 x 64 tiles with the slices' running sums handed on (k_gemm_kc); 49..64 groups: 16 x 16
-    // tiles; each in one round.  Past those bounds k_gemm_mx wins (2048->2048 x 320 rows a call
-    // of 25.0 us against 23.0, x 256 20.0 against 22.6; 4096->2048 x 180 27.9 against 26.3, x
-    // 100 21.9 against 24.1).
+    // 9.2 -> 7.0 us.  Up to 16 groups: 16 x 32 tiles (up to 16 rows) or 32 x 32 tiles while they
+    // fit one per CU, then 32 x 64 tiles while those do (16 waves of one group each above 8
+    // groups), then, above 8 groups, 32 x 32 tiles up to two per CU; 17..32 groups: 16 x 32
+    // tiles, then 32 x 32; 33..48 groups: 16 x 32 tiles, then 16 x 64 tiles with the slices'
+    // running sums handed on (k_gemm_kc); 49..64 groups: 16 x 16 tiles; each one per CU.  Past
+    // those bounds k_gemm_mx wins (2048->2048 x 320 rows a call of 25.0 us against 23.0, x 256
+    // 20.0 against 22.6; 4096->2048 x 180 27.9 against 26.3, x 100 21.9 against 24.1).
     {
         const uint32_t g = job.groups;
         if (g <= 16u) {

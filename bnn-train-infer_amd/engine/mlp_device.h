@@ -2,8 +2,11 @@
 // the blocks run there, and only the last block's outputs come back: one host wait per
 // chunk of rows instead of a write, a synchronous BNN_Execute and a read per block.  The
 // blocks run as one chained batch of the backend (BNNX_BatchCreateChain: each block's
-// GEMM_F32 and its post_scale * y + post_bias and ReLU, one launch for all of them), or,
-// for blocks wider than a chain takes, as one prepared batch of GEMM_F32 jobs per block
+// GEMM_F32 and its post_scale * y + post_bias and ReLU, one launch for all of them), which
+// reads the rows and writes the logits in page-locked host memory itself
+// (BNNX_ChainRunHost; with copies on either side while kernels are timed or launches are
+// outstanding), or, for blocks wider than a chain takes, as one prepared batch of GEMM_F32
+// jobs per block
 // (each row of a job is that sample's GEMV_F32, as SignLinear::apply_rows computes it)
 // followed by this engine's post-operation kernel (each operation rounded on its own as
 // mlp.cpp's host loop does).  The logits equal the host call pattern's bit for bit.

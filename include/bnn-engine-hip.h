@@ -8,16 +8,25 @@
  * row -- RMSNorm with the residual add, attention output, SiLU(gate)*up -- is
  * produced inside the layer's one launch) or, for layers wider than those take,
  * prepared batches (BNNX_BatchCreate), and the host waits once per BNNE_Decode
- * call.  The other path is the reference's call pattern: host
+ * call.  A call of three tokens or more (a prompt) runs them in blocks of up to 1024,
+ * every layer as a few multi-row launches.  The block's memory is made by the first such
+ * call, grows with longer ones and is kept until the context is freed: for each of up to
+ * 1024 tokens the activations of one layer (with width C, key/value width KV and
+ * feed-forward width FF: 4 C + 2 KV + 2 FF + max(C, FF) floats), the same again for the
+ * smaller sizes that it grew through, and up to 512 MB of attention scores (heads x tokens
+ * of the block x positions).  A call that finds no memory for it runs its tokens one by
+ * one.  The other path is the reference's call pattern: host
  * arithmetic, one synchronous BNN_Execute per linear layer chunk, the activations
  * copied across for every call.  Both compute the same logits bit for bit.
  * Statistics of the device path: execute_ns is the wait for the device,
  * transfer_ns the logits copy, device_calls the linear jobs run.
  *
- * A bnn-mlp context classifies on the device by default as well: a call's rows
- * are copied to the device once per chunk, every block runs there as a prepared
- * batch of GEMM_F32 jobs followed by its post_scale / post_bias / ReLU, and only
- * the logits come back (one host wait per chunk).  The other path is the
+ * A bnn-mlp context classifies on the device by default as well, in chunks of up to
+ * 256 rows: the rows are copied into page-locked memory, one launch reads them there,
+ * carries each through every block (GEMM_F32, post_scale / post_bias / ReLU) and writes
+ * the logits to page-locked memory, and the host waits once.  (Blocks wider than such a
+ * launch takes: the rows copied to the device, a prepared batch per block followed by
+ * its post-operation, the logits copied back.)  The other path is the
  * reference's call pattern: per block one write, the GEMM_F32 jobs and one read,
  * the post-operation on the host.  Both give the same logits bit for bit.  Its
  * device-path statistics: transfer_ns the two copies, execute_ns the wait.
