@@ -2,8 +2,8 @@
 
 s_barrier waits for no memory access and on gfx950 the compiler adds no wait before the
 builtin, so a hand-over through LDS needs its own s_waitcnt lgkmcnt(0).  A missing one shows
-in no result as long as the timing hides it; here the device assembly of this build is
-followed along every path, counting the LDS operations that may be outstanding."""
+in no result as long as the timing hides it; here the compiler's device assembly is followed
+along every path, counting the LDS operations that may be outstanding."""
 from __future__ import annotations
 
 import re

@@ -402,7 +402,9 @@ def test_block_growth_without_memory(pkg, tmp_path):
     ([("GEMM_F32", 256, 70, 4), ("GEMM", 256, 70, 4)], False),          # two small groups: the dots
     ([("GEMM_F32", 4096, 3000, 17), ("GEMV_F32", 512, 100, 1), ("GEMM", 4096, 200, 17),
       ("DOT_GROUPS", 4096, 1000, 33), ("GEMM_F32", 128, 5, 3), ("GEMM_F32", 4096, 65, 17)], False),
-], ids=["shared", "nine", "small", "small-two", "mixed"])
+    ([("DOT_GROUPS", 1024, 1000, 40)] * 4, False),                      # dots of few groups, four parts
+    ([("DOT_GROUPS", 640, 1301, 64), ("DOT_GROUPS", 640, 65, 64), ("DOT_GROUPS", 640, 4001, 64)], False),
+], ids=["shared", "nine", "small", "small-two", "mixed", "dots", "dots-odd"])
 def test_batch_jobs_on_the_matrix_cores(pkg, hipdev, oracle_fast, specs, shared):
     from test_hip_batch import _free, _mk_batch, _oracle, _outputs
     mats, xs, bi, bo, jobs, out_off, layouts = _mk_batch(pkg, hipdev, specs, seed=11)
